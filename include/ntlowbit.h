@@ -511,6 +511,13 @@ int ntlb_gemm_grouped_swiglu_quant_gu(int grid, const uint8_t* a, int64_t lda, c
                                       uint64_t offset, uint16_t* gu, int64_t ldgu, void* stream);
 
 /*
+ * Words of zeroed workspace that ntlb_nf4_quant / ntlb_fp8_persistent_quant of
+ * the n elements at w with scale blocks of `block` read: 0 where each block's
+ * amax stays inside one workgroup, ceil(n/block) for the two-pass kernels.
+ */
+int64_t ntlb_persistent_quant_ws_words(const void* w, int64_t n, int64_t block);
+
+/*
  * NF4 refresh of a persistent weight (the flat tensor of n elements):
  * _quantize_nf4_persistent + _pack_nibbles (layers.py:130-139, :156-169).
  * One scale per run of `block` consecutive elements (K for per_channel on an
@@ -518,7 +525,9 @@ int ntlb_gemm_grouped_swiglu_quant_gu(int grid, const uint8_t* a, int64_t lda, c
  * if finite and > 0 else 1 (layers.py:86-101).  code = argmin over the NF4
  * codebook (layers.py:60-83) of |clamp(w/s, -1, 1) - cb|, first minimum wins.
  * packed [ceil(n/2)]: element 2i in the low nibble of byte i.  amax_ws is a
- * caller-zeroed uint32 workspace of ceil(n/block) words; scales [ceil(n/block)].
+ * uint32 workspace of ceil(n/block) words, zeroed by the caller where
+ * ntlb_persistent_quant_ws_words is not 0 (else it is not touched); scales
+ * [ceil(n/block)].
  */
 int ntlb_nf4_quant(const void* w, int w_dtype, int64_t n, int64_t block, uint32_t* amax_ws, uint8_t* packed,
                    float* scales, void* stream);
@@ -542,7 +551,8 @@ int ntlb_mxfp4_dequant(const uint8_t* packed, const uint8_t* scales, int64_t n, 
  * Persistent FP8 (layers.py:104-127): scale = amax per block (K for
  * per_channel, n for per_tensor; finite and > 0 else 1), codes =
  * e4m3fn(clamp(w/s, -448, 448)); dequant = e4m3 value * scale cast to out_dtype.
- * amax_ws: caller-zeroed uint32 [ceil(n/block)].
+ * amax_ws: uint32 [ceil(n/block)], zeroed by the caller where
+ * ntlb_persistent_quant_ws_words is not 0 (else it is not touched).
  */
 int ntlb_fp8_persistent_quant(const void* w, int w_dtype, int64_t n, int64_t block, uint32_t* amax_ws,
                               uint8_t* codes, float* scales, void* stream);

@@ -396,34 +396,97 @@ struct AdamArgs {
 
 enum RefreshFmt : int { REFRESH_NONE = 0, REFRESH_NF4 = 1, REFRESH_FP8 = 2 };
 
+// The NF4 index of a quotient c in [-1, 1] by one table lookup and one
+// compare: nf4_index(c) is the number of thresholds below c, threshold i being
+// the largest float whose index is i (the fp32 distances to the two
+// neighbouring codebook values compare as argmin's do, ties to the lower
+// index).  The 32 buckets of width 1/16 over [-1, 1) hold at most one
+// threshold each, and every threshold lies at least 0.0016 inside its bucket,
+// so a bucket number rounded from fma(c, 16, 16) picks the right compare: entry
+// k gives that threshold (or +inf) and the index at the bucket's lower end;
+// entry 32 is c = 1.  The four-level binary search this replaces took about 40
+// VALU instructions per weight and bound the quantizers (the two-pass
+// per_channel quantize pass at [14336, 4096]: 79 us); the lookup takes six and
+// one 8-byte LDS read whose 33 entries lie in distinct banks.
+constexpr float kNF4t[15] = {-0x1.b239b2p-1f, -0x1.38a4e2p-1f, -0x1.d709p-2f, -0x1.5bd4eep-2f, -0x1.e079dap-3f,
+                             -0x1.1a7178p-3f, -0x1.74f0e4p-5f, 0x1.45f5fep-5f, 0x1.ec90c4p-4f, 0x1.a0cfcp-3f,
+                             0x1.2b05a8p-2f, 0x1.8ea7f2p-2f, 0x1.00da06p-1f, 0x1.491b5ep-1f, 0x1.b913b2p-1f};
+constexpr bool nf4_upper_nearer(int i, float c) {
+  const float lo = c - kNF4c[i], hi = kNF4c[i + 1] - c;  // c lies between the two
+  return hi < lo;
+}
+constexpr float next_float_up(float c) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, c);
+  return __builtin_bit_cast(float, (u >> 31) ? u - 1 : u + 1);
+}
+constexpr bool nf4_thresholds_exact() {
+  for (int i = 0; i < 15; ++i)
+    if (nf4_upper_nearer(i, kNF4t[i]) || !nf4_upper_nearer(i, next_float_up(kNF4t[i]))) return false;
+  return true;
+}
+static_assert(nf4_thresholds_exact(), "each threshold is the last float of the lower index");
+
+constexpr int NF4_ENTRIES = 33;
+// thread t < 33 fills entry t; the caller synchronizes before the first lookup
+__device__ __forceinline__ void nf4_table_fill(uint2* tab, int t) {
+  if (t >= NF4_ENTRIES) return;
+  const float lo = (float)t * 0.0625f - 1.0f;
+  uint32_t base = 0;
+  float thr = __builtin_inff();
+#pragma unroll
+  for (int i = 0; i < 15; ++i) {
+    base += kNF4t[i] < lo ? 1u : 0u;
+    if (kNF4t[i] >= lo && kNF4t[i] < lo + 0.0625f) thr = kNF4t[i];
+  }
+  tab[t] = make_uint2(__float_as_uint(thr), base);
+}
+
 // NF4 indices (layers.py:156-169) or e4m3 codes of clamp(w/s, +-448)
 // (layers.py:104-117) of 8 consecutive values w[0..8) at e0 with the scale s,
-// stored at their place in codes (4 packed bytes, or 8 code bytes)
+// stored at their place in codes (4 packed bytes, or 8 code bytes).
+//
+// fast: the block's values are finite, s is their amax (or 1 for a zero
+// block) and fast_div_ok(s) holds, and all 8 values lie inside n.  Then
+// |w/s| <= 1, the quotient comes from the exact reciprocal sequence of the fp8
+// quantizers with rs = 1/s (every quotient that can move a code, here |w/s| >=
+// 2^-10 for e4m3 and >= 0.039 for NF4, has a normal residual), and no clamp is
+// needed.  Otherwise each value is divided, clamped and encoded on its own.
 template <int RF>
-__device__ __forceinline__ void quant8_store(const float (&w)[8], float s, int64_t e0, int64_t n, uint8_t* codes) {
-  const bool full = e0 + 8 <= n;
-  // w / s by the exact reciprocal sequence of the fp8 quantizers wherever
-  // the scale allows it (fast_div_ok on s, which is the block amax or 1:
-  // every quotient that can move a code, here |w/s| >= 2^-10 for e4m3 and
-  // >= 0.039 for NF4, has a normal residual) and w is finite (a block with
-  // an infinity or a NaN has scale 1, and inf * 1 - inf would give NaN where
-  // the division gives inf), else by IEEE division: one division per 8
-  // weights instead of 8 (the NF4 pass was bound by its VALU work)
-  const bool fast = fast_div_ok<false>(__float_as_uint(s));
-  const float rs = fast ? 1.0f / s : 1.0f;
-  auto quot = [&](float x) {
-    if (fast && __builtin_isfinite(x)) {
-      const float y = x * rs;
-      const float e = __builtin_fmaf(-y, s, x);
-      return __builtin_copysignf(__builtin_fmaf(e, rs, y), x);
+__device__ __forceinline__ void quant8_store(const float (&w)[8], float s, float rs, bool fast, const uint2* tab,
+                                             int64_t e0, int64_t n, uint8_t* codes) {
+  if (fast) {
+    float c[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float y = w[i] * rs;
+      const float e = __builtin_fmaf(-y, s, w[i]);
+      c[i] = __builtin_fmaf(e, rs, y);
     }
-    return x / s;
-  };
+    if constexpr (RF == REFRESH_NF4) {
+      uint32_t word = 0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint2 t = tab[(uint32_t)__builtin_fmaf(c[i], 16.0f, 16.0f)];
+        word |= (t.y + (c[i] > __uint_as_float(t.x) ? 1u : 0u)) << (4 * i);
+      }
+      *reinterpret_cast<uint32_t*>(codes + e0 / 2) = word;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) c[i] = __builtin_copysignf(c[i], w[i]);
+      int lo = __builtin_amdgcn_cvt_pk_fp8_f32(c[0], c[1], 0, false);
+      lo = __builtin_amdgcn_cvt_pk_fp8_f32(c[2], c[3], lo, true);
+      int hi = __builtin_amdgcn_cvt_pk_fp8_f32(c[4], c[5], 0, false);
+      hi = __builtin_amdgcn_cvt_pk_fp8_f32(c[6], c[7], hi, true);
+      *reinterpret_cast<uint2*>(codes + e0) = make_uint2((uint32_t)lo, (uint32_t)hi);
+    }
+    return;
+  }
+  const bool full = e0 + 8 <= n;
   if constexpr (RF == REFRESH_NF4) {
     uint32_t word = 0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      float c = quot(w[i]);
+      float c = w[i] / s;
       c = (c < -1.0f) ? -1.0f : c;
       c = (c > 1.0f) ? 1.0f : c;
       word |= nf4_index(c) << (4 * i);
@@ -439,7 +502,7 @@ __device__ __forceinline__ void quant8_store(const float (&w)[8], float s, int64
     uint32_t c8[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      float c = quot(w[i]);
+      float c = w[i] / s;
       c = (c < -448.0f) ? -448.0f : c;
       c = (c > 448.0f) ? 448.0f : c;
       c8[i] = e4m3_rne(c);
@@ -465,6 +528,11 @@ template <int RF>
 __device__ __forceinline__ void refresh8(const float (&w)[8], uint32_t amax, int64_t e0, int64_t n, int64_t block,
                                          uint8_t* codes, float* scales, uint32_t* wave_amax, int tid) {
   const int lane = tid & 63, wave = tid >> 6;
+  __shared__ uint2 nf4_tab[RF == REFRESH_NF4 ? NF4_ENTRIES : 1];
+  if constexpr (RF == REFRESH_NF4) {
+    nf4_table_fill(nf4_tab, tid);
+    __syncthreads();
+  }
   const int gthreads = (int)(block >> 3);
   for (int off = 1; off < gthreads && off < 64; off <<= 1) amax = max(amax, (uint32_t)__shfl_xor((int)amax, off));
   if (gthreads > 64) {
@@ -479,7 +547,8 @@ __device__ __forceinline__ void refresh8(const float (&w)[8], uint32_t amax, int
   if (e0 >= n) return;
   const float s = (amax < 0x7F800000u && amax != 0u) ? __uint_as_float(amax) : 1.0f;
   if ((tid & (gthreads - 1)) == 0) scales[e0 / block] = s;
-  quant8_store<RF>(w, s, e0, n, codes);
+  const bool fast = amax < 0x7F800000u && fast_div_ok<false>(__float_as_uint(s)) && e0 + 8 <= n;
+  quant8_store<RF>(w, s, fast ? 1.0f / s : 1.0f, fast, nf4_tab, e0, n, codes);
 }
 
 // 8 consecutive values at e0 as fp32: one or two 16-byte loads when all 8 lie
@@ -621,11 +690,145 @@ __global__ void __launch_bounds__(256) flat_amax_chunks_kernel(const void* w, in
 template <int RF>
 __global__ void __launch_bounds__(256) flat_quant8_kernel(const void* w, int w_dtype, int64_t n, int64_t block,
                                                           const float* scales, uint8_t* codes) {
+  __shared__ uint2 nf4_tab[RF == REFRESH_NF4 ? NF4_ENTRIES : 1];
+  if constexpr (RF == REFRESH_NF4) {
+    nf4_table_fill(nf4_tab, threadIdx.x);
+    __syncthreads();
+  }
   const int64_t e0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
   if (e0 >= n) return;
   float v[8];
   load8f(w, w_dtype, e0, n, v);
-  quant8_store<RF>(v, scales[e0 / block], e0, n, codes);
+  // a scale other than 1 is the finite amax of its block
+  const float s = scales[e0 / block];
+  const bool fast = s != 1.0f && fast_div_ok<false>(__float_as_uint(s)) && e0 + 8 <= n;
+  quant8_store<RF>(v, s, fast ? 1.0f / s : 1.0f, fast, nf4_tab, e0, n, codes);
+}
+
+// One-pass quantizer with one scale per row (block elements, a multiple of 8,
+// at most 512 * CH * WPR): WPR waves hold a row in registers, CH 16-byte (fp32:
+// 32-byte) chunks per lane, so every weight is read once and the row's amax
+// needs no atomics, no zeroed workspace and no second launch.  HBM-bound: 2.5
+// bytes per bf16 weight (NF4).  At [14336, 4096] NF4 the call went from 102 to
+// 30 us (5.0 TB/s): it replaced an amax pass (27 us), a scale pass (5 us), a
+// quantize pass (79 us) and the workspace's fill by one launch.
+template <int RF, int IN_DT, int CH, int WPR>
+__global__ void __launch_bounds__(256) rows_quant_kernel(const void* w, int64_t rows, int block, uint8_t* codes,
+                                                         float* scales) {
+  __shared__ uint2 nf4_tab[RF == REFRESH_NF4 ? NF4_ENTRIES : 1];
+  __shared__ uint32_t red[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t row = WPR == 1 ? (int64_t)blockIdx.x * 4 + wave : (int64_t)blockIdx.x;
+  const int part = WPR == 1 ? 0 : wave;
+  const int nch = row < rows ? block >> 3 : 0;  // chunks of 8 values in the row
+  const int64_t e0 = row * block;
+  constexpr int NW = IN_DT == DT_F32 ? 2 : 1;
+  uint4 raw[CH][NW];
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    const int c = (j * WPR + part) * 64 + lane;
+#pragma unroll
+    for (int q = 0; q < NW; ++q) raw[j][q] = make_uint4(0, 0, 0, 0);
+    if (c < nch) {
+      const uint4* p = reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(w) +
+                                                      (e0 + (int64_t)c * 8) * (IN_DT == DT_F32 ? 4 : 2));
+#pragma unroll
+      for (int q = 0; q < NW; ++q) raw[j][q] = p[q];
+    }
+  }
+  if constexpr (RF == REFRESH_NF4) nf4_table_fill(nf4_tab, threadIdx.x);
+  auto floats = [&](int j, float (&v)[8]) {
+    if constexpr (IN_DT == DT_F32) {
+      const uint4 a = raw[j][0], b = raw[j][NW - 1];
+      const uint32_t u[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = __uint_as_float(u[i]);
+    } else {
+      const uint32_t u[4] = {raw[j][0].x, raw[j][0].y, raw[j][0].z, raw[j][0].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (IN_DT == DT_BF16) {
+          v[2 * i] = __uint_as_float(u[i] << 16);
+          v[2 * i + 1] = __uint_as_float(u[i] & 0xFFFF0000u);
+        } else {
+          v[2 * i] = __half2float(__ushort_as_half((unsigned short)(u[i] & 0xFFFFu)));
+          v[2 * i + 1] = __half2float(__ushort_as_half((unsigned short)(u[i] >> 16)));
+        }
+      }
+    }
+  };
+  uint32_t amax = 0;
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    if constexpr (IN_DT == DT_BF16) {
+      const uint4 r = raw[j][0];
+      const uint32_t m2 = pk_max_u16(pk_max_u16(r.x & 0x7FFF7FFFu, r.y & 0x7FFF7FFFu),
+                                     pk_max_u16(r.z & 0x7FFF7FFFu, r.w & 0x7FFF7FFFu));
+      amax = max(amax, max(m2 & 0xFFFFu, m2 >> 16) << 16);
+    } else {
+      float v[8];
+      floats(j, v);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) amax = max(amax, abs_bits(v[i]));
+    }
+  }
+  amax = wave_max_u32(amax);
+  if constexpr (WPR == 4) {
+    if (lane == 0) red[wave] = amax;
+  }
+  if constexpr (WPR == 4 || RF == REFRESH_NF4) __syncthreads();
+  if constexpr (WPR == 4) amax = max(max(red[0], red[1]), max(red[2], red[3]));
+  if (nch == 0) return;
+  const float s = (amax < 0x7F800000u && amax != 0u) ? __uint_as_float(amax) : 1.0f;
+  if (lane == 0 && part == 0) scales[row] = s;
+  const bool fast = amax < 0x7F800000u && fast_div_ok<false>(__float_as_uint(s));
+  const float rs = fast ? 1.0f / s : 1.0f;
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    const int c = (j * WPR + part) * 64 + lane;
+    if (c >= nch) break;
+    float v[8];
+    floats(j, v);
+    quant8_store<RF>(v, s, rs, fast, nf4_tab, e0 + (int64_t)c * 8, e0 + block, codes);
+  }
+}
+
+// Which blocks the row kernel takes.  Power-of-two blocks up to 2048 stay with
+// quant_blocks_onepass, which packs several blocks into a workgroup; below 64
+// values most of a wave's lanes would idle; above 16384 a row does not fit the
+// registers of four waves, and the two-pass kernels take it.
+static bool rows_block(const void* w, int64_t n, int64_t block) {
+  return block >= 64 && block <= 16384 && block % 8 == 0 && n % block == 0 && aligned(w, 16);
+}
+
+template <int RF>
+static void rows_quant(const void* w, int w_dtype, int64_t n, int64_t block, uint8_t* codes, float* scales,
+                       hipStream_t st) {
+  const int64_t rows = n / block;
+  const int b = (int)block;
+  auto go = [&](auto chc, auto wprc) {
+    constexpr int CH = decltype(chc)::value, WPR = decltype(wprc)::value;
+    const dim3 grd((unsigned)(WPR == 1 ? cdiv(rows, 4) : rows)), blk(256);
+    if (w_dtype == NTLB_BF16)
+      rows_quant_kernel<RF, DT_BF16, CH, WPR><<<grd, blk, 0, st>>>(w, rows, b, codes, scales);
+    else if (w_dtype == NTLB_F32)
+      rows_quant_kernel<RF, DT_F32, CH, WPR><<<grd, blk, 0, st>>>(w, rows, b, codes, scales);
+    else
+      rows_quant_kernel<RF, DT_F16, CH, WPR><<<grd, blk, 0, st>>>(w, rows, b, codes, scales);
+  };
+  using std::integral_constant;
+  if (block <= 512)
+    go(integral_constant<int, 1>(), integral_constant<int, 1>());
+  else if (block <= 1024)
+    go(integral_constant<int, 2>(), integral_constant<int, 1>());
+  else if (block <= 2048)
+    go(integral_constant<int, 4>(), integral_constant<int, 1>());
+  else if (block <= 4096)
+    go(integral_constant<int, 8>(), integral_constant<int, 1>());
+  else if (block <= 8192)
+    go(integral_constant<int, 4>(), integral_constant<int, 4>());
+  else
+    go(integral_constant<int, 8>(), integral_constant<int, 4>());
 }
 
 template <int RF>
@@ -1164,6 +1367,14 @@ static bool flat_two_pass(const void* w, int w_dtype, int64_t n, int64_t block, 
   return true;
 }
 
+// the one-launch quantizers (a block's values in one wave or workgroup) read no
+// workspace; the two-pass ones need it zeroed
+extern "C" int64_t ntlb_persistent_quant_ws_words(const void* w, int64_t n, int64_t block) {
+  if (n <= 0 || block < 1) return 0;
+  if ((onepass_block(block) && aligned(w, 16)) || rows_block(w, n, block)) return 0;
+  return cdiv(n, block);
+}
+
 extern "C" int ntlb_nf4_quant(const void* w, int w_dtype, int64_t n, int64_t block, uint32_t* amax_ws,
                               uint8_t* packed, float* scales, void* stream) {
   const char* fn = "ntlb_nf4_quant";
@@ -1181,6 +1392,10 @@ extern "C" int ntlb_nf4_quant(const void* w, int w_dtype, int64_t n, int64_t blo
   const int64_t threads = cdiv(n, 8);
   if (cdiv(threads, 256) > 0x7FFFFFFF) return fail(NTLB_EINVAL, "%s: too large", fn);
   hipStream_t st = as_stream(stream);
+  if (rows_block(w, n, block)) {
+    rows_quant<REFRESH_NF4>(w, w_dtype, n, block, packed, scales, st);
+    return check_launch(fn);
+  }
   if (flat_two_pass<REFRESH_NF4>(w, w_dtype, n, block, amax_ws, packed, scales, st)) return check_launch(fn);
   dim3 grd((unsigned)cdiv(threads, 256)), blk(256);
   if (w_dtype == NTLB_BF16)
@@ -1342,6 +1557,10 @@ extern "C" int ntlb_fp8_persistent_quant(const void* w, int w_dtype, int64_t n, 
   if (cdiv(cdiv(n, 8), 256) > 0x7FFFFFFF) return fail(NTLB_EINVAL, "%s: too large", fn);
   dim3 grd((unsigned)cdiv(cdiv(n, 8), 256)), blk(256);
   hipStream_t st = as_stream(stream);
+  if (rows_block(w, n, block)) {
+    rows_quant<REFRESH_FP8>(w, w_dtype, n, block, codes, scales, st);
+    return check_launch(fn);
+  }
   if (flat_two_pass<REFRESH_FP8>(w, w_dtype, n, block, amax_ws, codes, scales, st)) return check_launch(fn);
   if (w_dtype == NTLB_BF16)
     flat_block_amax_kernel<DT_BF16><<<grd, blk, 0, st>>>(w, n, block, amax_ws);

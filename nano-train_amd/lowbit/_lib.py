@@ -61,6 +61,7 @@ SIGNATURES = {
     "ntlb_gemm_grouped_swiglu_quant": [_I32, _P, _I64, _P, _I64, _I64, _I32, _P, _I64, _I64, _P, _I64, _I64, _I64,
                                        _P, _I32, _I64, _I64, _I64, _P, _P, _P, _I64, _P, _I64, _P, _I64, _I64, _P,
                                        _I32, _I32, _I32, _U64, _U64, _P],
+    "ntlb_persistent_quant_ws_words": [_P, _I64, _I64],
     "ntlb_nf4_quant": [_P, _I32, _I64, _I64, _P, _P, _P, _P],
     "ntlb_nf4_dequant": [_P, _P, _I64, _I64, _P, _I32, _P],
     "ntlb_mxfp4_quant": [_P, _I32, _I64, _P, _P, _P],
@@ -136,7 +137,7 @@ SIGNATURES = {
 
 # entry points that return a value instead of a status
 RESTYPES = {"ntlb_gemm_workspace_bytes": _I64, "ntlb_ep_record_bytes": _I64, "ntlb_colsum_workspace_bytes": _I64,
-            "ntlb_ep_value_record_bytes": _I64,
+            "ntlb_ep_value_record_bytes": _I64, "ntlb_persistent_quant_ws_words": _I64,
             "ntlb_gemm_lowbit_workspace_bytes": _I64, "ntlb_gemm_dq_workspace_bytes": _I64}
 
 _lib = None

@@ -53,6 +53,13 @@ def _flat(t: torch.Tensor) -> torch.Tensor:
     return t.detach().reshape(-1) if t.is_contiguous() else t.detach().contiguous().reshape(-1)
 
 
+def _amax_workspace(flat: torch.Tensor, n: int, block: int, nb: int) -> torch.Tensor:
+    """The amax workspace of the flat quantizers: zeroed where the two-pass
+    kernels accumulate into it (the one-launch kernels do not touch it)."""
+    zeroed = n > 0 and _lib.lib().ntlb_persistent_quant_ws_words(flat.data_ptr(), n, block) > 0
+    return (torch.zeros if zeroed else torch.empty)(max(nb, 1), dtype=torch.int32, device=flat.device)
+
+
 def quantize_nf4_blocks(tensor: torch.Tensor, block: int):
     """NF4 codes with one scale per `block` consecutive elements: (packed, scales[ceil(n/block)])."""
     flat = _flat(tensor)
@@ -60,7 +67,7 @@ def quantize_nf4_blocks(tensor: torch.Tensor, block: int):
     nb = ops.cdiv(n, block) if n else 0
     packed = torch.empty((n + 1) // 2, dtype=torch.uint8, device=flat.device)
     scales = torch.empty(nb, dtype=torch.float32, device=flat.device)
-    ws = torch.zeros(max(nb, 1), dtype=torch.int32, device=flat.device)
+    ws = _amax_workspace(flat, n, block, nb)
     call("ntlb_nf4_quant", flat.data_ptr(), ops._dtype_code(flat.dtype), n, block, ws.data_ptr(), packed.data_ptr(),
          scales.data_ptr(), ops._stream())
     return packed, scales
@@ -100,7 +107,7 @@ def quantize_fp8_persistent(tensor: torch.Tensor, *, granularity: str):
     nb = ops.cdiv(n, block) if n else 0
     codes = torch.empty(n, dtype=torch.uint8, device=flat.device)
     scales = torch.empty(nb, dtype=torch.float32, device=flat.device)
-    ws = torch.zeros(max(nb, 1), dtype=torch.int32, device=flat.device)
+    ws = _amax_workspace(flat, n, block, nb)
     call("ntlb_fp8_persistent_quant", flat.data_ptr(), ops._dtype_code(flat.dtype), n, block, ws.data_ptr(),
          codes.data_ptr(), scales.data_ptr(), ops._stream())
     return codes.view(torch.float8_e4m3fn).reshape(tensor.shape), scales.reshape(shape)

@@ -631,3 +631,39 @@ def test_persistent_forward_ragged_k_decodes_every_code_exactly(gpu_device, fmt,
         y = P.linear_fp8p(x, codes.to(gpu_device), sc.to(gpu_device), out_dtype=torch.float32)
     torch.cuda.synchronize()
     np.testing.assert_array_equal(y.cpu().numpy().T, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+@pytest.mark.parametrize("K", [72, 504, 520, 1032, 2056, 4096, 4104, 8192, 8200, 16384])
+def test_row_quantizer_edges(gpu_device, K, dtype):
+    """One scale per row with the row held in registers: rows on each side of
+    every register count (one to eight chunks a lane, one or four waves a row),
+    a row count that is no multiple of the rows per workgroup, and rows whose
+    scale the fast division does not take (zero, NaN, inf, subnormal amax) or
+    that lie at the codebook's thresholds (amax 1), for NF4 and FP8, bit for
+    bit against the oracle."""
+    from lowbit import persistent as P
+
+    w = seeded((11, K), seed=20261901 + K, std=0.02, dtype=torch.float32)
+    w[1] = 0.0
+    w[2, K // 3] = float("nan")
+    w[3, K - 1] = float("-inf")
+    w[4] *= 2.0 ** -20
+    w[5] = w[5].sign() * 1e-7 if dtype == torch.float16 else w[5] * 2.0 ** -130
+    cb = torch.from_numpy(np.asarray(O.NF4_CODEBOOK, dtype=np.float32))
+    mid = (cb[1:] + cb[:-1]) / 2
+    edges = torch.cat([cb, mid, *(torch.nextafter(mid, mid + d) for d in (1.0, -1.0))])
+    w[6, :len(edges)] = edges
+    w[6, len(edges):] = edges[torch.arange(K - len(edges)) % len(edges)]
+    w[7, 0], w[8, K - 1] = -3.0, 3.0  # amax at either end of the row
+    w[9, ::2] = -0.0
+    w = w.to(dtype)
+    wd = w.to(gpu_device)
+    packed, scale = P.quantize_nf4_persistent(wd, granularity="per_channel")
+    p_ref, s_ref = O.nf4_quant(to_np32(w), K)
+    assert_bits_equal(packed.cpu().numpy(), p_ref, "nf4 packed")
+    assert_bits_equal(scale.reshape(-1).cpu().numpy(), s_ref, "nf4 scale")
+    codes, scale = P.quantize_fp8_persistent(wd, granularity="per_channel")
+    c_ref, s_ref = O.fp8_persistent_quant(to_np32(w), K)
+    assert_bits_equal(codes.view(torch.uint8).cpu().numpy().reshape(-1), c_ref.reshape(-1), "fp8 codes")
+    assert_bits_equal(scale.reshape(-1).cpu().numpy(), s_ref, "fp8 scale")
