@@ -966,10 +966,10 @@ struct Raw32 {
   uint4 a, b;
 };
 
-// e4m3 weights 8j..8j+7 of the 32 of tile row r, half h: layers.py:121-127,
-// the code's value (hardware decode, exact for every code, NaN codes to NaN)
-// times the scale in fp32, rounded to bf16
-__device__ __forceinline__ void dequant8_fp8_to_lds(const Raw32& raw, float s, int j, uint8_t* tile, int r, int h) {
+// e4m3 weights 8j..8j+7 of the 32 as bf16: layers.py:121-127, the code's
+// value (hardware decode, exact for every code, NaN codes to NaN) times the
+// scale in fp32, rounded to bf16
+__device__ __forceinline__ uint4 dequant8_fp8(const Raw32& raw, float s, int j) {
   const uint32_t words[8] = {raw.a.x, raw.a.y, raw.a.z, raw.a.w, raw.b.x, raw.b.y, raw.b.z, raw.b.w};
   uint32_t out[4];
 #pragma unroll
@@ -981,7 +981,7 @@ __device__ __forceinline__ void dequant8_fp8_to_lds(const Raw32& raw, float s, i
     out[2 * w] = __builtin_bit_cast(uint32_t, p0);
     out[2 * w + 1] = __builtin_bit_cast(uint32_t, p1);
   }
-  *reinterpret_cast<uint4*>(tile + fswz(r, h * 4 + j)) = make_uint4(out[0], out[1], out[2], out[3]);
+  return make_uint4(out[0], out[1], out[2], out[3]);
 }
 
 // The 16 bf16 weight values an NF4 thread can meet in one K step (all 32 of
@@ -1051,12 +1051,11 @@ __device__ __forceinline__ StepDecode<FMT> decode_begin(float s) {
 }
 
 // weights 8j..8j+7 (4 packed bytes, low nibble first; or 8 e4m3 bytes) of
-// the 32 of tile row r, half h, as one 16-byte LDS chunk
+// the 32, as eight bf16 values
 template <int FMT>
-__device__ __forceinline__ void decode_chunk(const StepDecode<FMT>& d, const Raw32& rw, int j, uint8_t* tile, int r,
-                                             int h) {
+__device__ __forceinline__ uint4 decode8(const StepDecode<FMT>& d, const Raw32& rw, int j) {
   if constexpr (FMT == FMT_FP8P) {
-    dequant8_fp8_to_lds(rw, d.s, j, tile, r, h);
+    return dequant8_fp8(rw, d.s, j);
   } else if constexpr (FMT == FMT_MXFP4) {
     // byte b of the word holds weights 2b (low nibble) and 2b+1: the pair
     // the instruction returns in that order
@@ -1067,7 +1066,7 @@ __device__ __forceinline__ void decode_chunk(const StepDecode<FMT>& d, const Raw
                            __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, d.s, 2)),
                            __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, d.s, 3)));
     if (d.nan) out = make_uint4(0x7FC07FC0u, 0x7FC07FC0u, 0x7FC07FC0u, 0x7FC07FC0u);
-    *reinterpret_cast<uint4*>(tile + fswz(r, h * 4 + j)) = out;
+    return out;
   } else {
     const uint32_t words[4] = {rw.a.x, rw.a.y, rw.a.z, rw.a.w};
     const uint32_t w = words[j];
@@ -1080,10 +1079,16 @@ __device__ __forceinline__ void decode_chunk(const StepDecode<FMT>& d, const Raw
     const uint32_t h03 = __builtin_amdgcn_perm(ho, he, 0x05010400u);
     const uint32_t l47 = __builtin_amdgcn_perm(lo_, le, 0x07030602u);
     const uint32_t h47 = __builtin_amdgcn_perm(ho, he, 0x07030602u);
-    *reinterpret_cast<uint4*>(tile + fswz(r, h * 4 + j)) =
-        make_uint4(__builtin_amdgcn_perm(h03, l03, 0x05010400u), __builtin_amdgcn_perm(h03, l03, 0x07030602u),
-                   __builtin_amdgcn_perm(h47, l47, 0x05010400u), __builtin_amdgcn_perm(h47, l47, 0x07030602u));
+    return make_uint4(__builtin_amdgcn_perm(h03, l03, 0x05010400u), __builtin_amdgcn_perm(h03, l03, 0x07030602u),
+                      __builtin_amdgcn_perm(h47, l47, 0x05010400u), __builtin_amdgcn_perm(h47, l47, 0x07030602u));
   }
+}
+
+// decode8 into the 16-byte LDS chunk of tile row r, half h
+template <int FMT>
+__device__ __forceinline__ void decode_chunk(const StepDecode<FMT>& d, const Raw32& rw, int j, uint8_t* tile, int r,
+                                             int h) {
+  *reinterpret_cast<uint4*>(tile + fswz(r, h * 4 + j)) = decode8<FMT>(d, rw, j);
 }
 
 template <int FMT>
@@ -1344,6 +1349,133 @@ __global__ void __launch_bounds__(512, 1) gemm_lowbit_fused_kernel(FusedArgs g) 
   }
 }
 
+// ---------------------------------------------------------------------------
+// Dequant-fused GEMM for few rows: output tile 16*MB x 16*NB per workgroup of
+// WK waves, each wave the whole tile over its own range of K, the WK partial
+// tiles summed in wave order through LDS.  No operand is staged: a lane loads
+// the codes of 32 consecutive weights of one weight row per 128-K step (16 or
+// 32 bytes, next to the other lane groups' of that row) and the 32 matching
+// activations of its MB rows (from the caches: every workgroup reads them),
+// decodes to bf16 in registers and feeds v_mfma_f32_16x16x32_bf16.  The next
+// step's loads are in flight during a step.  With a 256x256 tile, 4 rows at N
+// 14336 ran 56 tiles (split four ways) and spent 63/64 of the matrix work on
+// padding rows; here N / (16 NB) workgroups of eight waves stream the weight.
+// ---------------------------------------------------------------------------
+template <int FMT, int MB, int NB, int WK>
+__global__ void __launch_bounds__(64 * WK) gemm_lowbit_rows_kernel(FusedArgs g) {
+  __shared__ __attribute__((aligned(16))) v4f red[WK][MB * NB][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15, gq = lane >> 4;
+  const int64_t n0 = (int64_t)blockIdx.x * (16 * NB), m0 = (int64_t)blockIdx.y * (16 * MB);
+  const int steps = (int)((g.K + 127) >> 7);
+  const int ks0 = (int)((int64_t)wave * steps / WK), ks1 = (int)((int64_t)(wave + 1) * steps / WK);
+  constexpr bool BYTE_CODES = FMT == FMT_FP8P;
+
+  // rows at or past M lie beyond the resource and read zero
+  __amdgpu_buffer_rsrc_t rx =
+      __builtin_amdgcn_make_buffer_rsrc((void*)g.x, (short)0, (int)(g.M * g.ldx * 2), 0x00020000);
+  uint32_t xoff[MB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) xoff[mb] = (uint32_t)((m0 + mb * 16 + li) * g.ldx * 2 + gq * 64);
+  const uint8_t* wrow[NB];
+  RowScales wsc[NB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) {
+    const int64_t n = min<int64_t>(n0 + nb * 16 + li, g.N - 1);  // columns past N are never stored
+    wrow[nb] = g.w + n * (BYTE_CODES ? g.K : g.K >> 1) + gq * (BYTE_CODES ? 32 : 16);
+    wsc[nb] = fused_row_scales<FMT>(g, n);
+  }
+  struct Stage {
+    Raw32 w[NB];
+    float sc[NB];
+    uint4 x[MB][4];
+  };
+  auto load = [&](Stage& s, int ks) {
+    const uint32_t k0 = (uint32_t)ks * 128 + gq * 32;
+    // K is a multiple of 64: the upper half of the last step can lie past it
+    // (zero codes, scale and activations there)
+    const bool in = k0 < (uint32_t)g.K;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      s.w[nb].a = make_uint4(0, 0, 0, 0);
+      s.w[nb].b = make_uint4(0, 0, 0, 0);
+      s.sc[nb] = 0.f;
+      if (in) {
+        const uint8_t* p = wrow[nb] + (int64_t)ks * (BYTE_CODES ? 128 : 64);
+        s.w[nb].a = *reinterpret_cast<const uint4*>(p);
+        if constexpr (BYTE_CODES) s.w[nb].b = *reinterpret_cast<const uint4*>(p + 16);
+        s.sc[nb] = fused_scale<FMT>(wsc[nb], k0);
+      }
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        s.x[mb][j] = __builtin_bit_cast(
+            uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                       rx, (int)(in ? xoff[mb] + (uint32_t)ks * 256 + 16 * j : 0x7FFFFFF0u), 0, 0));
+  };
+  v4f acc[MB][NB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = (v4f){0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](const Stage& s) {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      const StepDecode<FMT> d = decode_begin<FMT>(s.sc[nb]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const v8bf wv = __builtin_bit_cast(v8bf, decode8<FMT>(d, s.w[nb], j));
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+          acc[mb][nb] =
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, __builtin_bit_cast(v8bf, s.x[mb][j]), acc[mb][nb], 0, 0, 0);
+      }
+    }
+  };
+  if (ks0 < ks1) {
+    Stage s0, s1;
+    load(s0, ks0);
+    for (int ks = ks0; ks < ks1; ks += 2) {
+      if (ks + 1 < ks1) load(s1, ks + 1);
+      compute(s0);
+      if (ks + 1 < ks1) {
+        if (ks + 2 < ks1) load(s0, ks + 2);
+        compute(s1);
+      }
+    }
+  }
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) red[wave][mb * NB + nb][lane] = acc[mb][nb];
+  __syncthreads();
+  // lane l of block (mb, nb) holds row m0 + 16*mb + l%16, columns n0 + 16*nb + 4*(l/16) + 0..3
+  for (int q = threadIdx.x; q < MB * NB * 64; q += 64 * WK) {
+    const int b = q >> 6, l = q & 63;
+    v4f v = red[0][b][l];
+#pragma unroll
+    for (int w = 1; w < WK; ++w) v += red[w][b][l];
+    const int64_t m = m0 + (b / NB) * 16 + (l & 15);
+    const int64_t n = n0 + (b % NB) * 16 + (l >> 4) * 4;
+    if (m >= g.M || n >= g.N) continue;
+    if (g.bias) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] += load_elem(g.bias, g.bias_dtype, min<int64_t>(n + i, g.N - 1));
+    }
+    if (g.vec_out && n + 4 <= g.N && g.y_dtype == DT_BF16) {
+      const v2bf p0 = {(__bf16)v[0], (__bf16)v[1]}, p1 = {(__bf16)v[2], (__bf16)v[3]};
+      *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(g.y) + m * g.ldy + n) =
+          make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (n + i < g.N) store_elem(g.y, g.y_dtype, m * g.ldy + n + i, v[i]);
+    }
+  }
+}
+
 }  // namespace ntlb
 
 using namespace ntlb;
@@ -1454,6 +1586,45 @@ extern "C" int ntlb_mxfp4_dequant(const uint8_t* packed, const uint8_t* scales, 
 // the split-K tail's minimum K blocks (64 bf16 each) per range
 constexpr int FUSED_SPLIT_MIN_BLOCKS = 9;
 
+// Which products run on gemm_lowbit_rows_kernel, and with which tile
+// (mb = 0: the 256x256-tile kernel).  The smallest tile whose workgroups all
+// fit on the chip at once: smaller ones re-read the activations more often,
+// larger ones leave compute units idle.  Measured (NF4, K 4096, in a graph;
+// rows kernel / 256x256 tiles with their split tail, us): N 4096: 8.5 / 46 at
+// 16 rows, 15.8 / 46 at 64, 29.8 / 48 at 256, 57 / 55 at 512; N 14336: 18.6 /
+// 56 at 16 rows, 23.5 / 56 at 32, 30.5 / 56 at 64, 58 / 57 at 128; N = K = 1024:
+// 4.0 / 27 at 16 rows, 12.4 / 28 at 1024.  So past 64 rows the line lies where
+// 64x64 tiles no longer fit at once; up to 64 rows the weight is read once and
+// the rows kernel is ahead at every N.
+struct RowsPlan {
+  int mb, nb, wk;
+};
+static RowsPlan rows_plan(int64_t M, int64_t N) {
+  const int64_t cus = split_device_cus();
+  auto fits = [&](int mb, int nb) { return cdiv(M, 16 * mb) * cdiv(N, 16 * nb) <= cus; };
+  if (fits(1, 1)) return {1, 1, 8};
+  if (fits(1, 2)) return {1, 2, 8};
+  if (M <= 16) return {1, 4, 8};
+  if (fits(2, 2)) return {2, 2, 8};
+  if (M <= 32 || fits(2, 4)) return {2, 4, 8};
+  if (M <= 64 || fits(4, 4)) return {4, 4, 4};
+  return {0, 0, 0};
+}
+
+template <int FMT>
+static void rows_launch(const FusedArgs& g, const RowsPlan& p, hipStream_t st) {
+  const dim3 grd((unsigned)cdiv(g.N, 16 * p.nb), (unsigned)cdiv(g.M, 16 * p.mb)), blk(64 * p.wk);
+#define NTLB_ROWS_CASE(MB, NB, WK) \
+  if (p.mb == MB && p.nb == NB && p.wk == WK) gemm_lowbit_rows_kernel<FMT, MB, NB, WK><<<grd, blk, 0, st>>>(g)
+  NTLB_ROWS_CASE(1, 1, 8);
+  NTLB_ROWS_CASE(1, 2, 8);
+  NTLB_ROWS_CASE(1, 4, 8);
+  NTLB_ROWS_CASE(2, 2, 8);
+  NTLB_ROWS_CASE(2, 4, 8);
+  NTLB_ROWS_CASE(4, 4, 4);
+#undef NTLB_ROWS_CASE
+}
+
 static int fused_launch(int fmt, const char* fn, const void* x, int64_t ldx, const uint8_t* w, const void* scales,
                         int64_t block, const void* bias, int bias_dtype, int64_t M, int64_t N, int64_t K, void* y,
                         int y_dtype, int64_t ldy, void* workspace, int64_t ws_bytes, void* stream) {
@@ -1477,9 +1648,19 @@ static int fused_launch(int fmt, const char* fn, const void* x, int64_t ldx, con
   g.vec_out = aligned(y, 16) && ((ldy * dtype_size(y_dtype)) % 16 == 0);
   g.bias = bias; g.bias_dtype = bias_dtype;
   g.split_base = (int)tiles; g.split_s = 1; g.ws = nullptr; g.ws_count = nullptr;
+  if (workspace && !aligned(workspace, 256)) return fail(NTLB_EINVAL, "%s: workspace must be 256-byte aligned", fn);
+  const RowsPlan rp = rows_plan(M, N);
+  if (rp.mb) {
+    if (fmt == FMT_NF4)
+      rows_launch<FMT_NF4>(g, rp, as_stream(stream));
+    else if (fmt == FMT_MXFP4)
+      rows_launch<FMT_MXFP4>(g, rp, as_stream(stream));
+    else
+      rows_launch<FMT_FP8P>(g, rp, as_stream(stream));
+    return check_launch(fn);
+  }
   int64_t grid_wgs = tiles;
   if (workspace) {
-    if (!aligned(workspace, 256)) return fail(NTLB_EINVAL, "%s: workspace must be 256-byte aligned", fn);
     const SplitPlan plan = split_plan(tiles, (int)(K / FBK), FUSED_SPLIT_MIN_BLOCKS);
     if (plan.s > 1 && ws_bytes >= split_ws_bytes(plan)) {
       g.split_base = plan.base; g.split_s = plan.s;
@@ -1520,7 +1701,7 @@ extern "C" int ntlb_gemm_mxfp4(const void* x, int64_t ldx, const uint8_t* w_pack
 }
 
 extern "C" int64_t ntlb_gemm_lowbit_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % FBK) return 0;
+  if (M <= 0 || N <= 0 || K <= 0 || K % FBK || rows_plan(M, N).mb) return 0;
   const int64_t tiles = ((M + FBM - 1) / FBM) * ((N + FBN - 1) / FBN);
   if (tiles > 0x7FFFFFFF) return 0;
   return split_ws_bytes(split_plan(tiles, (int)(K / FBK), FUSED_SPLIT_MIN_BLOCKS));

@@ -667,3 +667,39 @@ def test_row_quantizer_edges(gpu_device, K, dtype):
     c_ref, s_ref = O.fp8_persistent_quant(to_np32(w), K)
     assert_bits_equal(codes.view(torch.uint8).cpu().numpy().reshape(-1), c_ref.reshape(-1), "fp8 codes")
     assert_bits_equal(scale.reshape(-1).cpu().numpy(), s_ref, "fp8 scale")
+
+
+@pytest.mark.parametrize("fmt", ["nf4", "mxfp4", "fp8p"])
+@pytest.mark.parametrize("M,N,K", [(1, 9, 64), (16, 4096, 192), (5, 8200, 128), (16, 16500, 64), (40, 3000, 320),
+                                   (64, 8200, 192), (200, 1100, 704)])
+def test_few_row_gemm_tiles(gpu_device, fmt, M, N, K):
+    """The few-row kernel at each of its output tiles (16x16 to 64x64), with
+    ragged last tiles, fewer 128-K steps than waves, and K an odd multiple of
+    64, against float64; fp32 output, so that the bound is that of the fp32
+    sums (K terms of at most 2^-24 relative each, a fraction of it measured)
+    and a dropped or doubled term shows; the bf16 output with a bias is the
+    rounding of that sum plus the bias."""
+    from lowbit import persistent as P
+
+    x = seeded((M, K), seed=20261950 + M).to(gpu_device)
+    w = seeded((N, K), seed=20261951 + N, std=0.02).to(gpu_device)
+    bias = seeded((N,), seed=20261952, std=0.5).to(gpu_device)
+    if fmt == "nf4":
+        c, s = P.quantize_nf4_blocks(w, 64)
+        run = lambda b, od: P.linear_nf4(x, c, s, out_features=N, block=64, bias=b, out_dtype=od)
+        deq = P.dequantize_nf4_blocks(c, s, num_values=N * K, block=64, target_dtype=torch.bfloat16)
+    elif fmt == "mxfp4":
+        c, s = P.quantize_mxfp4(w)
+        run = lambda b, od: P.linear_mxfp4(x, c, s, out_features=N, bias=b, out_dtype=od)
+        deq = P.dequantize_mxfp4(c, s, num_values=N * K, target_dtype=torch.bfloat16)
+    else:
+        c, s = P.quantize_fp8_persistent(w, granularity="per_channel")
+        run = lambda b, od: P.linear_fp8p(x, c, s, bias=b, out_dtype=od)
+        deq = P.dequantize_fp8_persistent(c, s, target_dtype=torch.bfloat16)
+    ref = torch.from_numpy(O.gemm_ref(to_np32(x), to_np32(deq).reshape(N, K))).double()
+    y = run(None, torch.float32).cpu().double()
+    assert float((y - ref).norm() / ref.norm()) <= K ** 0.5 * 2.0 ** -23
+    assert float((y - ref).abs().max() / ref.abs().max()) <= K * 2.0 ** -24
+    yb = run(bias, torch.bfloat16).cpu()
+    want = (run(None, torch.float32).cpu() + bias.cpu().float()).to(torch.bfloat16)
+    assert torch.equal(yb, want)
