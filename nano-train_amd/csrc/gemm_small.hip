@@ -1,0 +1,500 @@
+// Blockwise-scaled GEMM of few rows or few output tiles (the products that
+// leave most of the chip idle on 256x256 tiles): same operands, scales and
+// promotion as gemm.hip, output tiles of 16*MB x 16*NB.
+//
+// A workgroup of WK waves owns one tile and each wave multiplies the whole
+// tile over its own range of K blocks, so no wave waits for another before
+// the end; the WK partial tiles are summed in wave order through LDS.  A wave
+// copies its operand rows global -> LDS (16 bytes per lane, eight consecutive
+// lanes on one 128-byte row of a K block: reading the fragments straight from
+// global memory puts neighbouring lanes on different rows and costs four
+// times the address cycles), NS stages deep, into LDS that it alone reads, so
+// the K loop has no barrier: a stage is waited for with vmcnt.
+//
+// What bounds it: with few rows the weight codes' stream (every code is read
+// once, N / (16 NB) workgroups of 8 waves); with more rows the operands'
+// re-reads from L2 (each tile reads 16 (MB + NB) rows of K bytes).
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "ntlb_gemm_tile.h"
+#include "ntlb_host.h"
+#include "ntlb_splitk.h"
+
+namespace ntlb {
+
+// s_waitcnt with only vmcnt set
+constexpr int vmcnt_imm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
+
+// One wave's copies of a 16*MB-row A and 16*NB-row B K block into LDS: copy t
+// moves rows 8t .. 8t+7 (lane i: row i/8, physical chunk i%8, which holds the
+// logical chunk (i%8) ^ swz_perm(row); bit 3 of the row is t & 1).  Rows past
+// the matrix lie beyond the resource and read zero.
+template <int MB, int NB>
+struct WaveCopy {
+  static constexpr int COPIES = 2 * (MB + NB);
+  static constexpr int BYTES = (MB + NB) * 16 * BK;
+  __amdgpu_buffer_rsrc_t ra, rb;
+  uint32_t a0, a1, b0, b1;  // byte offsets of this lane's chunk for even and odd copies
+  uint32_t a16, b16;        // 16 rows in bytes
+  __device__ __forceinline__ void init(const GemmArgs& g, int64_t m0, int64_t n0, int lane) {
+    const int r = lane >> 3, c = lane & 7;
+    ra = __builtin_amdgcn_make_buffer_rsrc((void*)g.a, (short)0, (int)(g.M * g.lda), 0x00020000);
+    rb = __builtin_amdgcn_make_buffer_rsrc((void*)g.b, (short)0, (int)(g.N * g.ldb), 0x00020000);
+    a0 = (uint32_t)((m0 + r) * g.lda + ((c ^ swz_perm(r)) << 4));
+    a1 = (uint32_t)((m0 + 8 + r) * g.lda + ((c ^ swz_perm(8 + r)) << 4));
+    b0 = (uint32_t)((n0 + r) * g.ldb + ((c ^ swz_perm(r)) << 4));
+    b1 = (uint32_t)((n0 + 8 + r) * g.ldb + ((c ^ swz_perm(8 + r)) << 4));
+    a16 = (uint32_t)(16 * g.lda);
+    b16 = (uint32_t)(16 * g.ldb);
+  }
+  // A rows at lds, B rows after them
+  __device__ __forceinline__ void issue(uint8_t* lds, int kb) const {
+    const uint32_t k = (uint32_t)kb * BK;
+#pragma unroll
+    for (int t = 0; t < 2 * MB; ++t)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(lds + t * 8 * BK), 16, (t & 1) ? a1 : a0,
+                                               k + (t >> 1) * a16, 0, 0);
+#pragma unroll
+    for (int t = 0; t < 2 * NB; ++t)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(lds + (16 * MB + t * 8) * BK), 16,
+                                               (t & 1) ? b1 : b0, k + (t >> 1) * b16, 0, 0);
+  }
+};
+
+// The K loop of one wave over blocks [kb0, kb1), kb0 < kb1: acc += the
+// promoted partials.  s0 / s1 / s2 are this wave's stages (distinct LDS
+// objects, so that the copies in flight are seen not to alias the reads).
+template <int GRID, bool B_UNIFORM, int MB, int NB, int NS>
+__device__ __forceinline__ void small_k_loop(const GemmArgs& g, const WaveCopy<MB, NB>& cp, int64_t m0, int64_t n0,
+                                             int kb0, int kb1, uint8_t* s0, uint8_t* s1, uint8_t* s2, int lane,
+                                             v4f (&acc)[MB][NB]) {
+  const int li = lane & 15, gq = lane >> 4;
+  const float* sap[MB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+    sap[mb] = g.sa + (min<int64_t>(m0 + mb * 16 + li, g.M - 1) >> g.a_shift) * g.sa_row;
+  // B's scale: one per block for 128x128 blocks and tensor scales, else one
+  // per column (this lane's columns 4*gq .. 4*gq+3 of each 16)
+  const float* sbu = g.sb + (n0 >> g.b_shift) * g.sb_row;
+  float sam[NS][MB];
+  float sb1[NS];
+  v4f sbv[NS][B_UNIFORM ? 1 : NB];
+  auto stage = [&](int i) { return i == 0 ? s0 : i == 1 ? s1 : s2; };
+  auto issue = [&](auto ic, int kb) {
+    constexpr int I = decltype(ic)::value;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) sam[I][mb] = sap[mb][(int64_t)kb * g.sa_col];
+    if constexpr (B_UNIFORM) {
+      sb1[I] = sbu[(int64_t)kb * g.sb_col];
+    } else {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          sbv[I][nb][q] = g.sb[(min<int64_t>(n0 + nb * 16 + gq * 4 + q, g.N - 1) >> g.b_shift) * g.sb_row +
+                               (int64_t)kb * g.sb_col];
+    }
+    cp.issue(stage(I), kb);
+  };
+  auto compute = [&](auto ic) {
+    constexpr int I = decltype(ic)::value;
+    const uint8_t* ta = stage(I);
+    const uint8_t* tb = ta + 16 * MB * BK;
+    // the scales become visible here: a product of them moved up to an
+    // earlier step would wait for loads younger than that step's copies
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) asm volatile("" : "+v"(sam[I][mb]));
+    if constexpr (B_UNIFORM) {
+      asm volatile("" : "+v"(sb1[I]));
+    } else {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) asm volatile("" : "+v"(sbv[I][nb]));
+    }
+    v8i bf[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) bf[nb] = load_frag(tb, nb * 16, lane);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const v8i af = load_frag(ta, mb * 16, lane);
+      raw_t<GRID> d[NB];
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) d[nb] = mma_raw<GRID>(bf[nb], af);
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        if constexpr (B_UNIFORM) {
+          const float s = sam[I][mb] * sb1[I];
+          acc[mb][nb] += raw_f32<GRID>(d[nb]) * s;
+        } else {
+          acc[mb][nb] += (raw_f32<GRID>(d[nb]) * sbv[I][nb]) * sam[I][mb];
+        }
+      }
+    }
+  };
+  auto each = [](auto f) {
+    f(std::integral_constant<int, 0>());
+    f(std::integral_constant<int, 1>());
+    if constexpr (NS > 2) f(std::integral_constant<int, 2>());
+  };
+  // the first NS - 1 blocks (past the end: the last block again, never read)
+  each([&](auto ic) {
+    if constexpr (decltype(ic)::value < NS - 1) issue(ic, min(kb0 + decltype(ic)::value, kb1 - 1));
+  });
+  auto step = [&](auto ic, int kb) {
+    constexpr int I = decltype(ic)::value;
+    // this wave's reads of the stage refilled now are done (lgkmcnt(0))
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    asm volatile("" ::: "memory");
+    issue(std::integral_constant<int, (I + NS - 1) % NS>(), min(kb + NS - 1, kb1 - 1));
+    // loads return in order: with at most the younger stages' copies
+    // outstanding, this stage has landed
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 1) * WaveCopy<MB, NB>::COPIES));
+    asm volatile("" ::: "memory");
+    compute(ic);
+  };
+  int kb = kb0;
+  for (; kb + NS <= kb1; kb += NS) each([&](auto ic) { step(ic, kb + decltype(ic)::value); });
+  each([&](auto ic) {
+    if (kb + decltype(ic)::value < kb1) step(ic, kb + decltype(ic)::value);
+  });
+  // nothing of this wave is in flight into LDS past here
+  __builtin_amdgcn_s_waitcnt(0);
+  asm volatile("" ::: "memory");
+}
+
+// Row m, columns n .. n+3 of the output (bias, NaN flags, output type)
+__device__ __forceinline__ void small_store4(const GemmArgs& g, int64_t m, int64_t n, v4f v, const int32_t* nan_b) {
+  if (g.bias) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] += load_elem(g.bias, g.bias_dtype, min<int64_t>(n + q, g.N - 1));
+  }
+  const float qnan = __uint_as_float(0x7FC00000u);
+  if (g.nan_a && g.nan_a[m]) v = (v4f){qnan, qnan, qnan, qnan};
+  if (nan_b) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (nan_b[min<int64_t>(n + q, g.N - 1)]) v[q] = qnan;
+  }
+  if (g.vec_out && n + 4 <= g.N && g.y_dtype == DT_BF16) {
+    const v2bf p0 = {(__bf16)v[0], (__bf16)v[1]}, p1 = {(__bf16)v[2], (__bf16)v[3]};
+    *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(g.y) + m * g.ldy + n) =
+        make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (n + q < g.N) store_elem(g.y, g.y_dtype, m * g.ldy + n + q, v[q]);
+}
+
+template <int GRID, bool B_UNIFORM, int MB, int NB, int WK, int NS>
+__global__ void __launch_bounds__(64 * WK) gemm_small_kernel(GemmArgs g) {
+  constexpr int WB = WaveCopy<MB, NB>::BYTES;
+  static_assert(MB * NB * 1024 <= WB, "the partial tiles fit the first stage");
+  __shared__ __attribute__((aligned(16))) uint8_t st0[WK * WB];
+  __shared__ __attribute__((aligned(16))) uint8_t st1[WK * WB];
+  __shared__ __attribute__((aligned(16))) uint8_t st2[NS > 2 ? WK * WB : 16];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t n0 = (int64_t)blockIdx.x * (16 * NB), m0 = (int64_t)blockIdx.y * (16 * MB);
+  const int nk = (int)(g.Kp / BK);
+  const int kb0 = (int)((int64_t)wave * nk / WK), kb1 = (int)((int64_t)(wave + 1) * nk / WK);
+  v4f acc[MB][NB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = (v4f){0.f, 0.f, 0.f, 0.f};
+  if (kb0 < kb1) {
+    WaveCopy<MB, NB> cp;
+    cp.init(g, m0, n0, lane);
+    small_k_loop<GRID, B_UNIFORM, MB, NB, NS>(g, cp, m0, n0, kb0, kb1, st0 + wave * WB, st1 + wave * WB,
+                                              st2 + (NS > 2 ? wave * WB : 0), lane, acc);
+  }
+  __syncthreads();  // every wave is done with its stages: the partials go where the first one was
+  v4f* red = reinterpret_cast<v4f*>(st0);
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) red[(wave * MB * NB + mb * NB + nb) * 64 + lane] = acc[mb][nb];
+  __syncthreads();
+  // lane l of block (mb, nb) holds row m0 + 16*mb + l%16, columns n0 + 16*nb + 4*(l/16) + 0..3
+  for (int q = threadIdx.x; q < MB * NB * 64; q += 64 * WK) {
+    const int b = q >> 6, l = q & 63;
+    v4f v = red[q];
+#pragma unroll
+    for (int w = 1; w < WK; ++w) v += red[w * MB * NB * 64 + q];
+    const int64_t m = m0 + (b / NB) * 16 + (l & 15);
+    const int64_t n = n0 + (b % NB) * 16 + (l >> 4) * 4;
+    if (m < g.M && n < g.N) small_store4(g, m, n, v, g.nan_b);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// 128x128 tiles: four waves as 2 (M) x 2 (N), each 64x64, both operands of a K
+// block staged once per workgroup (32 KiB, double buffered), two workgroups
+// per compute unit.  For products whose 256x256 tiles do not fill the chip
+// (or leave a last wave of tiles mostly empty) but which are too large for
+// 64x64 tiles: per 16x16x128 MFMA a wave reads 1 KiB of LDS (0.75 on the
+// 256x256 tiles' 128x64 waves), which at the MFMA rate is the LDS bandwidth.
+// ---------------------------------------------------------------------------
+constexpr int MID = 128;
+constexpr int MID_TILE = MID * BK;  // 16 KiB per operand stage
+
+template <int GRID, bool B_UNIFORM, int ODT>
+__global__ void __launch_bounds__(256, 2) gemm_mid_kernel(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) uint8_t la0[MID_TILE];
+  __shared__ __attribute__((aligned(16))) uint8_t lb0[MID_TILE];
+  __shared__ __attribute__((aligned(16))) uint8_t la1[MID_TILE];
+  __shared__ __attribute__((aligned(16))) uint8_t lb1[MID_TILE];
+  __shared__ float ls0[2 * MID], ls1[2 * MID];  // A row scales, then B row scales
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  // each XCD walks a contiguous range of a raster of four row tiles
+  const int num_n = (int)((g.N + MID - 1) / MID), num_m = (int)((g.M + MID - 1) / MID);
+  int64_t m0, n0;
+  {
+    const int nwg = (int)gridDim.x, xcd = (int)blockIdx.x & 7, local = (int)blockIdx.x >> 3;
+    const int per = nwg >> 3, extra = nwg & 7;
+    const int pid = xcd * per + min(xcd, extra) + local;
+    constexpr int GROUP_M = 4;
+    const int group = pid / (GROUP_M * num_n);
+    const int gsize = min(num_m - group * GROUP_M, GROUP_M);
+    const int in_group = pid - group * GROUP_M * num_n;
+    m0 = (int64_t)(group * GROUP_M + in_group % gsize) * MID;
+    n0 = (int64_t)(in_group / gsize) * MID;
+  }
+  const bool own_a = tid < MID;
+  const int64_t srow = own_a ? min<int64_t>(m0 + tid, g.M - 1) : min<int64_t>(n0 + tid - MID, g.N - 1);
+  const float* s_src = own_a ? g.sa + (srow >> g.a_shift) * g.sa_row : g.sb + (srow >> g.b_shift) * g.sb_row;
+  const int64_t s_step = own_a ? g.sa_col : g.sb_col;
+  // wave w copies the 8-row groups w, w+4, w+8, w+12 of each operand (bit 3 of
+  // their rows is w & 1, so a lane's chunk is the same in all four)
+  const __amdgpu_buffer_rsrc_t ra =
+      __builtin_amdgcn_make_buffer_rsrc((void*)g.a, (short)0, (int)(g.M * g.lda), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb =
+      __builtin_amdgcn_make_buffer_rsrc((void*)g.b, (short)0, (int)(g.N * g.ldb), 0x00020000);
+  const int cr = wave * 8 + (lane >> 3), cc = (lane & 7) ^ swz_perm(cr);
+  const uint32_t a_off = (uint32_t)((m0 + cr) * g.lda + cc * 16), b_off = (uint32_t)((n0 + cr) * g.ldb + cc * 16);
+  const uint32_t a_grp = (uint32_t)(32 * g.lda), b_grp = (uint32_t)(32 * g.ldb);
+  auto issue = [&](uint8_t* la, uint8_t* lb, int kt, int j) {
+    const uint32_t k = (uint32_t)kt * BK;
+    const int r0 = (wave + 4 * j) * 8;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(la + r0 * BK), 16, a_off, k + j * a_grp, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(lb + r0 * BK), 16, b_off, k + j * b_grp, 0, 0);
+  };
+  const int nk = (int)(g.Kp / BK);
+  v4f acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) issue(la0, lb0, 0, j);
+  ls0[tid] = s_src[0];
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+
+  auto step = [&](auto bufc, int kt) {
+    constexpr int BUF = decltype(bufc)::value;
+    const uint8_t* ta = BUF ? la1 : la0;
+    const uint8_t* tb = BUF ? lb1 : lb0;
+    const float* s_cur = BUF ? ls1 : ls0;
+    // the last block copies itself into the idle stage: one basic block
+    const int kn = min(kt + 1, nk - 1);
+    const float s_next = s_src[(int64_t)kn * s_step];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) issue(BUF ? la0 : la1, BUF ? lb0 : lb1, kn, j);
+    v8i bf[4];
+#pragma unroll
+    for (int tn = 0; tn < 4; ++tn) bf[tn] = load_frag(tb, wn * 64 + tn * 16, lane);
+    float sam[4], sbu = 0.f;
+    v4f sbv[B_UNIFORM ? 1 : 4];
+#pragma unroll
+    for (int tm = 0; tm < 4; ++tm) sam[tm] = s_cur[wm * 64 + tm * 16 + (lane & 15)];
+    if constexpr (B_UNIFORM) {
+      sbu = s_cur[MID + wn * 64];
+    } else {
+#pragma unroll
+      for (int tn = 0; tn < 4; ++tn)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sbv[tn][q] = s_cur[MID + wn * 64 + tn * 16 + (lane >> 4) * 4 + q];
+    }
+    // as the 256x256 kernel: group tm's MFMAs are issued before group tm-1's
+    // results are promoted
+    raw_t<GRID> dp[4];
+#pragma unroll
+    for (int tm = 0; tm < 5; ++tm) {
+      raw_t<GRID> d[4];
+      if (tm < 4) {
+        const v8i af = load_frag(ta, wm * 64 + tm * 16, lane);
+#pragma unroll
+        for (int tn = 0; tn < 4; ++tn) d[tn] = mma_raw<GRID>(bf[tn], af);
+      }
+      if (tm > 0) {
+#pragma unroll
+        for (int tn = 0; tn < 4; ++tn) {
+          if constexpr (B_UNIFORM)
+            acc[tm - 1][tn] += raw_f32<GRID>(dp[tn]) * (sam[tm - 1] * sbu);
+          else
+            acc[tm - 1][tn] += (raw_f32<GRID>(dp[tn]) * sbv[tn]) * sam[tm - 1];
+        }
+      }
+      if (tm < 4) {
+#pragma unroll
+        for (int tn = 0; tn < 4; ++tn) dp[tn] = d[tn];
+      }
+    }
+    (BUF ? ls0 : ls1)[tid] = s_next;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+  };
+  for (int kt = 0; kt < nk; kt += 2) {
+    step(std::integral_constant<int, 0>(), kt);
+    if (kt + 1 < nk) step(std::integral_constant<int, 1>(), kt + 1);
+  }
+
+  // epilogue: each wave stages 32 of its 64 rows at a time in its 16 KiB of the
+  // idle stages and stores whole 128-byte (fp32: 256-byte) row segments
+  uint8_t* stage_w = wave == 0 ? la0 : wave == 1 ? lb0 : wave == 2 ? la1 : lb1;
+  constexpr int esz = ODT == DT_F32 ? 4 : 2, pitch = 64 * esz + 16, cpr = 64 * esz / 16, epc = 16 / esz;
+  static_assert(32 * pitch <= MID_TILE, "staged rows fit a stage");
+  const float qnan = __uint_as_float(0x7FC00000u);
+#pragma unroll
+  for (int part = 0; part < 2; ++part) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int tm = part * 2 + t;
+      const bool nan_m = g.nan_a && g.nan_a[min<int64_t>(m0 + wm * 64 + tm * 16 + (lane & 15), g.M - 1)] != 0;
+#pragma unroll
+      for (int tn = 0; tn < 4; ++tn) {
+        v4f v = acc[tm][tn];
+        const int64_t n = n0 + wn * 64 + tn * 16 + (lane >> 4) * 4;
+        if (g.bias) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) v[q] += load_elem(g.bias, g.bias_dtype, min<int64_t>(n + q, g.N - 1));
+        }
+        if (g.nan_b) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) v[q] = g.nan_b[min<int64_t>(n + q, g.N - 1)] ? qnan : v[q];
+        }
+        if (nan_m) v = (v4f){qnan, qnan, qnan, qnan};
+        uint8_t* dst = stage_w + (t * 16 + (lane & 15)) * pitch + (tn * 16 + (lane >> 4) * 4) * esz;
+        if constexpr (ODT == DT_F32) {
+          *reinterpret_cast<v4f*>(dst) = v;
+        } else if constexpr (ODT == DT_BF16) {
+          const v2bf p0 = {(__bf16)v[0], (__bf16)v[1]}, p1 = {(__bf16)v[2], (__bf16)v[3]};
+          *reinterpret_cast<uint2*>(dst) =
+              make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
+        } else {
+          const __half h[4] = {f32_to_f16(v[0]), f32_to_f16(v[1]), f32_to_f16(v[2]), f32_to_f16(v[3])};
+          *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(h);
+        }
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's staging writes are done
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < cpr / 2; ++j) {
+      const int q = lane + 64 * j, row = q / cpr, c = q % cpr;
+      const int64_t m = m0 + wm * 64 + part * 32 + row, n = n0 + wn * 64 + c * epc;
+      const uint8_t* src = stage_w + row * pitch + c * 16;
+      if (m >= g.M || n >= g.N) continue;
+      uint8_t* ydst = reinterpret_cast<uint8_t*>(g.y) + (m * g.ldy + n) * esz;
+      if (g.vec_out && n + epc <= g.N) {
+        store16_nt(ydst, src);
+      } else {
+        using E = std::conditional_t<esz == 4, uint32_t, uint16_t>;
+#pragma nounroll
+        for (int e = 0; e < epc && n + e < g.N; ++e)
+          reinterpret_cast<E*>(ydst)[e] = reinterpret_cast<const E*>(src)[e];
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // the re-reads are done before the next part overwrites
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+struct SmallPlan {
+  int mb, nb, wk, ns;
+};
+
+// Which kernel a dense product takes (mb = 8: 128x128 tiles; mb = 0: the
+// 256x256 tiles of gemm.hip).  The smallest tile whose workgroups all run at
+// once (one per compute unit, or two of the 64 KiB ones): a smaller one re-reads
+// the operands more often, a larger one leaves compute units idle.  Measured
+// (e4m3, bf16 out, in a graph, us; this kernel / 256x256 tiles):
+//   N = K = 4096: 5.8 / 30 at 16 rows, 7 / 31 at 48, 9.4 / 33 at 128, 12.6 / 37 at
+//   256, 21 / 41 at 512, 36 / 48 at 1003 (128x128 tiles), 42 / 61 at 2048, 85 /
+//   63 at 4096; N 1541, K 1000: 3.6 / 15 at 16 rows, 14.5 / 28 at 1003, 19 / 29
+//   at 2048, 26 / 34 at 4096; N 18432, K 7168: 30 / 64 at 16 rows, 41 / 64 at 48,
+//   79 / 67 at 128.
+// Between 128x128 and 256x256 tiles the two estimates decide: 1.3 us a K block
+// for a chip full of 128x128 tiles, 1.75 us for 256x256 tiles plus 10 us around
+// the loop, or 30 us where a split-K tail exchanges partial tiles.
+static SmallPlan small_plan(int64_t M, int64_t N, int nk) {
+  const int64_t cus = split_device_cus();
+  auto wgs = [&](int64_t rows, int64_t cols) { return cdiv(M, rows) * cdiv(N, cols); };
+  // up to four K blocks there is nothing to divide among waves: one wave per
+  // tile, its blocks in order (N 4096, K 256: 3.0 / 9.0 at 16 rows, 4.2 / 9.2 at
+  // 128, 6.6 / 10.2 at 300; N 1541, K 384: 10.3 / 22 at 1003 rows, where
+  // 128x128 tiles take 14)
+  if (nk <= 4 && wgs(16, 16) <= 24 * cus) return {1, 1, 1, 3};
+  if (wgs(16, 16) <= cus) return {1, 1, 8, 2};
+  if (wgs(16, 32) <= cus || M <= 16) return {1, 2, 4, 3};
+  if (wgs(32, 32) <= cus) return {2, 2, 4, 3};
+  if (wgs(32, 64) <= cus) return {2, 4, 4, 3};
+  if (wgs(64, 64) <= cus) return {4, 4, 4, 2};
+  if (wgs(64, 64) <= 2 * cus) return {4, 4, 2, 2};
+  if (wgs(MID, MID) <= 2 * cus) {
+    const SplitPlan sp = split_plan(wgs(256, 256), nk, SPLIT_MIN_BLOCKS);
+    const double mid = 1.3 * nk + 4, big = 1.75 * nk / sp.s + (sp.s > 1 ? 30 : 10);
+    if (mid < big) return {8, 8, 4, 2};
+  }
+  return {0, 0, 0, 0};
+}
+
+bool small_gemm_fits(int64_t M, int64_t N, int64_t Kp) { return small_plan(M, N, (int)(Kp / BK)).mb != 0; }
+
+template <int GRID, bool B_UNIFORM>
+static void small_launch(const SmallPlan& p, const GemmArgs& g, hipStream_t st) {
+  if (p.mb == 8) {
+    const dim3 grd((unsigned)(cdiv(g.M, MID) * cdiv(g.N, MID))), blk(256);
+    if (g.y_dtype == DT_F32)
+      gemm_mid_kernel<GRID, B_UNIFORM, DT_F32><<<grd, blk, 0, st>>>(g);
+    else if (g.y_dtype == DT_F16)
+      gemm_mid_kernel<GRID, B_UNIFORM, DT_F16><<<grd, blk, 0, st>>>(g);
+    else
+      gemm_mid_kernel<GRID, B_UNIFORM, DT_BF16><<<grd, blk, 0, st>>>(g);
+    return;
+  }
+  const dim3 grd((unsigned)cdiv(g.N, 16 * p.nb), (unsigned)cdiv(g.M, 16 * p.mb)), blk(64 * p.wk);
+#define NTLB_SMALL_CASE(MB, NB, WK, NS)                                                      \
+  if (p.mb == MB && p.nb == NB && p.wk == WK && p.ns == NS) {                                \
+    gemm_small_kernel<GRID, B_UNIFORM, MB, NB, WK, NS><<<grd, blk, 0, st>>>(g);              \
+    return;                                                                                  \
+  }
+  NTLB_SMALL_CASE(1, 1, 1, 3)
+  NTLB_SMALL_CASE(1, 1, 8, 2)
+  NTLB_SMALL_CASE(1, 2, 4, 3)
+  NTLB_SMALL_CASE(2, 2, 4, 3)
+  NTLB_SMALL_CASE(2, 4, 4, 3)
+  NTLB_SMALL_CASE(4, 4, 4, 2)
+  NTLB_SMALL_CASE(4, 4, 2, 2)
+#undef NTLB_SMALL_CASE
+}
+
+void small_gemm_launch(int grid, bool b_uniform, const GemmArgs& g, hipStream_t st) {
+  const SmallPlan p = small_plan(g.M, g.N, (int)(g.Kp / BK));
+  if (grid == GRID_E4M3) {
+    if (b_uniform)
+      small_launch<GRID_E4M3, true>(p, g, st);
+    else
+      small_launch<GRID_E4M3, false>(p, g, st);
+  } else {
+    if (b_uniform)
+      small_launch<GRID_INT, true>(p, g, st);
+    else
+      small_launch<GRID_INT, false>(p, g, st);
+  }
+}
+
+}  // namespace ntlb
