@@ -511,6 +511,49 @@ int ntlb_gemm_grouped_swiglu_quant_gu(int grid, const uint8_t* a, int64_t lda, c
                                       uint64_t offset, uint16_t* gu, int64_t ldgu, void* stream);
 
 /*
+ * One low-bit Linear per call (te_backend.py:229-260 with 1x128 activation
+ * tiles and 128x128 weight blocks): Y = X_dq . W_dq^T + bias over the codes'
+ * fp32 q * s values, its straight-through backward, and the backward with
+ * quantized gradients.  The caller fills the shape fields of a plan (x [M, K]
+ * with row pitch ldx, weight [N, K] with ldw, element dtypes; y has x's dtype)
+ * and ntlb_linear_plan_init the sizes: code_bytes of the code buffer that the
+ * forward writes and the straight-through backward reads, scratch bytes of
+ * each backward, and the bytes of the zeroed split-K workspace each call can
+ * use (as ntlb_gemm_blockscaled_ws; 0 or NULL: none).  A plan holds no
+ * pointers and is not written after its init, so threads and streams may
+ * share it.  Buffers are 256-byte aligned; y, dx and dw are contiguous.
+ */
+typedef struct ntlb_linear_plan {
+  int64_t M, N, K, ldx, ldw;
+  int x_dtype, w_dtype, bias_dtype, grid, qmax, rounding;
+  uint64_t seed;
+  int64_t code_bytes, ste_bytes, ste_pad_bytes, recipe_bytes, forward_ws, ste_ws, recipe_ws;
+} ntlb_linear_plan;
+
+int ntlb_linear_plan_init(ntlb_linear_plan* plan);
+
+/* Forward; the activation draws at Philox offset `offset`, the weight at
+ * offset + 1.  bias optional [N]. */
+int ntlb_linear_forward(const ntlb_linear_plan* plan, const void* x, const void* w, const void* bias, void* codes,
+                        void* y, void* workspace, int64_t ws_bytes, uint64_t offset, void* stream);
+
+/* Straight-through backward of bf16 layers from the forward's code buffer:
+ * dx = dY . bf16(W_dq), dw = dY^T . bf16(X_dq), db = the column sum of dY;
+ * each output optional.  scratch: ste_bytes, or ste_pad_bytes where dY needs a
+ * padded copy (N % 64 != 0, lddy % 8 != 0 or dY not 16-byte aligned). */
+int ntlb_linear_ste_backward(const ntlb_linear_plan* plan, const void* dy, int64_t lddy, const void* codes, void* dx,
+                             void* dw, void* db, int db_dtype, void* scratch, int64_t scratch_bytes, void* workspace,
+                             int64_t ws_bytes, void* stream);
+
+/* Backward with quantized gradients (dY per 1x128 and 128x1 tile at Philox
+ * offset + 2, W at offset + 1, X at offset + 4); dY, dx and dw in x's dtype,
+ * each output optional; scratch: recipe_bytes. */
+int ntlb_linear_recipe_backward(const ntlb_linear_plan* plan, const void* dy, int64_t lddy, const void* x,
+                                const void* w, void* dx, void* dw, void* db, int db_dtype, void* scratch,
+                                int64_t scratch_bytes, void* workspace, int64_t ws_bytes, uint64_t offset,
+                                void* stream);
+
+/*
  * Words of zeroed workspace that ntlb_nf4_quant / ntlb_fp8_persistent_quant of
  * the n elements at w with scale blocks of `block` read: 0 where each block's
  * amax stays inside one workgroup, ceil(n/block) for the two-pass kernels.

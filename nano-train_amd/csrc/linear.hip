@@ -1,0 +1,275 @@
+// One low-bit Linear call per entry point: the launches of a forward, of its
+// straight-through backward and of the quantized-gradient backward, issued
+// from one host call over one code buffer and one scratch buffer
+// (te_backend.py:229-260 and its autograd; the recipe of benchmark config 3).
+// The device work is that of the separate entry points; what this file adds
+// on the device is the zeroing of the NaN row flags (int grid only, one
+// launch for all of them) and the padded copy of a dY whose rows are not whole
+// 64-column steps.
+//
+// NaN row flags: an int-grid code of -128 is an ordinary number to the matrix
+// cores, so the GEMM needs flags.  e4m3 codes carry NaN themselves (0x7F): the
+// MFMA's result is NaN wherever an operand row or column holds one, which is
+// what the flags would write, so e4m3 products run without them.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "ntlb_device.h"
+#include "ntlb_host.h"
+
+namespace ntlb {
+
+__global__ void __launch_bounds__(256) zero_words_kernel(uint32_t* p, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) p[i] = 0u;
+}
+
+// dst [M, ldd] (ldd % 8 == 0, 16-byte aligned) = src [M, N] of 16-bit values,
+// zero past column N.  Eight columns per thread; bound by its 2-byte loads'
+// issue when the rows are not aligned (they are not when this runs).
+__global__ void __launch_bounds__(256) pad_rows16_kernel(const uint16_t* src, int64_t lds, int64_t M, int64_t N,
+                                                         uint16_t* dst, int64_t ldd) {
+  const int64_t per = ldd >> 3;
+  const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (q >= M * per) return;
+  const int64_t m = q / per, c = (q - m * per) * 8;
+  const uint16_t* s = src + m * lds + c;
+  uint32_t w[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t lo = c + 2 * i < N ? s[2 * i] : 0u, hi = c + 2 * i + 1 < N ? s[2 * i + 1] : 0u;
+    w[i] = lo | (hi << 16);
+  }
+  *reinterpret_cast<uint4*>(dst + m * ldd + c) = make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+static int64_t up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
+
+// consecutive 256-byte aligned pieces of a buffer
+struct Carve {
+  int64_t at = 0;
+  int64_t take(int64_t bytes) {
+    const int64_t o = at;
+    at += up(bytes, 256);
+    return o;
+  }
+};
+
+// the code buffer: X codes and scales, W codes and scales, NaN flags of X's
+// then W's rows (int grid)
+struct CodeLayout {
+  int64_t xc, xs, wc, ws, flags, bytes;
+};
+static CodeLayout code_layout(const ntlb_linear_plan& p) {
+  const int64_t kp = up(p.K, 128), T = kp / 128;
+  Carve c;
+  CodeLayout l;
+  l.xc = c.take(p.M * kp);
+  l.xs = c.take(T * up(p.M, 4) * 4);
+  l.wc = c.take(p.N * kp);
+  l.ws = c.take(cdiv(p.N, 128) * T * 4);
+  l.flags = p.grid == NTLB_GRID_INT ? c.take((p.M + p.N) * 4) : -1;
+  l.bytes = c.at;
+  return l;
+}
+
+// the straight-through backward's scratch: the column sum's partials, and the
+// padded dY (only touched where dY needs it)
+struct SteLayout {
+  int64_t colsum, dy, bytes;
+};
+static SteLayout ste_layout(const ntlb_linear_plan& p) {
+  Carve c;
+  SteLayout l;
+  l.colsum = c.take(std::max<int64_t>(ntlb_colsum_workspace_bytes(p.M, p.N), 4));
+  l.dy = c.take(p.M * up(p.N, 64) * 2);
+  l.bytes = c.at;
+  return l;
+}
+
+// the recipe backward's scratch
+struct RecipeLayout {
+  int64_t colsum, yc, ys, ytc, yts, wc, wtc, ws, xtc, xts, flags, bytes;
+};
+static RecipeLayout recipe_layout(const ntlb_linear_plan& p) {
+  const int64_t kp = up(p.K, 128), np = up(p.N, 128), mp = up(p.M, 128);
+  Carve c;
+  RecipeLayout l;
+  l.colsum = c.take(std::max<int64_t>(ntlb_colsum_workspace_bytes(p.M, p.N), 4));
+  l.yc = c.take(p.M * np);
+  l.ys = c.take(np / 128 * up(p.M, 4) * 4);
+  l.ytc = c.take(p.N * mp);
+  l.yts = c.take(mp / 128 * up(p.N, 4) * 4);
+  l.wc = c.take(p.N * kp);
+  l.wtc = c.take(p.K * np);
+  l.ws = c.take(np / 128 * (kp / 128) * 4);
+  l.xtc = c.take(p.K * mp);
+  l.xts = c.take(mp / 128 * up(p.K, 4) * 4);
+  l.flags = p.grid == NTLB_GRID_INT ? c.take((p.M + p.N + p.K) * 4) : -1;
+  l.bytes = c.at;
+  return l;
+}
+
+static int check_plan(const char* fn, const ntlb_linear_plan* p) {
+  if (!p) return fail(NTLB_EINVAL, "%s: NULL plan", fn);
+  if (p->M < 1 || p->N < 1 || p->K < 1 || p->ldx < p->K || p->ldw < p->K)
+    return fail(NTLB_EINVAL, "%s: bad shape or row pitch", fn);
+  if (!valid_dtype(p->x_dtype) || !valid_dtype(p->w_dtype)) return fail(NTLB_EINVAL, "%s: bad dtype", fn);
+  if (p->grid != NTLB_GRID_INT && p->grid != NTLB_GRID_E4M3) return fail(NTLB_EINVAL, "%s: bad grid %d", fn, p->grid);
+  return NTLB_OK;
+}
+
+static void zero_words(void* p, int64_t n, hipStream_t st) {
+  zero_words_kernel<<<(unsigned)cdiv(n, 256), 256, 0, st>>>(reinterpret_cast<uint32_t*>(p), n);
+}
+
+}  // namespace ntlb
+
+using namespace ntlb;
+
+extern "C" int ntlb_linear_plan_init(ntlb_linear_plan* p) {
+  const char* fn = "ntlb_linear_plan_init";
+  if (int rc = check_plan(fn, p)) return rc;
+  const int64_t kp = up(p->K, 128), np = up(p->N, 128), mp = up(p->M, 128);
+  p->code_bytes = code_layout(*p).bytes;
+  p->ste_bytes = ste_layout(*p).dy;
+  p->ste_pad_bytes = ste_layout(*p).bytes;
+  p->recipe_bytes = recipe_layout(*p).bytes;
+  p->forward_ws = ntlb_gemm_workspace_bytes(p->M, p->N, kp);
+  p->ste_ws = ntlb_gemm_dq_workspace_bytes(NTLB_BF16, p->M, p->K, p->N);
+  p->recipe_ws = std::max(ntlb_gemm_workspace_bytes(p->M, p->K, np), ntlb_gemm_workspace_bytes(p->N, p->K, mp));
+  return NTLB_OK;
+}
+
+extern "C" int ntlb_linear_forward(const ntlb_linear_plan* p, const void* x, const void* w, const void* bias,
+                                   void* codes, void* y, void* workspace, int64_t ws_bytes, uint64_t offset,
+                                   void* stream) {
+  const char* fn = "ntlb_linear_forward";
+  if (int rc = check_plan(fn, p)) return rc;
+  if (!x || !w || !codes || !y) return fail(NTLB_EINVAL, "%s: NULL pointer", fn);
+  if (!aligned(codes, 256)) return fail(NTLB_EINVAL, "%s: the code buffer must be 256-byte aligned", fn);
+  const CodeLayout l = code_layout(*p);
+  uint8_t* b = reinterpret_cast<uint8_t*>(codes);
+  const int64_t kp = up(p->K, 128), T = kp / 128, m4 = up(p->M, 4);
+  int32_t* nan_x = l.flags >= 0 ? reinterpret_cast<int32_t*>(b + l.flags) : nullptr;
+  int32_t* nan_w = nan_x ? nan_x + p->M : nullptr;
+  if (nan_x) zero_words(nan_x, p->M + p->N, as_stream(stream));
+  int rc = ntlb_quant_tile_1x128(x, p->x_dtype, p->M, p->K, p->ldx, p->grid, p->qmax, p->rounding,
+                                 NTLB_SCALE_AFTER_DIVIDE, p->seed, offset, b + l.xc, kp,
+                                 reinterpret_cast<float*>(b + l.xs), 1, m4, nullptr, 0, 0, nan_x, stream);
+  if (rc) return rc;
+  rc = ntlb_quant_block_128x128(w, p->w_dtype, p->N, p->K, p->ldw, p->grid, p->qmax, p->rounding,
+                                NTLB_SCALE_AFTER_DIVIDE, p->seed, offset + 1, b + l.wc, kp, nullptr, 0,
+                                reinterpret_cast<float*>(b + l.ws), T, 1, nullptr, 0, 0, nan_w, stream);
+  if (rc) return rc;
+  return ntlb_gemm_blockscaled_ws(p->grid, b + l.xc, kp, reinterpret_cast<const float*>(b + l.xs), 1, m4, 0,
+                                  b + l.wc, kp, reinterpret_cast<const float*>(b + l.ws), T, 1, 7, p->M, p->N, kp,
+                                  bias, p->bias_dtype, y, p->x_dtype, p->N, nan_x, nan_w, workspace, ws_bytes,
+                                  stream);
+}
+
+extern "C" int ntlb_linear_ste_backward(const ntlb_linear_plan* p, const void* dy, int64_t lddy, const void* codes,
+                                        void* dx, void* dw, void* db, int db_dtype, void* scratch,
+                                        int64_t scratch_bytes, void* workspace, int64_t ws_bytes, void* stream) {
+  const char* fn = "ntlb_linear_ste_backward";
+  if (int rc = check_plan(fn, p)) return rc;
+  if (!dy || !scratch || ((dx || dw) && !codes)) return fail(NTLB_EINVAL, "%s: NULL pointer", fn);
+  if (p->x_dtype != NTLB_BF16 || p->w_dtype != NTLB_BF16) return fail(NTLB_EUNSUPPORTED, "%s: bf16 only", fn);
+  if (lddy < p->N) return fail(NTLB_EINVAL, "%s: lddy < N", fn);
+  const CodeLayout l = code_layout(*p);
+  const SteLayout sl = ste_layout(*p);
+  const uint8_t* b = reinterpret_cast<const uint8_t*>(codes);
+  uint8_t* s = reinterpret_cast<uint8_t*>(scratch);
+  const int64_t kp = up(p->K, 128), T = kp / 128, m4 = up(p->M, 4), n64 = up(p->N, 64);
+  const bool pad_dy = p->N % 64 || lddy % 8 || !aligned(dy, 16);
+  if (!aligned(scratch, 256) || scratch_bytes < (pad_dy ? sl.bytes : sl.dy))
+    return fail(NTLB_EINVAL, "%s: the scratch is misaligned or too small", fn);
+  if (pad_dy) {
+    // both GEMMs and the column sum read whole 16-byte chunks of dY's rows,
+    // the dgrad whole 64-column steps: one padded copy serves all three
+    const int64_t q = p->M * (n64 >> 3);
+    if (cdiv(q, 256) > 0x7FFFFFFF) return fail(NTLB_EINVAL, "%s: too large", fn);
+    uint16_t* pad = reinterpret_cast<uint16_t*>(s + sl.dy);
+    pad_rows16_kernel<<<(unsigned)cdiv(q, 256), 256, 0, as_stream(stream)>>>(
+        reinterpret_cast<const uint16_t*>(dy), lddy, p->M, p->N, pad, n64);
+    dy = pad;
+    lddy = n64;
+  }
+  if (dx) {
+    const int rc = ntlb_gemm_ste_dgrad_ws(NTLB_BF16, dy, lddy, p->M, p->N, p->grid, b + l.wc, kp,
+                                          reinterpret_cast<const float*>(b + l.ws), T, 1, 7, p->K, dx, NTLB_BF16,
+                                          p->K, workspace, ws_bytes, stream);
+    if (rc) return rc;
+  }
+  if (dw) {
+    const int rc = ntlb_gemm_ste_wgrad(NTLB_BF16, dy, lddy, p->M, p->N, p->grid, b + l.xc, kp,
+                                       reinterpret_cast<const float*>(b + l.xs), 1, m4, 0, p->K, dw, NTLB_BF16,
+                                       p->K, stream);
+    if (rc) return rc;
+  }
+  if (db)
+    return ntlb_colsum(dy, NTLB_BF16, p->M, p->N, lddy, reinterpret_cast<float*>(s + sl.colsum), sl.dy - sl.colsum,
+                       db, db_dtype, stream);
+  return check_launch(fn);
+}
+
+extern "C" int ntlb_linear_recipe_backward(const ntlb_linear_plan* p, const void* dy, int64_t lddy, const void* x,
+                                           const void* w, void* dx, void* dw, void* db, int db_dtype, void* scratch,
+                                           int64_t scratch_bytes, void* workspace, int64_t ws_bytes,
+                                           uint64_t offset, void* stream) {
+  const char* fn = "ntlb_linear_recipe_backward";
+  if (int rc = check_plan(fn, p)) return rc;
+  if (!dy || !scratch || !x || !w) return fail(NTLB_EINVAL, "%s: NULL pointer", fn);
+  if (lddy < p->N) return fail(NTLB_EINVAL, "%s: lddy < N", fn);
+  const RecipeLayout l = recipe_layout(*p);
+  if (!aligned(scratch, 256) || scratch_bytes < l.bytes)
+    return fail(NTLB_EINVAL, "%s: the scratch is misaligned or too small", fn);
+  uint8_t* b = reinterpret_cast<uint8_t*>(scratch);
+  const int64_t kp = up(p->K, 128), np = up(p->N, 128), mp = up(p->M, 128), T = kp / 128;
+  const int64_t m4 = up(p->M, 4), n4 = up(p->N, 4), k4 = up(p->K, 4);
+  const int rule = NTLB_SCALE_AFTER_DIVIDE, dt = p->x_dtype;
+  int32_t* nan_m = l.flags >= 0 ? reinterpret_cast<int32_t*>(b + l.flags) : nullptr;
+  int32_t* nan_n = nan_m ? nan_m + p->M : nullptr;
+  int32_t* nan_k = nan_m ? nan_n + p->N : nullptr;
+  float* ys = reinterpret_cast<float*>(b + l.ys);
+  float* yts = reinterpret_cast<float*>(b + l.yts);
+  float* wsc = reinterpret_cast<float*>(b + l.ws);
+  float* xts = reinterpret_cast<float*>(b + l.xts);
+  int rc = NTLB_OK;
+  if (nan_m && (dx || dw)) zero_words(nan_m, p->M + p->N + p->K, as_stream(stream));
+  // dY's 1x128 and 128x1 quantizations share one Philox offset: one pass over
+  // dY writes both where its rows allow
+  const bool dual = dx && dw && p->N % 8 == 0 && lddy % 8 == 0 && aligned(dy, 16) && dt != NTLB_F16;
+  if (dual)
+    rc = ntlb_quant_dual_1x128_128x1(dy, dt, p->M, p->N, lddy, p->grid, p->qmax, p->rounding, rule, p->seed,
+                                     offset + 2, offset + 2, b + l.yc, np, ys, 1, m4, nan_m, b + l.ytc, mp, yts, 1,
+                                     n4, nan_n, stream);
+  if (dx && !rc) {
+    if (!dual)
+      rc = ntlb_quant_tile_1x128(dy, dt, p->M, p->N, lddy, p->grid, p->qmax, p->rounding, rule, p->seed, offset + 2,
+                                 b + l.yc, np, ys, 1, m4, nullptr, 0, 0, nan_m, stream);
+    if (!rc)
+      rc = ntlb_quant_block_128x128(w, p->w_dtype, p->N, p->K, p->ldw, p->grid, p->qmax, p->rounding, rule, p->seed,
+                                    offset + 1, b + l.wc, kp, b + l.wtc, np, wsc, T, 1, nullptr, 0, 0, nullptr,
+                                    stream);
+    if (!rc)
+      rc = ntlb_gemm_blockscaled_ws(p->grid, b + l.yc, np, ys, 1, m4, 0, b + l.wtc, np, wsc, 1, T, 7, p->M, p->K, np,
+                                    nullptr, 0, dx, dt, p->K, nan_m, nullptr, workspace, ws_bytes, stream);
+  }
+  if (dw && !rc) {
+    if (!dual)
+      rc = ntlb_quant_tile_128x1_t(dy, dt, p->M, p->N, lddy, p->grid, p->qmax, p->rounding, rule, p->seed,
+                                   offset + 2, b + l.ytc, mp, yts, 1, n4, nullptr, 0, 0, nan_n, stream);
+    if (!rc)
+      rc = ntlb_quant_tile_128x1_t(x, p->x_dtype, p->M, p->K, p->ldx, p->grid, p->qmax, p->rounding, rule, p->seed,
+                                   offset + 4, b + l.xtc, mp, xts, 1, k4, nullptr, 0, 0, nan_k, stream);
+    if (!rc)
+      rc = ntlb_gemm_blockscaled_ws(p->grid, b + l.ytc, mp, yts, 1, n4, 0, b + l.xtc, mp, xts, 1, k4, 0, p->N, p->K,
+                                    mp, nullptr, 0, dw, dt, p->K, nan_n, nan_k, workspace, ws_bytes, stream);
+  }
+  if (db && !rc)
+    rc = ntlb_colsum(dy, dt, p->M, p->N, lddy, reinterpret_cast<float*>(b + l.colsum), l.yc - l.colsum, db, db_dtype,
+                     stream);
+  return rc;
+}

@@ -61,6 +61,10 @@ SIGNATURES = {
     "ntlb_gemm_grouped_swiglu_quant": [_I32, _P, _I64, _P, _I64, _I64, _I32, _P, _I64, _I64, _P, _I64, _I64, _I64,
                                        _P, _I32, _I64, _I64, _I64, _P, _P, _P, _I64, _P, _I64, _P, _I64, _I64, _P,
                                        _I32, _I32, _I32, _U64, _U64, _P],
+    "ntlb_linear_plan_init": [_P],
+    "ntlb_linear_forward": [_P, _P, _P, _P, _P, _P, _P, _I64, _U64, _P],
+    "ntlb_linear_ste_backward": [_P, _P, _I64, _P, _P, _P, _P, _I32, _P, _I64, _P, _I64, _P],
+    "ntlb_linear_recipe_backward": [_P, _P, _I64, _P, _P, _P, _P, _P, _I32, _P, _I64, _P, _I64, _U64, _P],
     "ntlb_persistent_quant_ws_words": [_P, _I64, _I64],
     "ntlb_nf4_quant": [_P, _I32, _I64, _I64, _P, _P, _P, _P],
     "ntlb_nf4_dequant": [_P, _P, _I64, _I64, _P, _I32, _P],
@@ -135,6 +139,16 @@ SIGNATURES = {
     "ntlb_ep_combine_values": [_P, _I64, _I64, _I32, _P, _I32, _P, _I32, _I64, _I64, _P, _I32, _I64, _P, _P],
 }
 
+
+class LinearPlan(ctypes.Structure):
+    """ntlb_linear_plan"""
+
+    _fields_ = [("M", _I64), ("N", _I64), ("K", _I64), ("ldx", _I64), ("ldw", _I64),
+                ("x_dtype", _I32), ("w_dtype", _I32), ("bias_dtype", _I32), ("grid", _I32), ("qmax", _I32),
+                ("rounding", _I32), ("seed", _U64), ("code_bytes", _I64), ("ste_bytes", _I64), ("ste_pad_bytes", _I64),
+                ("recipe_bytes", _I64), ("forward_ws", _I64), ("ste_ws", _I64), ("recipe_ws", _I64)]
+
+
 # entry points that return a value instead of a status
 RESTYPES = {"ntlb_gemm_workspace_bytes": _I64, "ntlb_ep_record_bytes": _I64, "ntlb_colsum_workspace_bytes": _I64,
             "ntlb_ep_value_record_bytes": _I64, "ntlb_persistent_quant_ws_words": _I64,
@@ -175,8 +189,7 @@ def lib() -> ctypes.CDLL:
 
 def call(name: str, *args) -> None:
     """Call an entry point and raise on a non-zero status."""
-    fn = getattr(lib(), name)
-    rc = fn(*args)
+    rc = getattr(_lib or lib(), name)(*args)
     if rc != NTLB_OK:
         msg = lib().ntlb_last_error().decode(errors="replace")
         exc = ValueError if rc == NTLB_EINVAL else LowBitKernelError

@@ -42,6 +42,7 @@ There is no CPU path: CPU tensors raise.
 
 from __future__ import annotations
 
+import ctypes
 import itertools
 import threading
 from typing import Optional
@@ -161,12 +162,121 @@ def _reference_operand(t: torch.Tensor, dq: torch.Tensor, dtype: torch.dtype, sr
     return ops.ste_value(t, dq) if sr else dq
 
 
+class _LinearPlan:
+    """The shape of one linear call for ntlb_linear_forward and its backwards:
+    sizes and layouts, no pointers and no tensors, and constant once made (so
+    calls of any thread or stream share it)."""
+
+    __slots__ = ("c", "ref", "M", "N", "K", "code_bytes", "ws_bytes")
+
+    def __init__(self, M, N, K, ldx, ldw, xdt, wdt, bdt, grid, qmax, rounding, seed) -> None:
+        self.c = _lib.LinearPlan(M=M, N=N, K=K, ldx=ldx, ldw=ldw, x_dtype=ops._dtype_code(xdt),
+                                 w_dtype=ops._dtype_code(wdt), bias_dtype=0 if bdt is None else ops._dtype_code(bdt),
+                                 grid=grid, qmax=qmax, rounding=rounding, seed=seed)
+        self.ref = ctypes.addressof(self.c)
+        self.M, self.N, self.K = M, N, K
+        _lib.call("ntlb_linear_plan_init", self.ref)
+        self.code_bytes = self.c.code_bytes
+        self.ws_bytes = self.c.forward_ws
+
+    def qtensors(self, buf: torch.Tensor):
+        """The code buffer's activation and weight as QTensors (views)."""
+        M, N, K, grid = self.M, self.N, self.K, self.c.grid
+        T, m4 = ops.cdiv(K, 128), ops.cdiv(M, 4) * 4
+        at = 0
+
+        def piece(nbytes):
+            nonlocal at
+            v = buf[at:at + nbytes]
+            at += ops.cdiv(nbytes, 256) * 256
+            return v
+
+        xc = piece(M * T * 128).view(M, T * 128)
+        xs = piece(T * m4 * 4).view(torch.float32).view(T, m4)
+        wc = piece(N * T * 128).view(N, T * 128)
+        ws = piece(ops.cdiv(N, 128) * T * 4).view(torch.float32).view(-1, T)
+        flags = piece((M + N) * 4).view(torch.int32) if grid == _lib.GRID_INT else None
+        nx, nw = (None, None) if flags is None else (flags[:M], flags[M:])
+        return (QTensor(xc, xs, 1, m4, 0, grid, M, K, nx, None), QTensor(wc, ws, T, 1, 7, grid, N, K, nw, None))
+
+
+_MAX_PLANS = 64
+_RECIPE_DTYPES = (torch.bfloat16, torch.float32)
+
+
+def _rows_2d(t: torch.Tensor, cols: int) -> torch.Tensor:
+    """t as [rows, cols] with unit column stride and a row pitch of at least cols"""
+    t2 = t if t.dim() == 2 else t.reshape(-1, cols)
+    s = t2.stride()
+    return t2 if s[1] == 1 and s[0] >= cols else t2.contiguous()
+
+
+def _workspace(need: int, device):
+    ws = ops.split_workspace(need, device)
+    return (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
+
+
+def _ste_backward(plan: _LinearPlan, dy2, buf, needs, x_shape, bias_dtype):
+    """dX, dW, db of the straight-through rule from the forward's code buffer (bf16)"""
+    dev, bf = dy2.device, torch.bfloat16
+    dx = torch.empty(x_shape, dtype=bf, device=dev) if needs[0] else None
+    dw = torch.empty((plan.N, plan.K), dtype=bf, device=dev) if needs[1] else None
+    db = torch.empty((plan.N,), dtype=bias_dtype, device=dev) if needs[2] and bias_dtype is not None else None
+    ld, ptr = dy2.stride(0), dy2.data_ptr()
+    padded = plan.N % 64 != 0 or ld % 8 != 0 or ptr % 16 != 0
+    scratch = torch.empty(plan.c.ste_pad_bytes if padded else plan.c.ste_bytes, dtype=torch.uint8, device=dev)
+    ws, ws_bytes = _workspace(plan.c.ste_ws if needs[0] else 0, dev)
+    _lib.call("ntlb_linear_ste_backward", plan.ref, ptr, ld, None if buf is None else buf.data_ptr(), ops._ptr(dx),
+              ops._ptr(dw), ops._ptr(db), 0 if db is None else ops._dtype_code(bias_dtype), scratch.data_ptr(),
+              scratch.numel(), ws, ws_bytes, ops._stream())
+    return dx, dw, db
+
+
+def _recipe_backward(plan: _LinearPlan, dy2, x2, weight, needs, x_shape, bias_dtype, base):
+    """dX, dW, db of the quantized-gradient recipe; dY, x and weight of one dtype"""
+    dev, dt = dy2.device, dy2.dtype
+    dx = torch.empty(x_shape, dtype=dt, device=dev) if needs[0] else None
+    dw = torch.empty((plan.N, plan.K), dtype=dt, device=dev) if needs[1] else None
+    db = torch.empty((plan.N,), dtype=bias_dtype, device=dev) if needs[2] and bias_dtype is not None else None
+    scratch = torch.empty(plan.c.recipe_bytes, dtype=torch.uint8, device=dev)
+    ws, ws_bytes = _workspace(plan.c.recipe_ws, dev)
+    _lib.call("ntlb_linear_recipe_backward", plan.ref, dy2.data_ptr(), dy2.stride(0), x2.data_ptr(),
+              weight.data_ptr(), ops._ptr(dx), ops._ptr(dw), ops._ptr(db),
+              0 if db is None else ops._dtype_code(bias_dtype), scratch.data_ptr(), scratch.numel(), ws, ws_bytes,
+              base, ops._stream())
+    return dx, dw, db
+
+
 class _HipLowBitLinear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias, backend: "HipLowBitBackend"):
+        needs = ctx.needs_input_grad
         out_dtype = x.dtype
         K = x.shape[-1]
         N = weight.shape[0]
+        ctx.plan = None
+        if backend._one_call(x, weight, bias, needs):
+            x2 = _rows_2d(x, K)
+            plan = backend._plan(x2, weight, bias)
+            base = backend._next_offset()
+            dev = x.device
+            buf = torch.empty(plan.code_bytes, dtype=torch.uint8, device=dev)
+            y = torch.empty((*x.shape[:-1], N), dtype=out_dtype, device=dev)
+            ws, ws_bytes = (None, 0) if plan.ws_bytes == 0 else _workspace(plan.ws_bytes, dev)
+            if bias is not None and bias.stride(-1) != 1:
+                bias = bias.contiguous()
+            _lib.call("ntlb_linear_forward", plan.ref, x2.data_ptr(), weight.data_ptr(),
+                      None if bias is None else bias.data_ptr(), buf.data_ptr(), y.data_ptr(), ws, ws_bytes, base,
+                      ops._stream())
+            if needs[0] or needs[1] or needs[2]:
+                ctx.plan, ctx.backend, ctx.offset = plan, backend, base
+                ctx.bias_dtype = None if bias is None else bias.dtype
+                ctx.x_shape, ctx.x_dtype, ctx.w_dtype = x.shape, out_dtype, weight.dtype
+                if backend.backward_recipe == "ste":
+                    ctx.save_for_backward(buf)
+                else:
+                    ctx.save_for_backward(x2, weight)
+            return y
         x2 = x.reshape(-1, K)
         if x2.stride(-1) != 1:
             x2 = x2.contiguous()
@@ -259,6 +369,36 @@ class _HipLowBitLinear(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         backend: HipLowBitBackend = ctx.backend
+        plan, needs = ctx.plan, ctx.needs_input_grad
+        if plan is not None:
+            dy2 = _rows_2d(dy, plan.N)
+            if backend.backward_recipe == "ste":
+                (buf,) = ctx.saved_tensors
+                if dy2.dtype == torch.bfloat16 and ctx.x_dtype == torch.bfloat16 and ctx.w_dtype == torch.bfloat16:
+                    return (*_ste_backward(plan, dy2, buf, needs, ctx.x_shape, ctx.bias_dtype), None)
+                # another gradient dtype: the dequantized operands on the fp32 GEMM
+                qx, qw = plan.qtensors(buf)
+                dx = dw = None
+                if needs[0]:
+                    wdq = ops.dequant(qw, out_dtype=ctx.w_dtype)
+                    op = _gemm_op_dtype(dy2.dtype, wdq.dtype)
+                    dx = ops.gemm_dense(dy2.to(op), wdq.to(op), b_transposed=True,
+                                        out_dtype=ctx.x_dtype).reshape(ctx.x_shape)
+                if needs[1]:
+                    xdq = ops.dequant(qx, out_dtype=ctx.x_dtype)
+                    op = _gemm_op_dtype(dy2.dtype, xdq.dtype)
+                    dw = ops.gemm_dense_tn(dy2.to(op), xdq.to(op), out_dtype=ctx.w_dtype)
+            else:
+                x2, weight = ctx.saved_tensors
+                if (dy2.dtype == ctx.x_dtype == ctx.w_dtype and dy2.dtype in _RECIPE_DTYPES
+                        and x2.stride(0) == plan.c.ldx and weight.stride(0) == plan.c.ldw):
+                    return (*_recipe_backward(plan, dy2, x2, weight, needs, ctx.x_shape, ctx.bias_dtype, ctx.offset),
+                            None)
+                dx, dw = _fp8_recipe_backward(backend, dy2, x2, weight, ctx.offset, needs)
+                dx = None if dx is None else dx.to(ctx.x_dtype).reshape(ctx.x_shape)
+                dw = None if dw is None else dw.to(ctx.w_dtype)
+            db = ops.colsum(dy2, out_dtype=ctx.bias_dtype) if needs[2] and ctx.bias_dtype is not None else None
+            return dx, dw, db, None
         dy2 = dy.reshape(-1, dy.shape[-1])
         if dy2.stride(-1) != 1:
             dy2 = dy2.contiguous()
@@ -373,12 +513,41 @@ class HipLowBitBackend:
         self.seed = int(seed)
         self._calls = 0
         self._lock = threading.Lock()
+        self._plans: dict = {}
 
     def _next_offset(self) -> int:
         with self._lock:
             c = self._calls
             self._calls += 1
         return c * _OFFSETS_PER_CALL
+
+    def _one_call(self, x, weight, bias, needs) -> bool:
+        """Whether the linear runs as one native call per direction: the recipe's
+        granularities in blockscaled mode, and a backward that reads codes (the
+        straight-through rule of bf16 layers under round to nearest) or
+        quantizes its own operands."""
+        if (self._activation_granularity != "tile_1x128" or self._weight_granularity != "block_128x128"
+                or self.forward_mode != "blockscaled" or weight.dim() != 2 or weight.stride(1) != 1
+                or weight.stride(0) < weight.shape[1] or weight.shape[0] == 0
+                or (bias is not None and bias.device.type != "cuda")):
+            return False
+        if (needs[0] or needs[1]) and self.backward_recipe == "ste":
+            return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
+                    and self._rounding_mode != "stochastic")
+        return True
+
+    def _plan(self, x2, weight, bias) -> _LinearPlan:
+        key = (x2.shape[0], weight.shape, x2.stride(0), weight.stride(0), x2.dtype, weight.dtype,
+               None if bias is None else bias.dtype)
+        plan = self._plans.get(key)
+        if plan is None:
+            plan = _LinearPlan(x2.shape[0], weight.shape[0], weight.shape[1], x2.stride(0), weight.stride(0), x2.dtype,
+                               weight.dtype, key[-1], ops.grid_code(self.code_format), (1 << (self.bits - 1)) - 1,
+                               ops.rounding_code(self._rounding_mode), self.seed)
+            if len(self._plans) >= _MAX_PLANS:  # ragged batches: keep it bounded
+                self._plans.clear()
+            self._plans[key] = plan
+        return plan
 
     def linear(self, input_tensor: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
         if input_tensor.device.type != "cuda" or weight.device.type != "cuda":

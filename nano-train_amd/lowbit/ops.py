@@ -29,8 +29,15 @@ def _dtype_code(dt: torch.dtype) -> int:
         raise TypeError(f"unsupported dtype {dt}; expected float32, bfloat16 or float16") from exc
 
 
+_current_device = torch._C._cuda_getDevice if hasattr(torch._C, "_cuda_getDevice") else torch.cuda.current_device
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The handle of torch's current stream on the current device."""
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_current_device())  # no Stream object per call
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:

@@ -1,0 +1,116 @@
+"""The one-call linear (ntlb_linear_forward and its two backwards) against the
+general path of HipLowBitBackend, which issues the same quantizers and GEMMs
+one by one: outputs and gradients bit for bit, over the dtypes, code formats,
+roundings and backward rules the one-call route accepts, ragged and strided
+operands, a dY whose rows need the padded copy, gradients of a subset of the
+inputs, and NaN and infinite values.  e4m3 runs without NaN row flags there, so
+the NaN cases compare its products with the flagged ones."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from _gpu_util import seeded
+
+pytestmark = pytest.mark.gpu
+
+
+def _backend(fmt, rounding, recipe, K, N):
+    from lowbit.backend import HipLowBitBackend
+    from lowbit.contracts import LowBitKernelSpec
+
+    spec = LowBitKernelSpec("linear", K, N, True, "tile_1x128", "block_128x128", rounding)
+    return HipLowBitBackend(mode="fp8", kernel_spec=spec, code_format=fmt, backward=recipe, seed=77)
+
+
+def _same(a, b):
+    if a is None or b is None:
+        return a is None and b is None
+    a, b = a.detach(), b.detach()
+    if a.shape != b.shape or a.dtype != b.dtype:
+        return False
+    nan = torch.isnan(a)
+    return torch.equal(nan, torch.isnan(b)) and torch.equal(a[~nan], b[~nan])
+
+
+def _both(fmt, rounding, recipe, x, w, b, dy, grads=(True, True, True), general_dy=None):
+    """[y, dx, dw, db] through the one-call route and through the general one"""
+    out = []
+    for general in (False, True):
+        be = _backend(fmt, rounding, recipe, w.shape[1], w.shape[0])
+        calls = []
+        if general:
+            be._one_call = lambda *a: False
+        else:
+            orig = be._one_call
+            be._one_call = lambda *a: calls.append(orig(*a)) or calls[-1]
+        t = [None if v is None else v.detach().requires_grad_(g) for v, g in zip((x, w, b), grads)]
+        y = be.linear(*t)
+        wanted = [v for v in t if v is not None and v.requires_grad]
+        up = general_dy if general and general_dy is not None else dy
+        g = list(torch.autograd.grad(y, wanted, up)) if wanted else []
+        out.append([y] + [g.pop(0) if v is not None and v.requires_grad else None for v in t])
+        if not general:
+            assert calls == [True], "the case should take the one-call route"
+    return out
+
+
+@pytest.mark.parametrize("fmt", ["e4m3", "int_grid"])
+@pytest.mark.parametrize("recipe,rounding", [("ste", "nearest"), ("fp8", "nearest"), ("fp8", "stochastic")])
+@pytest.mark.parametrize("mnk", [(1, 64, 128), (37, 129, 257), (130, 320, 200), (300, 1541, 1000)])
+def test_one_call_equals_the_general_path(gpu_device, mnk, fmt, recipe, rounding):
+    M, N, K = mnk
+    x = seeded((M, K), seed=20262101, outliers=0.01).to(gpu_device)
+    w = seeded((N, K), seed=20262102, std=0.02).to(gpu_device)
+    b = seeded((N,), seed=20262103).to(gpu_device)
+    dy = seeded((M, N), seed=20262104, std=1e-3).to(gpu_device)
+    one, gen = _both(fmt, rounding, recipe, x, w, b, dy)
+    assert all(_same(p, q) for p, q in zip(one, gen))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_other_dtypes(gpu_device, dtype):
+    """forward without gradients for every rounding, and the fp32 recipe backward"""
+    x = seeded((2, 35, 300), seed=20262111, dtype=dtype).to(gpu_device)
+    w = seeded((200, 300), seed=20262112, std=0.02, dtype=dtype).to(gpu_device)
+    b = seeded((200,), seed=20262113, dtype=dtype).to(gpu_device)
+    for rounding in ("nearest", "stochastic"):
+        one, gen = _both("e4m3", rounding, "ste", x, w, b, None, grads=(False, False, False))
+        assert _same(one[0], gen[0])
+    dy = seeded((2, 35, 200), seed=20262114, std=1e-3, dtype=dtype).to(gpu_device)
+    one, gen = _both("int_grid", "nearest", "fp8", x, w, b, dy)
+    assert all(_same(p, q) for p, q in zip(one, gen))
+
+
+@pytest.mark.parametrize("recipe", ["ste", "fp8"])
+@pytest.mark.parametrize("grads", [(True, False, False), (False, True, False), (False, False, True)])
+def test_gradient_subsets_and_strides(gpu_device, recipe, grads):
+    """3-D input, a column-sliced x and weight (row pitch above K), a dY that is
+    a slice at an odd column, and one whose rows are one expanded row"""
+    M, N, K = 66, 192, 256
+    x = seeded((M, K + 24), seed=20262121).to(gpu_device)[:, :K].reshape(2, M // 2, K)
+    w = seeded((N, K + 8), seed=20262122, std=0.02).to(gpu_device)[:, :K]
+    b = seeded((N,), seed=20262123).to(gpu_device)
+    big = seeded((2, M // 2, N + 3), seed=20262124, std=1e-3).to(gpu_device)
+    for dy in (big[..., :N], big[..., 3:], big[:1, :1, :N].expand(2, M // 2, N)):
+        one, gen = _both("e4m3", "nearest", recipe, x, w, b, dy, grads, general_dy=dy.contiguous())
+        assert all(_same(p, q) for p, q in zip(one, gen))
+
+
+@pytest.mark.parametrize("fmt", ["e4m3", "int_grid"])
+@pytest.mark.parametrize("recipe", ["ste", "fp8"])
+@pytest.mark.parametrize("mnk", [(20, 72, 200), (300, 700, 1500), (1100, 2100, 700)])
+def test_nan_and_inf_operands(gpu_device, mnk, fmt, recipe):
+    """NaN and infinities in x, the weight and dY: NaN exactly where the flagged
+    products of the general path have it, every other value the same"""
+    M, N, K = mnk
+    x = seeded((M, K), seed=20262131).to(gpu_device)
+    w = seeded((N, K), seed=20262132, std=0.02).to(gpu_device)
+    dy = seeded((M, N), seed=20262133, std=1e-3).to(gpu_device)
+    x[3, 17], x[5, K - 1], x[M - 1, 4] = float("nan"), float("inf"), float("-inf")
+    w[7, 100], w[N - 1, 5] = float("nan"), float("inf")
+    dy[9, 11], dy[2, N - 1] = float("nan"), float("inf")
+    one, gen = _both(fmt, "nearest", recipe, x, w, None, dy)
+    assert torch.isnan(one[0][3]).all() and torch.isnan(one[0][:, 7]).all() and not torch.isnan(one[0][0, 0])
+    assert all(_same(p, q) for p, q in zip(one, gen))
