@@ -511,6 +511,15 @@ int ntlb_gemm_grouped_swiglu_quant_gu(int grid, const uint8_t* a, int64_t lda, c
                                       uint64_t offset, uint16_t* gu, int64_t ldgu, void* stream);
 
 /*
+ * ntlb_gemm_dense_tn over bf16 operands, Y[M,N] = A^T . B (A stored [K, M], B
+ * [K, N]), with the output tile chosen by shape: products that leave most of
+ * the chip idle on 256x256 tiles take tiles down to 16x16, where the fp32 sums
+ * over K are formed in ranges.
+ */
+int ntlb_gemm_bf16_tn(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                      void* y, int y_dtype, int64_t ldy, void* stream);
+
+/*
  * One low-bit Linear per call (te_backend.py:229-260 with 1x128 activation
  * tiles and 128x128 weight blocks): Y = X_dq . W_dq^T + bias over the codes'
  * fp32 q * s values, its straight-through backward, and the backward with

@@ -96,7 +96,7 @@ def build(verbose: bool = False) -> str:
     with open(RESOURCES, "w") as fh:
         json.dump(resources, fh, indent=0, sort_keys=True)
     tmp = LIB + ".tmp"
-    cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]
+    cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-Wl,--no-undefined", "-o", tmp, *objs]
     subprocess.run(cmd, check=True)
     os.replace(tmp, LIB)
     if verbose:

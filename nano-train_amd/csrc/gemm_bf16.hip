@@ -1,0 +1,433 @@
+// bf16 GEMM on tiles below 256x256, fp32 accumulation: the products of
+// gemm_dq.hip over plain bf16 matrices whose 256x256 tiles would leave most of
+// the chip idle (the gradients of small layers, the dense GEMMs).
+//
+// 16*MB x 16*NB tiles, a workgroup's WK waves dividing the contraction, each
+// wave with its own multi-stage LDS copies and no barrier in the K loop, as
+// gemm_small.hip (whose comment gives the reasons); and 128x128 tiles, staged
+// once per workgroup of four waves, as its gemm_mid_kernel.  A K step is 64
+// values (128 bytes).  Operands stored transposed are copied as stored and read
+// with ds_read_b64_tr_b16 (lane layout: gemm_dq.hip).
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "ntlb_device.h"
+#include "ntlb_gemm_bf16.h"
+#include "ntlb_host.h"
+#include "ntlb_splitk.h"
+
+namespace ntlb {
+namespace bfs {
+
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+typedef __attribute__((address_space(3))) v4s* lds_v4s_ptr;
+
+constexpr int ROWB = 128;   // bytes of a row's K step
+constexpr int KSTEP = 64;
+
+constexpr int vmcnt_imm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
+
+// Row-major stage [16*B rows][128 bytes]: 16-byte chunk c of row r at slot
+// c ^ perm(r), conflict-free for the 16-row fragment reads
+__device__ __forceinline__ int row_perm(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+
+// Transposed stage [64 contraction rows][16*B operand rows]: 2*B chunks per
+// contraction row.  A 16-lane group of ds_read_b64_tr_b16 reads 32 bytes of
+// each of four consecutive contraction rows, the next group those 16 further:
+// the XOR spreads these eight 32-byte pieces over the 256 bytes of banks (for
+// rows of 32 bytes the two groups share them).
+template <int B>
+__device__ __forceinline__ int tr_perm(int k) {
+  if constexpr (B >= 8) return (2 * (k & 3)) ^ (8 * ((k >> 4) & 1));  // 256-byte rows
+  if constexpr (B == 4) return 2 * (((k >> 1) & 1) | (((k >> 4) & 1) << 1));
+  if constexpr (B == 2) return 2 * ((k >> 4) & 1);
+  return 0;
+}
+
+// MFMA fragments of one K step: row = lane%16 of 16 operand rows, contraction
+// 16g .. 16g+15 with g = lane/16
+template <bool TR, int B>
+__device__ __forceinline__ v8i frag(const uint8_t* tile, int row0, int lane) {
+  const int g = lane >> 4;
+  v8i f;
+  if constexpr (!TR) {
+    const int r = row0 + (lane & 15);
+    const uint4 lo = *reinterpret_cast<const uint4*>(tile + r * ROWB + (((2 * g) ^ row_perm(r)) << 4));
+    const uint4 hi = *reinterpret_cast<const uint4*>(tile + r * ROWB + (((2 * g + 1) ^ row_perm(r)) << 4));
+    f[0] = (int)lo.x; f[1] = (int)lo.y; f[2] = (int)lo.z; f[3] = (int)lo.w;
+    f[4] = (int)hi.x; f[5] = (int)hi.y; f[6] = (int)hi.z; f[7] = (int)hi.w;
+  } else {
+    const int j = (lane >> 2) & 3, q = lane & 3;
+    const int c = (row0 >> 3) + (q >> 1);
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      const int k = 16 * g + 4 * h + j;
+      const v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_v4s_ptr)(tile + k * (32 * B) + ((c ^ tr_perm<B>(k)) << 4) + (q & 1) * 8));
+      f[2 * h] = (int)(((uint32_t)(uint16_t)v[1] << 16) | (uint16_t)v[0]);
+      f[2 * h + 1] = (int)(((uint32_t)(uint16_t)v[3] << 16) | (uint16_t)v[2]);
+    }
+  }
+  return f;
+}
+
+__device__ __forceinline__ v4f mma(const v8i& p, const v8i& q, v4f acc) {
+  const v4i pl = {p[0], p[1], p[2], p[3]}, ph = {p[4], p[5], p[6], p[7]};
+  const v4i ql = {q[0], q[1], q[2], q[3]}, qh = {q[4], q[5], q[6], q[7]};
+  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, pl), __builtin_bit_cast(v8bf, ql), acc, 0, 0,
+                                                0);
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, ph), __builtin_bit_cast(v8bf, qh), acc, 0,
+                                                 0, 0);
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t operand_rsrc(const Bf16Operand& o) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)o.p, (short)0, (int)((o.tr ? o.kvalid : o.rows) * o.ld * 2),
+                                           0x00020000);
+}
+
+// The copies of one operand's K step (16*B operand rows, 2*B KiB-copies of 64
+// lanes) by NW waves, wave w taking copies w, w + NW, ...  The LDS side is
+// linear in (copy, lane); the lane's global offset carries the swizzle.  Copies
+// of one parity differ by a constant, so two lane offsets serve all.
+template <bool TR, int B, int NW>
+struct Copies {
+  static constexpr int COUNT = 2 * B / NW;
+  static_assert(2 * B % NW == 0, "whole copies per wave");
+  __amdgpu_buffer_rsrc_t rs;
+  uint32_t off[COUNT];
+  uint32_t kstep;  // bytes per K step
+  int wave;
+  __device__ __forceinline__ void init(const Bf16Operand& o, int64_t r0, int w, int lane) {
+    rs = operand_rsrc(o);
+    wave = w;
+    kstep = TR ? (uint32_t)(KSTEP * o.ld * 2) : (uint32_t)ROWB;
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i) {
+      const int slot = (w + NW * i) * 64 + lane;
+      if constexpr (TR) {
+        const int k = slot / (2 * B), c = (slot % (2 * B)) ^ tr_perm<B>(k);
+        off[i] = (uint32_t)(k * o.ld * 2 + (r0 + 8 * c) * 2);
+      } else {
+        const int r = slot >> 3, c = (slot & 7) ^ row_perm(r);
+        off[i] = (uint32_t)((r0 + r) * o.ld * 2 + c * 16);
+      }
+    }
+  }
+  __device__ __forceinline__ void issue(uint8_t* stage, int ks) const {
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(stage + (wave + NW * i) * 1024), 16, off[i],
+                                               (uint32_t)ks * kstep, 0, 0);
+  }
+};
+
+__device__ __forceinline__ void store4(const Bf16Args& g, int64_t m, int64_t n, v4f v) {
+  if (g.bias) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] += load_elem(g.bias, g.bias_dtype, min<int64_t>(n + q, g.N - 1));
+  }
+  if (g.vec_out && n + 4 <= g.N && g.y_dtype == DT_BF16) {
+    const v2bf p0 = {(__bf16)v[0], (__bf16)v[1]}, p1 = {(__bf16)v[2], (__bf16)v[3]};
+    *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(g.y) + m * g.ldy + n) =
+        make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (n + q < g.N) store_elem(g.y, g.y_dtype, m * g.ldy + n + q, v[q]);
+}
+
+template <bool TA, bool TB, int MB, int NB, int WK, int NS>
+__global__ void __launch_bounds__(64 * WK) gemm_bf16_small_kernel(Bf16Args g) {
+  constexpr int WB = (MB + NB) * 16 * ROWB;
+  static_assert(MB * NB * 1024 <= WB, "the partial tiles fit the first stage");
+  __shared__ __attribute__((aligned(16))) uint8_t st0[WK * WB];
+  __shared__ __attribute__((aligned(16))) uint8_t st1[WK * WB];
+  __shared__ __attribute__((aligned(16))) uint8_t st2[NS > 2 ? WK * WB : 16];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t n0 = (int64_t)blockIdx.x * (16 * NB), m0 = (int64_t)blockIdx.y * (16 * MB);
+  const int nk = (int)(g.Kc / KSTEP);
+  const int k0 = (int)((int64_t)wave * nk / WK), k1 = (int)((int64_t)(wave + 1) * nk / WK);
+  v4f acc[MB][NB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = (v4f){0.f, 0.f, 0.f, 0.f};
+  if (k0 < k1) {
+    Copies<TA, MB, 1> ca;
+    Copies<TB, NB, 1> cb;
+    ca.init(g.a, m0, 0, lane);
+    cb.init(g.b, n0, 0, lane);
+    uint8_t* const s0 = st0 + wave * WB;
+    uint8_t* const s1 = st1 + wave * WB;
+    uint8_t* const s2 = st2 + (NS > 2 ? wave * WB : 0);
+    auto stage = [&](int i) { return i == 0 ? s0 : i == 1 ? s1 : s2; };
+    auto issue = [&](int i, int ks) {
+      ca.issue(stage(i), ks);
+      cb.issue(stage(i) + MB * 16 * ROWB, ks);
+    };
+    auto each = [](auto f) {
+      f(std::integral_constant<int, 0>());
+      f(std::integral_constant<int, 1>());
+      if constexpr (NS > 2) f(std::integral_constant<int, 2>());
+    };
+    auto step = [&](auto ic, int ks) {
+      constexpr int I = decltype(ic)::value;
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // the reads of the stage refilled now are done
+      asm volatile("" ::: "memory");
+      issue((I + NS - 1) % NS, min(ks + NS - 1, k1 - 1));
+      // in-order returns: with only the younger stages' copies outstanding,
+      // this stage has landed
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 1) * 2 * (MB + NB)));
+      asm volatile("" ::: "memory");
+      const uint8_t* ta = stage(I);
+      const uint8_t* tb = ta + MB * 16 * ROWB;
+      v8i bf[NB];
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) bf[nb] = frag<TB, NB>(tb, nb * 16, lane);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        const v8i af = frag<TA, MB>(ta, mb * 16, lane);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = mma(bf[nb], af, acc[mb][nb]);
+      }
+    };
+    each([&](auto ic) {
+      if constexpr (decltype(ic)::value < NS - 1) issue(decltype(ic)::value, min(k0 + decltype(ic)::value, k1 - 1));
+    });
+    int ks = k0;
+    for (; ks + NS <= k1; ks += NS) each([&](auto ic) { step(ic, ks + decltype(ic)::value); });
+    each([&](auto ic) {
+      if (ks + decltype(ic)::value < k1) step(ic, ks + decltype(ic)::value);
+    });
+    __builtin_amdgcn_s_waitcnt(0);  // nothing of this wave is in flight into LDS past here
+    asm volatile("" ::: "memory");
+  }
+  __syncthreads();
+  v4f* red = reinterpret_cast<v4f*>(st0);
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) red[(wave * MB * NB + mb * NB + nb) * 64 + lane] = acc[mb][nb];
+  __syncthreads();
+  // lane l of block (mb, nb): row m0 + 16*mb + l%16, columns n0 + 16*nb + 4*(l/16) + 0..3
+  for (int q = threadIdx.x; q < MB * NB * 64; q += 64 * WK) {
+    const int b = q >> 6, l = q & 63;
+    v4f v = red[q];
+#pragma unroll
+    for (int w = 1; w < WK; ++w) v += red[w * MB * NB * 64 + q];
+    const int64_t m = m0 + (b / NB) * 16 + (l & 15);
+    const int64_t n = n0 + (b % NB) * 16 + (l >> 4) * 4;
+    if (m < g.M && n < g.N) store4(g, m, n, v);
+  }
+}
+
+constexpr int MID = 128;
+
+template <bool TA, bool TB, int ODT>
+__global__ void __launch_bounds__(256, 2) gemm_bf16_mid_kernel(Bf16Args g) {
+  constexpr int ST = MID * ROWB;  // 16 KiB per operand stage
+  __shared__ __attribute__((aligned(16))) uint8_t la0[ST];
+  __shared__ __attribute__((aligned(16))) uint8_t lb0[ST];
+  __shared__ __attribute__((aligned(16))) uint8_t la1[ST];
+  __shared__ __attribute__((aligned(16))) uint8_t lb1[ST];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  // each XCD walks a contiguous range of a raster of four row tiles
+  const int num_n = (int)((g.N + MID - 1) / MID), num_m = (int)((g.M + MID - 1) / MID);
+  int64_t m0, n0;
+  {
+    const int nwg = (int)gridDim.x, xcd = (int)blockIdx.x & 7, local = (int)blockIdx.x >> 3;
+    const int per = nwg >> 3, extra = nwg & 7;
+    const int pid = xcd * per + min(xcd, extra) + local;
+    constexpr int GROUP_M = 4;
+    const int group = pid / (GROUP_M * num_n);
+    const int gsize = min(num_m - group * GROUP_M, GROUP_M);
+    const int in_group = pid - group * GROUP_M * num_n;
+    m0 = (int64_t)(group * GROUP_M + in_group % gsize) * MID;
+    n0 = (int64_t)(in_group / gsize) * MID;
+  }
+  Copies<TA, 8, 4> ca;
+  Copies<TB, 8, 4> cb;
+  ca.init(g.a, m0, wave, lane);
+  cb.init(g.b, n0, wave, lane);
+  const int nk = (int)(g.Kc / KSTEP);
+  v4f acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
+  ca.issue(la0, 0);
+  cb.issue(lb0, 0);
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  auto step = [&](auto bufc, int ks) {
+    constexpr int BUF = decltype(bufc)::value;
+    const uint8_t* ta = BUF ? la1 : la0;
+    const uint8_t* tb = BUF ? lb1 : lb0;
+    const int kn = min(ks + 1, nk - 1);  // the last step copies itself into the idle stage
+    ca.issue(BUF ? la0 : la1, kn);
+    cb.issue(BUF ? lb0 : lb1, kn);
+    v8i bf[4];
+#pragma unroll
+    for (int tn = 0; tn < 4; ++tn) bf[tn] = frag<TB, 8>(tb, wn * 64 + tn * 16, lane);
+#pragma unroll
+    for (int tm = 0; tm < 4; ++tm) {
+      const v8i af = frag<TA, 8>(ta, wm * 64 + tm * 16, lane);
+#pragma unroll
+      for (int tn = 0; tn < 4; ++tn) acc[tm][tn] = mma(bf[tn], af, acc[tm][tn]);
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+  };
+  for (int ks = 0; ks < nk; ks += 2) {
+    step(std::integral_constant<int, 0>(), ks);
+    if (ks + 1 < nk) step(std::integral_constant<int, 1>(), ks + 1);
+  }
+  // each wave stages 32 of its 64 rows at a time and stores whole row segments
+  uint8_t* stage_w = wave == 0 ? la0 : wave == 1 ? lb0 : wave == 2 ? la1 : lb1;
+  constexpr int esz = ODT == DT_F32 ? 4 : 2, pitch = 64 * esz + 16, cpr = 64 * esz / 16, epc = 16 / esz;
+  static_assert(32 * pitch <= ST, "staged rows fit a stage");
+#pragma unroll
+  for (int part = 0; part < 2; ++part) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int tn = 0; tn < 4; ++tn) {
+        v4f v = acc[part * 2 + t][tn];
+        if (g.bias) {
+          const int64_t n = n0 + wn * 64 + tn * 16 + (lane >> 4) * 4;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) v[q] += load_elem(g.bias, g.bias_dtype, min<int64_t>(n + q, g.N - 1));
+        }
+        uint8_t* dst = stage_w + (t * 16 + (lane & 15)) * pitch + (tn * 16 + (lane >> 4) * 4) * esz;
+        if constexpr (ODT == DT_F32) {
+          *reinterpret_cast<v4f*>(dst) = v;
+        } else if constexpr (ODT == DT_BF16) {
+          const v2bf p0 = {(__bf16)v[0], (__bf16)v[1]}, p1 = {(__bf16)v[2], (__bf16)v[3]};
+          *reinterpret_cast<uint2*>(dst) =
+              make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
+        } else {
+          const __half h[4] = {f32_to_f16(v[0]), f32_to_f16(v[1]), f32_to_f16(v[2]), f32_to_f16(v[3])};
+          *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(h);
+        }
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < cpr / 2; ++j) {
+      const int q = lane + 64 * j, row = q / cpr, c = q % cpr;
+      const int64_t m = m0 + wm * 64 + part * 32 + row, n = n0 + wn * 64 + c * epc;
+      const uint8_t* src = stage_w + row * pitch + c * 16;
+      if (m >= g.M || n >= g.N) continue;
+      uint8_t* ydst = reinterpret_cast<uint8_t*>(g.y) + (m * g.ldy + n) * esz;
+      if (g.vec_out && n + epc <= g.N) {
+        store16_nt(ydst, src);
+      } else {
+        using E = std::conditional_t<esz == 4, uint32_t, uint16_t>;
+#pragma nounroll
+        for (int e = 0; e < epc && n + e < g.N; ++e)
+          reinterpret_cast<E*>(ydst)[e] = reinterpret_cast<const E*>(src)[e];
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// every instance explicitly: the host stubs of implicitly instantiated ones
+// are not all emitted here (ROCm 7.2 hipcc)
+#define NTLB_BF16_CASES(X) X(1, 1, 8, 2) X(1, 2, 4, 3) X(2, 2, 4, 3) X(2, 4, 4, 3) X(4, 4, 4, 2) X(4, 4, 2, 2)
+#define NTLB_BF16_INST(MB, NB, WK, NS)                                                            \
+  template __global__ void gemm_bf16_small_kernel<true, true, MB, NB, WK, NS>(Bf16Args);          \
+  template __global__ void gemm_bf16_small_kernel<false, true, MB, NB, WK, NS>(Bf16Args);         \
+  template __global__ void gemm_bf16_small_kernel<false, false, MB, NB, WK, NS>(Bf16Args);
+#define NTLB_BF16_MID_INST(ODT)                                        \
+  template __global__ void gemm_bf16_mid_kernel<true, true, ODT>(Bf16Args);   \
+  template __global__ void gemm_bf16_mid_kernel<false, true, ODT>(Bf16Args);  \
+  template __global__ void gemm_bf16_mid_kernel<false, false, ODT>(Bf16Args);
+NTLB_BF16_CASES(NTLB_BF16_INST)
+NTLB_BF16_MID_INST(DT_F32)
+NTLB_BF16_MID_INST(DT_BF16)
+NTLB_BF16_MID_INST(DT_F16)
+#undef NTLB_BF16_INST
+#undef NTLB_BF16_MID_INST
+
+struct Plan {
+  int mb, nb, wk, ns;
+};
+
+// The tile of a product (mb = 8: 128x128; mb = 0: the 256x256 tiles of
+// gemm_dq.hip): the smallest one whose workgroups all run at once, as the
+// blockwise products choose it.  Measured (both operands transposed, bf16 out,
+// in a graph, us; this kernel / 256x256 tiles): 1000 x K 1003: 4.9 / 25 at 64
+// rows, 7.8 / 25 at 512, 9.9 / 26 at 1003, 13.7 / 26 at 1541, 19 / 27 at 4096;
+// 2048 x K 2048: 7.7 / 44 at 128 rows, 12.4 / 44 at 512, 21 / 46 at 1003, 33 / 45
+// at 2048, 36 / 46 at 4096.  Between 128x128 and 256x256 tiles the estimates
+// decide: 1.05 us a K step for 128x128 tiles, 1.4 for 256x256 ones, whose
+// split-K tail (big_split: the caller has its workspace) adds about 30 us.
+static Plan plan(int64_t M, int64_t N, int nk, bool big_split) {
+  const int64_t cus = split_device_cus();
+  auto wgs = [&](int64_t rows, int64_t cols) { return cdiv(M, rows) * cdiv(N, cols); };
+  if (wgs(16, 16) <= cus) return {1, 1, 8, 2};
+  if (wgs(16, 32) <= cus || M <= 16) return {1, 2, 4, 3};
+  if (wgs(32, 32) <= cus) return {2, 2, 4, 3};
+  if (wgs(32, 64) <= cus) return {2, 4, 4, 3};
+  if (wgs(64, 64) <= cus) return {4, 4, 4, 2};
+  if (wgs(64, 64) <= 2 * cus) return {4, 4, 2, 2};
+  if (wgs(MID, MID) <= 2 * cus) {
+    const int split = big_split ? split_plan(wgs(256, 256), nk, DQ_SPLIT_MIN_STEPS).s : 1;
+    if (1.05 * nk + 3 < 1.4 * nk / split + (split > 1 ? 30 : 6)) return {8, 8, 4, 2};
+  }
+  return {0, 0, 0, 0};
+}
+
+template <bool TA, bool TB>
+static void launch(const Plan& p, const Bf16Args& g, hipStream_t st) {
+  if (p.mb == 8) {
+    const dim3 grd((unsigned)(cdiv(g.M, MID) * cdiv(g.N, MID))), blk(256);
+    if (g.y_dtype == DT_F32)
+      gemm_bf16_mid_kernel<TA, TB, DT_F32><<<grd, blk, 0, st>>>(g);
+    else if (g.y_dtype == DT_F16)
+      gemm_bf16_mid_kernel<TA, TB, DT_F16><<<grd, blk, 0, st>>>(g);
+    else
+      gemm_bf16_mid_kernel<TA, TB, DT_BF16><<<grd, blk, 0, st>>>(g);
+    return;
+  }
+  const dim3 grd((unsigned)cdiv(g.N, 16 * p.nb), (unsigned)cdiv(g.M, 16 * p.mb)), blk(64 * p.wk);
+#define NTLB_BF16_CASE(MB, NB, WK, NS)                                                  \
+  if (p.mb == MB && p.nb == NB && p.wk == WK && p.ns == NS) {                           \
+    gemm_bf16_small_kernel<TA, TB, MB, NB, WK, NS><<<grd, blk, 0, st>>>(g);             \
+    return;                                                                             \
+  }
+  NTLB_BF16_CASES(NTLB_BF16_CASE)
+#undef NTLB_BF16_CASE
+}
+
+}  // namespace bfs
+
+bool bf16_small_fits(int64_t M, int64_t N, int64_t Kc, bool big_split) {
+  return bfs::plan(M, N, (int)(Kc / bfs::KSTEP), big_split).mb != 0;
+}
+
+void bf16_small_launch(const Bf16Args& g, hipStream_t st) {
+  const int nk = (int)(g.Kc / bfs::KSTEP);
+  bfs::Plan p = bfs::plan(g.M, g.N, nk, false);
+  if (g.a.tr)
+    bfs::launch<true, true>(p, g, st);
+  else if (g.b.tr)
+    bfs::launch<false, true>(p, g, st);
+  else
+    bfs::launch<false, false>(p, g, st);
+}
+
+}  // namespace ntlb

@@ -59,6 +59,7 @@
 #include <type_traits>
 
 #include "ntlb_device.h"
+#include "ntlb_gemm_bf16.h"
 #include "ntlb_host.h"
 #include "ntlb_splitk.h"
 
@@ -1141,12 +1142,70 @@ __global__ void __launch_bounds__(256) colsum_partial_kernel(const void* x, int6
   }
 }
 
+// The same sums where the chunks above would be fewer than the compute units:
+// 64 rows by 128 columns per workgroup, a wave's 16 rows all loaded before
+// they are added (dY 1003 x 1541: 16 workgroups and 38 us became 208 and 5).
+constexpr int CS_ROWS_S = 64, CS_COLS_S = 128;
+
+template <int IN_DT>
+__global__ void __launch_bounds__(256) colsum_partial_small_kernel(const void* x, int64_t M, int64_t N, int64_t ld,
+                                                                   float* part) {
+  __shared__ float red[4][CS_COLS_S];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t n = (int64_t)blockIdx.x * CS_COLS_S + lane * 2, chunk = blockIdx.y;
+  constexpr int esz = IN_DT == DT_F32 ? 4 : 2;
+  const bool vec = n + 2 <= N && ((uintptr_t)x % (2 * esz) == 0) && (ld % 2 == 0);
+  float v[16][2];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int64_t r = chunk * CS_ROWS_S + wave + 4 * i;
+    v[i][0] = v[i][1] = 0.f;
+    if (r >= M) continue;
+    if (vec) {
+      if constexpr (IN_DT == DT_F32) {
+        const float2 t = *reinterpret_cast<const float2*>(reinterpret_cast<const float*>(x) + r * ld + n);
+        v[i][0] = t.x;
+        v[i][1] = t.y;
+      } else {
+        const uint32_t t = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint16_t*>(x) + r * ld + n);
+        v[i][0] = IN_DT == DT_BF16 ? __uint_as_float(t << 16) : __half2float(__ushort_as_half((unsigned short)t));
+        v[i][1] = IN_DT == DT_BF16 ? __uint_as_float(t & 0xFFFF0000u)
+                                   : __half2float(__ushort_as_half((unsigned short)(t >> 16)));
+      }
+    } else {
+      if (n < N) v[i][0] = load_elem(x, IN_DT, r * ld + n);
+      if (n + 1 < N) v[i][1] = load_elem(x, IN_DT, r * ld + n + 1);
+    }
+  }
+  float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    s0 += v[i][0];
+    s1 += v[i][1];
+  }
+  red[wave][lane * 2] = s0;
+  red[wave][lane * 2 + 1] = s1;
+  __syncthreads();
+  if (tid < CS_COLS_S) {
+    const int64_t nn = (int64_t)blockIdx.x * CS_COLS_S + tid;
+    if (nn < N) part[chunk * N + nn] = ((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid];
+  }
+}
+
 __global__ void __launch_bounds__(256) colsum_finish_kernel(const float* part, int64_t chunks, int64_t N, void* out,
                                                             int out_dtype) {
   const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (n >= N) return;
   float s = 0.f;
-  for (int64_t c = 0; c < chunks; ++c) s += part[c * N + n];
+  int64_t c = 0;
+  for (; c + 8 <= chunks; c += 8) {  // eight loads in flight, added in chunk order
+    float p[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) p[i] = part[(c + i) * N + n];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s += p[i];
+  }
+  for (; c < chunks; ++c) s += part[c * N + n];
   store_elem(out, out_dtype, n, s);
 }
 
@@ -1276,10 +1335,8 @@ int check_codes(const char* fn, const char* what, const uint8_t* codes, int64_t 
   return NTLB_OK;
 }
 
-// the split-K tail's minimum K steps per range, as for the blockwise GEMM
-// (a K step here is 128 bytes per row, the MFMA work of one of its blocks)
-constexpr int DQ_SPLIT_MIN_STEPS = 9;
-
+// (a K step here is 128 bytes per row, the MFMA work of one block of the
+// blockwise GEMM, whose minimum per range DQ_SPLIT_MIN_STEPS repeats)
 SplitPlan dq_plan(int64_t M, int64_t N, int64_t Kc, int el) {
   const int64_t tiles = ((M + TM - 1) / TM) * ((N + TN - 1) / TN);
   return split_plan(tiles, (int)(Kc / (el == EL_BF16 ? 64 : 32)), DQ_SPLIT_MIN_STEPS);
@@ -1828,9 +1885,12 @@ extern "C" int ntlb_gemm_dense_tn(int op_dtype, const void* a, int64_t lda, cons
   return finish(fn, g, el, SRC_TDIRECT, SRC_TDIRECT, y_dtype, ldy, stream);
 }
 
+// whether the 256-row x 512-column chunks would leave compute units idle
+static bool colsum_small(int64_t M, int64_t N) { return cdiv(M, CS_ROWS) * cdiv(N, CS_COLS) < split_device_cus(); }
+
 extern "C" int64_t ntlb_colsum_workspace_bytes(int64_t M, int64_t N) {
   if (M <= 0 || N <= 0) return 0;
-  return (M + CS_ROWS - 1) / CS_ROWS * N * 4;
+  return cdiv(M, colsum_small(M, N) ? CS_ROWS_S : CS_ROWS) * N * 4;
 }
 
 extern "C" int ntlb_colsum(const void* x, int x_dtype, int64_t M, int64_t N, int64_t ldx, float* workspace,
@@ -1841,20 +1901,46 @@ extern "C" int ntlb_colsum(const void* x, int x_dtype, int64_t M, int64_t N, int
   if (N == 0) return NTLB_OK;
   if (!out) return fail(NTLB_EINVAL, "%s: NULL output", fn);
   hipStream_t st = as_stream(stream);
-  const int64_t chunks = (M + CS_ROWS - 1) / CS_ROWS;
+  const bool small = colsum_small(M, N);
+  const int64_t chunks = cdiv(M, small ? CS_ROWS_S : CS_ROWS);
   if (M > 0) {
     if (!x || !workspace) return fail(NTLB_EINVAL, "%s: NULL input or workspace", fn);
     if (ws_bytes < ntlb_colsum_workspace_bytes(M, N)) return fail(NTLB_EINVAL, "%s: workspace too small", fn);
-    const int64_t gx = (N + CS_COLS - 1) / CS_COLS;
+    const int64_t gx = cdiv(N, small ? CS_COLS_S : CS_COLS);
     if (gx > 0x7FFFFFFF || chunks > 65535) return fail(NTLB_EUNSUPPORTED, "%s: too large", fn);
-    dim3 grd((unsigned)gx, (unsigned)chunks);
+    const dim3 grd((unsigned)gx, (unsigned)chunks);
+    auto go = [&](auto dtc) {
+      constexpr int DT = decltype(dtc)::value;
+      if (small)
+        colsum_partial_small_kernel<DT><<<grd, 256, 0, st>>>(x, M, N, ldx, workspace);
+      else
+        colsum_partial_kernel<DT><<<grd, 256, 0, st>>>(x, M, N, ldx, workspace);
+    };
     if (x_dtype == NTLB_BF16)
-      colsum_partial_kernel<DT_BF16><<<grd, 256, 0, st>>>(x, M, N, ldx, workspace);
+      go(std::integral_constant<int, DT_BF16>());
     else if (x_dtype == NTLB_F32)
-      colsum_partial_kernel<DT_F32><<<grd, 256, 0, st>>>(x, M, N, ldx, workspace);
+      go(std::integral_constant<int, DT_F32>());
     else
-      colsum_partial_kernel<DT_F16><<<grd, 256, 0, st>>>(x, M, N, ldx, workspace);
+      go(std::integral_constant<int, DT_F16>());
   }
   colsum_finish_kernel<<<(unsigned)((N + 255) / 256), 256, 0, st>>>(workspace, chunks, N, out, out_dtype);
+  return check_launch(fn);
+}
+
+extern "C" int ntlb_gemm_bf16_tn(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N,
+                                 int64_t K, void* y, int y_dtype, int64_t ldy, void* stream) {
+  const char* fn = "ntlb_gemm_bf16_tn";
+  const int64_t kc = (K + 63) / 64 * 64;
+  if (M < 1 || N < 1 || K < 1 || !a || !b || !y || lda < M || ldb < N || !aligned(a, 16) || !aligned(b, 16) ||
+      lda % 8 || ldb % 8 || (K + 64) * lda * 2 >= (int64_t)0x7FFFFFFF || (K + 64) * ldb * 2 >= (int64_t)0x7FFFFFFF ||
+      !valid_dtype(y_dtype) || ldy < N || !bf16_small_fits(M, N, kc, false))
+    return ntlb_gemm_dense_tn(NTLB_BF16, a, lda, b, ldb, M, N, K, y, y_dtype, ldy, stream);  // or its error
+  Bf16Args g{};
+  g.a = Bf16Operand{a, lda, M, K, true};
+  g.b = Bf16Operand{b, ldb, N, K, true};
+  g.M = M; g.N = N; g.Kc = kc;
+  g.y = y; g.y_dtype = y_dtype; g.ldy = ldy;
+  g.vec_out = aligned(y, 16) && ((ldy * dtype_size(y_dtype)) % 16 == 0);
+  bf16_small_launch(g, as_stream(stream));
   return check_launch(fn);
 }

@@ -16,6 +16,7 @@
 #include <algorithm>
 
 #include "ntlb_device.h"
+#include "ntlb_gemm_bf16.h"
 #include "ntlb_host.h"
 
 namespace ntlb {
@@ -42,6 +43,56 @@ __global__ void __launch_bounds__(256) pad_rows16_kernel(const uint16_t* src, in
     w[i] = lo | (hi << 16);
   }
   *reinterpret_cast<uint4*>(dst + m * ldd + c) = make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// The bf16 operands of small straight-through gradients, bf16(q * s) from the
+// forward's codes: weight rows (one scale per 128x128 block) into wd, then
+// activation rows (one per row and block) into xd, both with row pitch ld = K
+// rounded up to 8; either can be absent (0 rows).  A workgroup of the gradient
+// GEMMs' 256x256 tiles decodes inside the GEMM; on 16x16 to 128x128 tiles each
+// code would be decoded again by every tile that reads it, and this one pass
+// over a few MB costs less (N 1541, K 1000, 1003 rows: about 3 us).
+struct DecodeArgs {
+  const uint8_t* wc;
+  const float* ws;
+  const uint8_t* xc;
+  const float* xs;
+  int64_t wrows, xrows, kp, T, m4, ld;
+  uint16_t *wd, *xd;
+};
+
+template <int GRID>
+__global__ void __launch_bounds__(256) decode_operands_kernel(DecodeArgs a) {
+#pragma clang fp contract(off)
+  typedef float v2f __attribute__((ext_vector_type(2)));
+  const int64_t per = a.ld >> 3, q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (q >= (a.wrows + a.xrows) * per) return;
+  int64_t r = q / per;
+  const int64_t c = (q - r * per) * 8;
+  const bool is_w = r < a.wrows;
+  if (!is_w) r -= a.wrows;
+  const uint2 w = *reinterpret_cast<const uint2*>((is_w ? a.wc : a.xc) + r * a.kp + c);
+  const float s = is_w ? a.ws[(r >> 7) * a.T + (c >> 7)] : a.xs[(c >> 7) * a.m4 + r];
+  const uint32_t words[2] = {w.x, w.y};
+  uint32_t out[4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    float v[4];
+    if constexpr (GRID == GRID_E4M3) {
+      const v2f lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)words[h], false);
+      const v2f hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)words[h], true);
+      v[0] = lo[0] * s; v[1] = lo[1] * s; v[2] = hi[0] * s; v[3] = hi[1] * s;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int code = (int)(int8_t)(uint8_t)(words[h] >> (8 * i));
+        v[i] = code == -128 ? __uint_as_float(0x7FC00000u) : (float)code * s;
+      }
+    }
+    out[2 * h] = (uint32_t)f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1]) << 16);
+    out[2 * h + 1] = (uint32_t)f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16);
+  }
+  *reinterpret_cast<uint4*>((is_w ? a.wd : a.xd) + r * a.ld + c) = make_uint4(out[0], out[1], out[2], out[3]);
 }
 
 static int64_t up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
@@ -74,15 +125,23 @@ static CodeLayout code_layout(const ntlb_linear_plan& p) {
   return l;
 }
 
-// the straight-through backward's scratch: the column sum's partials, and the
-// padded dY (only touched where dY needs it)
+// the straight-through backward's scratch: the column sum's partials, the
+// decoded operands of the gradients that run on tiles below 256x256 (-1: the
+// GEMM decodes), and the padded dY (only touched where dY needs it)
 struct SteLayout {
-  int64_t colsum, dy, bytes;
+  int64_t colsum, wd, xd, dy, bytes;
 };
 static SteLayout ste_layout(const ntlb_linear_plan& p) {
   Carve c;
   SteLayout l;
+  const int64_t k8 = up(p.K, 8), lim = (int64_t)0x7FFFFFFF;
+  const bool small_dx = bf16_small_fits(p.M, p.K, up(p.N, 64), true) && (p.M + 256) * (up(p.N, 64) + 8) * 2 < lim &&
+                        (p.N + 64) * k8 * 2 < lim;
+  const bool small_dw = bf16_small_fits(p.N, p.K, up(p.M, 64), false) && (p.M + 64) * (up(p.N, 64) + 8) * 2 < lim &&
+                        (p.M + 64) * k8 * 2 < lim;
   l.colsum = c.take(std::max<int64_t>(ntlb_colsum_workspace_bytes(p.M, p.N), 4));
+  l.wd = small_dx ? c.take(p.N * k8 * 2) : -1;
+  l.xd = small_dw ? c.take(p.M * k8 * 2) : -1;
   l.dy = c.take(p.M * up(p.N, 64) * 2);
   l.bytes = c.at;
   return l;
@@ -196,13 +255,55 @@ extern "C" int ntlb_linear_ste_backward(const ntlb_linear_plan* p, const void* d
     dy = pad;
     lddy = n64;
   }
-  if (dx) {
+  // row pitches beyond the padded one could leave 32-bit offsets
+  const bool near_rows = lddy <= n64 + 8;
+  const bool small_dx = dx && sl.wd >= 0 && near_rows, small_dw = dw && sl.xd >= 0 && near_rows;
+  if (small_dx || small_dw) {
+    DecodeArgs d{};
+    d.wc = b + l.wc; d.ws = reinterpret_cast<const float*>(b + l.ws);
+    d.xc = b + l.xc; d.xs = reinterpret_cast<const float*>(b + l.xs);
+    d.wrows = small_dx ? p->N : 0;
+    d.xrows = small_dw ? p->M : 0;
+    d.kp = kp; d.T = T; d.m4 = m4; d.ld = up(p->K, 8);
+    d.wd = reinterpret_cast<uint16_t*>(s + std::max<int64_t>(sl.wd, 0));
+    d.xd = reinterpret_cast<uint16_t*>(s + std::max<int64_t>(sl.xd, 0));
+    const int64_t q = (d.wrows + d.xrows) * (d.ld >> 3);
+    if (cdiv(q, 256) > 0x7FFFFFFF) return fail(NTLB_EINVAL, "%s: too large", fn);
+    const unsigned wgs = (unsigned)cdiv(q, 256);
+    if (p->grid == NTLB_GRID_E4M3)
+      decode_operands_kernel<GRID_E4M3><<<wgs, 256, 0, as_stream(stream)>>>(d);
+    else
+      decode_operands_kernel<GRID_INT><<<wgs, 256, 0, as_stream(stream)>>>(d);
+    Bf16Args g{};
+    g.y_dtype = NTLB_BF16;
+    g.ldy = g.N = p->K;
+    if (small_dx) {
+      g.a = Bf16Operand{dy, lddy, p->M, 0, false};
+      g.b = Bf16Operand{d.wd, d.ld, p->K, p->N, true};
+      g.M = p->M;
+      g.Kc = n64;
+      g.y = dx;
+      g.vec_out = aligned(dx, 16) && p->K % 8 == 0;
+      bf16_small_launch(g, as_stream(stream));
+    }
+    if (small_dw) {
+      g.a = Bf16Operand{dy, lddy, p->N, p->M, true};
+      g.b = Bf16Operand{d.xd, d.ld, p->K, p->M, true};
+      g.M = p->N;
+      g.Kc = up(p->M, 64);
+      g.y = dw;
+      g.vec_out = aligned(dw, 16) && p->K % 8 == 0;
+      bf16_small_launch(g, as_stream(stream));
+    }
+    if (int rc = check_launch(fn)) return rc;
+  }
+  if (dx && !small_dx) {
     const int rc = ntlb_gemm_ste_dgrad_ws(NTLB_BF16, dy, lddy, p->M, p->N, p->grid, b + l.wc, kp,
                                           reinterpret_cast<const float*>(b + l.ws), T, 1, 7, p->K, dx, NTLB_BF16,
                                           p->K, workspace, ws_bytes, stream);
     if (rc) return rc;
   }
-  if (dw) {
+  if (dw && !small_dw) {
     const int rc = ntlb_gemm_ste_wgrad(NTLB_BF16, dy, lddy, p->M, p->N, p->grid, b + l.xc, kp,
                                        reinterpret_cast<const float*>(b + l.xs), 1, m4, 0, p->K, dw, NTLB_BF16,
                                        p->K, stream);

@@ -1,0 +1,46 @@
+// bf16 GEMMs on tiles below 256x256 (gemm_bf16.hip): what their callers pass.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+namespace ntlb {
+
+// One operand of Y[M,N] = A . B^T over plain bf16 matrices.
+//   tr = false: [rows, >= Kc] row-major, the contraction contiguous; columns
+//     past the contraction are zero or meet zeros of the other operand
+//   tr = true: stored transposed, element (r, k) at p[k * ld + r]; contraction
+//     rows at or past kvalid read zero
+// 16-byte aligned with whole 16-byte rows, addressed with 32-bit byte offsets
+// ((rows + 256) * ld * 2 and (kvalid + 64) * ld * 2 below 2^31).
+struct Bf16Operand {
+  const void* p;
+  int64_t ld;
+  int64_t rows;
+  int64_t kvalid;
+  bool tr;
+};
+
+struct Bf16Args {
+  Bf16Operand a, b;
+  int64_t M, N, Kc;  // Kc a multiple of 64
+  const void* bias;
+  int bias_dtype;
+  void* y;
+  int y_dtype;
+  int64_t ldy;
+  int vec_out;  // y 16-byte aligned with 16-byte row pitch
+};
+
+// split-K tail of the 256x256-tile GEMMs over dequantized operands: minimum K
+// steps per range
+constexpr int DQ_SPLIT_MIN_STEPS = 9;
+
+// whether a product of this shape runs on these tiles rather than on 256x256
+// ones (big_split: those would have a split-K workspace), and the launch (a tr
+// B with a non-tr A, both tr, or neither)
+bool bf16_small_fits(int64_t M, int64_t N, int64_t Kc, bool big_split);
+void bf16_small_launch(const Bf16Args& g, hipStream_t st);
+
+}  // namespace ntlb

@@ -61,6 +61,7 @@ SIGNATURES = {
     "ntlb_gemm_grouped_swiglu_quant": [_I32, _P, _I64, _P, _I64, _I64, _I32, _P, _I64, _I64, _P, _I64, _I64, _I64,
                                        _P, _I32, _I64, _I64, _I64, _P, _P, _P, _I64, _P, _I64, _P, _I64, _I64, _P,
                                        _I32, _I32, _I32, _U64, _U64, _P],
+    "ntlb_gemm_bf16_tn": [_P, _I64, _P, _I64, _I64, _I64, _I64, _P, _I32, _I64, _P],
     "ntlb_linear_plan_init": [_P],
     "ntlb_linear_forward": [_P, _P, _P, _P, _P, _P, _P, _I64, _U64, _P],
     "ntlb_linear_ste_backward": [_P, _P, _I64, _P, _P, _P, _P, _I32, _P, _I64, _P, _I64, _P],

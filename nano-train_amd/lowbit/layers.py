@@ -67,7 +67,8 @@ class _FusedPersistentLinear(torch.autograd.Function):
             dx = P.dgrad(dy2, codes, scale, fmt=fmt, out_features=N, in_features=K,
                          out_dtype=x.dtype).reshape(x.shape)
         if ctx.needs_input_grad[1]:
-            dw = ops.gemm_dense_tn(dy2, x.reshape(-1, K).to(dy2.dtype), out_dtype=wdt)
+            tn = ops.gemm_bf16_tn if dy2.dtype == torch.bfloat16 else ops.gemm_dense_tn
+            dw = tn(dy2, x.reshape(-1, K).to(dy2.dtype), out_dtype=wdt)
         if ctx.needs_input_grad[2]:
             db = ops.colsum(dy2, out_dtype=bdt)
         return dx, dw, db, None, None, None, None

@@ -827,6 +827,23 @@ def gemm_dense_tn(a: torch.Tensor, b: torch.Tensor, *, out_dtype: torch.dtype = 
     return out
 
 
+def gemm_bf16_tn(a: torch.Tensor, b: torch.Tensor, *, out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
+    """gemm_dense_tn of bf16 matrices with the output tile chosen by shape
+    (ntlb_gemm_bf16_tn): small products sum K in ranges."""
+    _require_device(a, b)
+    if a.dtype != torch.bfloat16 or b.dtype != torch.bfloat16:
+        raise TypeError("gemm_bf16_tn takes bf16 operands")
+    K, M = a.shape
+    if b.shape[0] != K:
+        raise ValueError(f"contraction mismatch: {K} vs {b.shape[0]}")
+    N = b.shape[1]
+    ap, bp = _pad_cols(a, 8), _pad_cols(b, 8)
+    out = torch.empty((M, N), dtype=out_dtype, device=a.device)
+    call("ntlb_gemm_bf16_tn", ap.data_ptr(), ap.stride(0), bp.data_ptr(), bp.stride(0), M, N, K, out.data_ptr(),
+         _dtype_code(out_dtype), out.stride(0), _stream())
+    return out
+
+
 _colsum_ws: dict = {}
 
 
