@@ -740,6 +740,10 @@ extern "C" int ntlb_gemm_grouped_blockscaled(int grid, const uint8_t* a, int64_t
   g.split_base = 0; g.split_s = 1; g.ws = nullptr; g.ws_count = nullptr;
   const bool b_uniform = (b_shift == 7) || (sb_row == 0);
   hipStream_t st = as_stream(stream);
+  if (b_uniform && small_grouped_fits(M_total, n_experts, N)) {
+    small_grouped_launch(grid, g, st);
+    return check_launch(fn);
+  }
   dim3 grd((unsigned)tiles), blk(NTHREADS);
   if (grid == NTLB_GRID_E4M3) {
     if (b_uniform)
@@ -879,6 +883,10 @@ extern "C" int ntlb_gemm_grouped_swiglu_quant_gu(int grid, const uint8_t* a, int
                          seed, offset);
   if (rc) return rc;
   hipStream_t st = as_stream(stream);
+  if (small_grouped_fits(M_total, n_experts, N)) {
+    small_grouped_swiglu_launch(grid, g, st);
+    return check_launch(fn);
+  }
   dim3 grd((unsigned)tiles), blk(NTHREADS);
   if (grid == NTLB_GRID_E4M3)
     gemm_blockscaled_kernel<GRID_E4M3, true, true, EPI_SWIGLU><<<grd, blk, 0, st>>>(g);

@@ -497,4 +497,231 @@ void small_gemm_launch(int grid, bool b_uniform, const GemmArgs& g, hipStream_t 
   }
 }
 
+// ---------------------------------------------------------------------------
+// Per-expert products of few rows each (the expert loop while generating, or
+// at small batches).  The 256x256-tile kernels give an expert's 8 rows a whole
+// tile: 31/32 of the matrix work is padding and two rounds of tiles of 56 K
+// blocks set the time, at 45% of the memory rate the weights could stream at.
+// Here a wave owns 16*MB rows by 16*NB columns of one expert over all of K (the
+// sums are those of the 256x256 tiles, bit for bit) and streams its weight
+// rows through NS LDS stages of its own.
+// ---------------------------------------------------------------------------
+
+// Row tile `pid` of experts in order, `rows` rows each: the expert, its first
+// row in the tile and its end.  Wave-uniform; false past the last tile.
+__device__ __forceinline__ bool expert_tile(const int32_t* offsets, int n_experts, int rows, int pid, int lane, int& e,
+                                            int& m0, int& hi) {
+  int before = 0;
+  for (int base = 0; base < n_experts; base += 64) {
+    const int i = base + lane;
+    const int lo = i < n_experts ? offsets[i] : 0, end = i < n_experts ? offsets[i + 1] : 0;
+    const int tiles = (end - lo + rows - 1) / rows;
+    int incl = tiles;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int t = __shfl_up(incl, d);
+      if (lane >= d) incl += t;
+    }
+    const uint64_t hit = __ballot(before + incl > pid);
+    if (hit) {
+      const int l = __builtin_ctzll(hit);
+      e = __builtin_amdgcn_readfirstlane(base + l);
+      const int first = before + __shfl(incl, l) - __shfl(tiles, l);
+      m0 = __builtin_amdgcn_readfirstlane(__shfl(lo, l) + (pid - first) * rows);
+      hi = __builtin_amdgcn_readfirstlane(__shfl(end, l));
+      return true;
+    }
+    before += __shfl(incl, 63);
+  }
+  return false;
+}
+
+__device__ __forceinline__ void take_expert(GemmArgs& g, int e, int hi) {
+  g.M = hi;  // rows at or past the expert's end read zero and are not stored
+  g.b += (int64_t)e * g.b_estride;
+  g.sb += (int64_t)e * g.sb_estride;
+  if (g.nan_b) g.nan_b += (int64_t)e * g.N;
+}
+
+template <int GRID, int MB, int NB, int NS>
+__global__ void __launch_bounds__(256) gemm_small_grouped_kernel(GemmArgs g) {
+  constexpr int WB = WaveCopy<MB, NB>::BYTES;
+  __shared__ __attribute__((aligned(16))) uint8_t st0[4 * WB];
+  __shared__ __attribute__((aligned(16))) uint8_t st1[4 * WB];
+  __shared__ __attribute__((aligned(16))) uint8_t st2[NS > 2 ? 4 * WB : 16];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t n0 = ((int64_t)blockIdx.x * 4 + wave) * (16 * NB);
+  int e, m0, hi;
+  if (n0 >= g.N || !expert_tile(g.offsets, g.n_experts, 16 * MB, (int)blockIdx.y, lane, e, m0, hi)) return;
+  take_expert(g, e, hi);
+  v4f acc[MB][NB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = (v4f){0.f, 0.f, 0.f, 0.f};
+  WaveCopy<MB, NB> cp;
+  cp.init(g, m0, n0, lane);
+  small_k_loop<GRID, true, MB, NB, NS>(g, cp, m0, n0, 0, (int)(g.Kp / BK), st0 + wave * WB, st1 + wave * WB,
+                                            st2 + (NS > 2 ? wave * WB : 0), lane, acc);
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      const int64_t m = m0 + mb * 16 + (lane & 15), n = n0 + nb * 16 + (lane >> 4) * 4;
+      if (m < g.M && n < g.N) small_store4(g, m, n, acc[mb][nb], g.nan_b);
+    }
+}
+
+// The gate/up projection with the SwiGLU and h's 1x128 quantization: eight
+// waves of 32 columns make the 128 gate and 128 up columns of one h tile; the
+// bf16 projections meet in LDS and 16 lanes finish an h tile of a row (the
+// arithmetic of gemm.hip's swiglu_quant_rows).
+template <int GRID, int MB, int NS, bool SR>
+__global__ void __launch_bounds__(512) gemm_small_grouped_swiglu_kernel(GemmArgs g) {
+#pragma clang fp contract(off)
+  constexpr int WB = WaveCopy<MB, 2>::BYTES;
+  static_assert(16 * MB * 512 <= 8 * WB, "the projections fit the first stage");
+  __shared__ __attribute__((aligned(16))) uint8_t st0[8 * WB];
+  __shared__ __attribute__((aligned(16))) uint8_t st1[8 * WB];
+  __shared__ __attribute__((aligned(16))) uint8_t st2[NS > 2 ? 8 * WB : 16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int e, m0, hi;
+  if (!expert_tile(g.offsets, g.n_experts, 16 * MB, (int)blockIdx.y, lane, e, m0, hi)) return;
+  take_expert(g, e, hi);
+  const int64_t n0 = (int64_t)blockIdx.x * 256, nw = n0 + wave * 32;
+  v4f acc[MB][2];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) acc[mb][0] = acc[mb][1] = (v4f){0.f, 0.f, 0.f, 0.f};
+  WaveCopy<MB, 2> cp;
+  cp.init(g, m0, nw, lane);
+  small_k_loop<GRID, true, MB, 2, NS>(g, cp, m0, nw, 0, (int)(g.Kp / BK), st0 + wave * WB, st1 + wave * WB,
+                                      st2 + (NS > 2 ? wave * WB : 0), lane, acc);
+  __syncthreads();  // every wave is done with its stages
+  const float qnan = __uint_as_float(0x7FC00000u);
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+    const int r = mb * 16 + (lane & 15);
+    const bool nan_m = g.nan_a && g.nan_a[min<int64_t>(m0 + r, g.M - 1)] != 0;
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+      const int c = wave * 32 + nb * 16 + (lane >> 4) * 4;
+      float v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        v[q] = nan_m || (g.nan_b && g.nan_b[n0 + c + q] != 0) ? qnan : acc[mb][nb][q];
+      // 512-byte rows, 16-byte units swizzled by row
+      *reinterpret_cast<uint2*>(st0 + r * 512 + (((c >> 3) ^ (r & 15)) << 4) + (c & 4) * 2) =
+          make_uint2((uint32_t)f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1]) << 16),
+                     (uint32_t)f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16));
+    }
+  }
+  __syncthreads();
+  for (int r = tid >> 4; r < 16 * MB; r += 32) {
+    const int64_t m = m0 + r;
+    if (m >= g.M) break;  // uniform over the row's 16 lanes
+    const int u = tid & 15;  // h columns 8u .. 8u+7 of the tile
+    const uint4 gw = *reinterpret_cast<const uint4*>(st0 + r * 512 + ((u ^ (r & 15)) << 4));
+    const uint4 uw = *reinterpret_cast<const uint4*>(st0 + r * 512 + (((16 + u) ^ (r & 15)) << 4));
+    if (g.gu) {
+      uint16_t* gup = g.gu + m * g.ldgu + n0 + u * 8;
+      *reinterpret_cast<uint4*>(gup) = gw;
+      *reinterpret_cast<uint4*>(gup + 128) = uw;
+    }
+    const uint32_t gg[4] = {gw.x, gw.y, gw.z, gw.w}, uu[4] = {uw.x, uw.y, uw.z, uw.w};
+    float hv[8];
+    uint32_t hb[4], amax = 0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const float gv = bf16_bits_to_f32((gg[q >> 1] >> (16 * (q & 1))) & 0xFFFFu);
+      const float uv = bf16_bits_to_f32((uu[q >> 1] >> (16 * (q & 1))) & 0xFFFFu);
+      const float sg = bf16_bits_to_f32(f32_to_bf16_bits(gv / (1.0f + expf(-gv))));
+      const uint32_t h = f32_to_bf16_bits(sg * uv);
+      amax = max(amax, (h & 0x7FFFu) << 16);
+      hv[q] = bf16_bits_to_f32(h);
+      hb[q >> 1] = (q & 1) ? (hb[q >> 1] | (h << 16)) : h;
+    }
+    amax = row16_max_u32(amax);
+    const float s = scale_from_amax_bits(amax, g.h_qmaxf, g.h_scale_rule);
+    const float rs = fast_div_ok<SR>(amax) ? 1.0f / s : 1.0f;
+    const int64_t j0 = n0 / 2 + u * 8;
+    uint32_t rb[8], lo, hi32;
+    float q8[8];
+    sr_words<SR>((uint64_t)(m * g.I + j0), g.h_seed, g.h_offset, rb);
+    const bool nan = quant8_tile_rs<GRID, SR, false>(hv, amax, s, rs, g.h_qmaxf, rb, lo, hi32, q8);
+    *reinterpret_cast<uint2*>(g.hc + m * g.ldhc + j0) = make_uint2(lo, hi32);
+    if (g.h) *reinterpret_cast<uint4*>(g.h + m * g.ldh + j0) = make_uint4(hb[0], hb[1], hb[2], hb[3]);
+    if (u == 0) {
+      g.hs[m * g.hs_row + (n0 / 256) * g.hs_col] = s;
+      if (nan && g.h_nan) atomicOr(g.h_nan + m, 1);
+    }
+  }
+}
+
+// Row blocks of 16 per tile for R rows over E experts of N weight rows each, 0
+// for the 256x256 tiles.  The rows of each expert are known on the device only,
+// so the average decides: skewed counts cost more tiles of one weight, which
+// its XCDs' L2 hold.  us, 256x256 tiles | MB 1 | MB 2, rows routed unevenly:
+//   gate/up 32 experts 4096 x 7168   average 1: 124 |  86 |  87   4: 224 | 141 | 150   8: 228 | 186 | 166
+//     (8 rows: 5.6 TB/s of codes)            16: 230 | 218 | 205  32: 234 | 259 | 237  64: 247 | 406 | 299
+//   down 32 experts 7168 x 2048      average 1:  56 |  46 |  46   4: 105 |  88 |  89   8: 135 | 103 |  95
+//                                            16: 135 | 118 | 111  32: 137 | 159 | 129  64: 140 | 250 | 187
+//   gate/up 8 experts 2048 x 2048            1:  40 |  20 |  19  32:  40 |  19 |  21  64:  47 |  27 |  20  128: 46 | 38 | 35
+//   down 8 experts 2048 x 1024               1:  17 |  10 |  10  32:  17 |  10 |  12  64:  19 |  16 |  12  128: 19 | 22 | 21
+// So up to 24 rows each, and up to 64 where the 256x256 tiles leave half of
+// the chip's 256 compute units without a tile.
+static int grouped_mb(int64_t R, int64_t E, int64_t N) {
+  if (E > 16384) return 0;  // the row tiles are the grid's y
+  if (R <= 4 * E) return 1;
+  const bool few = (cdiv(R, 256) + E) * cdiv(N, 256) <= 128;
+  return R <= (few ? 64 : 24) * E ? 2 : 0;
+}
+
+bool small_grouped_fits(int64_t R, int64_t E, int64_t N) { return grouped_mb(R, E, N) != 0; }
+
+template <int GRID>
+static void grouped_launch(const GemmArgs& g, hipStream_t st) {
+  const int mb = grouped_mb(g.M, g.n_experts, g.N);
+  // no more row tiles than rows, and one ragged tile per expert
+  const int64_t tiles = std::min<int64_t>(g.M, cdiv(g.M, 16 * mb) + g.n_experts);
+  // column workgroups in whole rounds over the XCDs: an expert's row tiles then
+  // read the same weight rows through the same L2
+  const dim3 grd((unsigned)(cdiv(g.N, 4 * 64) + 7) / 8 * 8, (unsigned)tiles);
+  if (mb == 1)
+    gemm_small_grouped_kernel<GRID, 1, 4, 3><<<grd, 256, 0, st>>>(g);
+  else
+    gemm_small_grouped_kernel<GRID, 2, 4, 2><<<grd, 256, 0, st>>>(g);
+}
+
+void small_grouped_launch(int grid, const GemmArgs& g, hipStream_t st) {
+  if (grid == GRID_E4M3)
+    grouped_launch<GRID_E4M3>(g, st);
+  else
+    grouped_launch<GRID_INT>(g, st);
+}
+
+template <int GRID, bool SR>
+static void grouped_swiglu_launch(const GemmArgs& g, hipStream_t st) {
+  const int mb = grouped_mb(g.M, g.n_experts, g.N);
+  const int64_t tiles = std::min<int64_t>(g.M, cdiv(g.M, 16 * mb) + g.n_experts);
+  const dim3 grd((unsigned)(g.N / 256), (unsigned)tiles);
+  if (mb == 1)
+    gemm_small_grouped_swiglu_kernel<GRID, 1, 3, SR><<<grd, 512, 0, st>>>(g);
+  else
+    gemm_small_grouped_swiglu_kernel<GRID, 2, 2, SR><<<grd, 512, 0, st>>>(g);
+}
+
+void small_grouped_swiglu_launch(int grid, const GemmArgs& g, hipStream_t st) {
+  if (grid == GRID_E4M3) {
+    if (g.h_sr)
+      grouped_swiglu_launch<GRID_E4M3, true>(g, st);
+    else
+      grouped_swiglu_launch<GRID_E4M3, false>(g, st);
+  } else {
+    if (g.h_sr)
+      grouped_swiglu_launch<GRID_INT, true>(g, st);
+    else
+      grouped_swiglu_launch<GRID_INT, false>(g, st);
+  }
+}
+
 }  // namespace ntlb

@@ -161,4 +161,10 @@ constexpr int SPLIT_MIN_BLOCKS = 9;
 bool small_gemm_fits(int64_t M, int64_t N, int64_t Kp);
 void small_gemm_launch(int grid, bool b_uniform, const GemmArgs& g, hipStream_t st);
 
+// the same for per-expert products: M_total rows over n_experts experts of N
+// weight rows, B's scale uniform over a wave's columns
+bool small_grouped_fits(int64_t M_total, int64_t n_experts, int64_t N);
+void small_grouped_launch(int grid, const GemmArgs& g, hipStream_t st);
+void small_grouped_swiglu_launch(int grid, const GemmArgs& g, hipStream_t st);
+
 }  // namespace ntlb

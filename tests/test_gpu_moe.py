@@ -305,3 +305,44 @@ def test_grouped_gemm_tile_boundaries(gpu_device, fmt, grid):
         lo = sum(counts[:e])
         if c:
             assert rel_fro_bf16(y[lo:lo + c], ref[lo:lo + c]) <= 1e-3, f"expert {e} ({c} rows)"
+
+
+@pytest.mark.parametrize("fmt", ["e4m3", "int_grid"])
+@pytest.mark.parametrize("E,counts", [
+    (70, {0: 1, 3: 16, 64: 17, 69: 40}),  # 16-row tiles; the expert search passes its first 64
+    (6, {0: 33, 2: 32, 3: 1, 5: 130}),  # 32-row tiles, one expert with a lot more than the average
+])
+def test_few_rows_per_expert_match_single_expert_calls(gpu_device, fmt, E, counts):
+    """The few-row expert tiles against the 256x256 tiles, which the same rows
+    take when each expert is called on its own (more than 64 rows for the one
+    expert): both sum the K blocks in order, so every output bit agrees."""
+    from lowbit import moe, ops
+
+    H, I, N = 384, 256, 384
+    counts = [counts.get(e, 0) for e in range(E)]
+    T = sum(counts) + 3  # rows past the last expert belong to nobody
+    x = seeded((T, H), seed=20262401, outliers=0.01).to(gpu_device)
+    x[0, 7] = float("nan")
+    qx = ops.quant_tile_1x128(x, fmt=fmt, want_nan_rows=True)
+    wc, ws, wn = moe.quantize_expert_weights(seeded((E, N, H), seed=20262402, std=0.03).to(gpu_device), fmt=fmt)
+    gc, gs, gn = moe.quantize_expert_weights(seeded((E, 2 * I, H), seed=20262403, std=0.03).to(gpu_device), fmt=fmt)
+    wn[:, 5] = gn[:, 130] = 1
+    bounds = np.concatenate([[0], np.cumsum(counts)])
+    offs = torch.tensor(bounds, dtype=torch.int32, device=gpu_device)
+    kw = dict(fmt=fmt, rounding="stochastic", seed=43, offset=5, want_nan_rows=True)
+    gu = torch.zeros((T, 2 * I), dtype=torch.bfloat16, device=gpu_device)
+    y = ops.gemm_grouped_blockscaled(qx, wc, ws, offs, N=N, b_nan_rows=wn)
+    h, qh = ops.gemm_swiglu_quant(qx, gc, gs, offsets=offs, b_nan_rows=gn, gu_out=gu, **kw)
+    bits = lambda t: t.view(torch.int16)  # noqa: E731
+    for e in np.flatnonzero(counts):
+        r = slice(int(bounds[e]), int(bounds[e + 1]))
+        one = torch.tensor([r.start, r.stop], dtype=torch.int32, device=gpu_device)
+        gu1 = torch.zeros_like(gu)
+        y1 = ops.gemm_grouped_blockscaled(qx, wc[e:e + 1], ws[e:e + 1], one, N=N, b_nan_rows=wn[e:e + 1])
+        h1, qh1 = ops.gemm_swiglu_quant(qx, gc[e:e + 1], gs[e:e + 1], offsets=one, b_nan_rows=gn[e:e + 1],
+                                        gu_out=gu1, **kw)
+        assert torch.equal(bits(y[r]), bits(y1[r])), f"expert {e}"
+        assert torch.equal(bits(h[r]), bits(h1[r])) and torch.equal(bits(gu[r]), bits(gu1[r])), f"expert {e}"
+        assert torch.equal(qh.codes[r], qh1.codes[r]) and torch.equal(qh.scales[:, r], qh1.scales[:, r])
+        assert torch.equal(qh.nan_rows[r], qh1.nan_rows[r])
+    assert int(gu[T - 3:].count_nonzero()) == 0
