@@ -28,6 +28,7 @@
 // metadata in that order for the grouped GEMM.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "ntlb_device.h"
@@ -102,7 +103,7 @@ __global__ void __launch_bounds__(EP_SCAN_THREADS) ep_scan_kernel(int32_t* hist,
                                                                   int64_t* counts, int32_t* offsets) {
   __shared__ int32_t base[EP_MAX_BUCKETS + 1];
   __shared__ int32_t wsum[EP_SCAN_THREADS / 64 + 1];
-  for (int d = threadIdx.x; d <= buckets; d += EP_SCAN_THREADS) base[d] = 0;  // n == 0: every offset is 0
+  for (int d = threadIdx.x; d <= buckets; d += EP_SCAN_THREADS) base[d] = 0;
   const int64_t L = nb * buckets;
   const int64_t seg = (L + EP_SCAN_THREADS - 1) / EP_SCAN_THREADS;
   const int64_t lo = min<int64_t>(L, (int64_t)threadIdx.x * seg), hi = min<int64_t>(L, lo + seg);
@@ -110,18 +111,16 @@ __global__ void __launch_bounds__(EP_SCAN_THREADS) ep_scan_kernel(int32_t* hist,
   for (int64_t j = lo; j < hi; ++j) s += hist[j];
   int32_t total;
   int32_t run = ep_block_scan(s, wsum, &total);  // its barriers also order the base[] clears above
-  if (nb > 0) {
-    int64_t d = (lo + nb - 1) / nb, next = d * nb;  // first bucket starting at or after lo
-    for (int64_t j = lo; j < hi; ++j) {
-      if (j == next) {
-        base[d] = run;  // bucket d starts with block 0
-        ++d;
-        next += nb;
-      }
-      const int32_t c = hist[j];
-      hist[j] = run;
-      run += c;
+  int64_t d0 = (lo + nb - 1) / nb, next = d0 * nb;  // first bucket starting at or after lo
+  for (int64_t j = lo; j < hi; ++j) {
+    if (j == next) {
+      base[d0] = run;  // bucket d0 starts with block 0
+      ++d0;
+      next += nb;
     }
+    const int32_t c = hist[j];
+    hist[j] = run;
+    run += c;
   }
   if (threadIdx.x == 0) base[buckets] = total;
   __syncthreads();
@@ -147,6 +146,55 @@ __global__ void __launch_bounds__(EP_BLOCK) ep_place_kernel(const uint8_t* keys,
   const int32_t p = start[(int64_t)b * gridDim.x + blockIdx.x] + rank;
   if (pos) pos[i] = p;
   if (inv) inv[p] = (int32_t)i;
+}
+
+// The three passes in one workgroup, for n <= EP_SCAN_THREADS keys: histogram,
+// exclusive scan and stable places all in LDS.  Such a sort is launch latency
+// alone (256 keys, 32 buckets: three kernels of 4.6, 4.6 and 5.9 us became one
+// of 7.2); the limit is one key per thread of the largest workgroup.
+__global__ void __launch_bounds__(EP_SCAN_THREADS) ep_partition_small_kernel(const uint8_t* keys, int key_dt,
+                                                                             int64_t stride, int n, int64_t divisor,
+                                                                             int buckets, int32_t* pos, int32_t* inv,
+                                                                             int64_t* counts, int32_t* offsets) {
+  __shared__ int32_t h[EP_MAX_BUCKETS];
+  __shared__ int32_t kb[EP_SCAN_THREADS] __attribute__((aligned(16)));
+  __shared__ int32_t wsum[EP_SCAN_THREADS / 64 + 1];
+  const int i = threadIdx.x;
+  const int b = i < n ? ep_bucket(keys, key_dt, stride, i, divisor, buckets) : -1;
+  for (int d = i; d < buckets; d += EP_SCAN_THREADS) h[d] = 0;
+  kb[i] = b;
+  __syncthreads();
+  if (b >= 0) atomicAdd(&h[b], 1);
+  __syncthreads();
+  // a thread's contiguous segment of buckets, as in ep_scan_kernel
+  const int seg = (buckets + EP_SCAN_THREADS - 1) / EP_SCAN_THREADS;
+  const int lo = min(buckets, i * seg), hi = min(buckets, lo + seg);
+  int32_t s = 0, total;
+  for (int d = lo; d < hi; ++d) s += h[d];
+  int32_t run = ep_block_scan(s, wsum, &total);
+  for (int d = lo; d < hi; ++d) {
+    const int32_t c = h[d];
+    h[d] = run;
+    if (offsets) offsets[d] = run;
+    if (counts) counts[d] = c;
+    run += c;
+  }
+  if (i == 0 && offsets) offsets[buckets] = total;
+  __syncthreads();
+  if (b < 0) return;
+  // earlier keys of the same bucket: those of the waves before (four a read,
+  // the same address in every lane), then those of the own wave
+  int rank = 0;
+  const int wave0 = i & ~63;
+  for (int j = 0; j < wave0; j += 4) {
+    const int4 q = *reinterpret_cast<const int4*>(kb + j);
+    rank += (q.x == b) + (q.y == b) + (q.z == b) + (q.w == b);
+  }
+#pragma unroll 8
+  for (int j = 0; j < 64; ++j) rank += (kb[wave0 + j] == b && wave0 + j < i) ? 1 : 0;
+  const int32_t p = h[b] + rank;
+  if (pos) pos[i] = p;
+  if (inv) inv[p] = i;
 }
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -392,6 +440,8 @@ __global__ void __launch_bounds__(256) ep_combine_kernel(const uint8_t* rec, int
 // nothing).  Per expert,
 // the product is rounded to the promoted dtype of y and w (ROUND_P: both the
 // output dtype) and the sum to the output dtype, as the two torch ops do.
+// blockIdx.y takes the columns [cols * y, +cols): few tokens split their rows
+// over workgroups, each of one pass over its columns.
 constexpr int COMBINE_ROWS_THREADS = 128;
 
 template <int OUT_DT, bool ROUND_P>
@@ -399,12 +449,13 @@ __global__ void __launch_bounds__(COMBINE_ROWS_THREADS) moe_combine_rows_kernel(
                                                                const int32_t* pos,
                                                                const void* topk_idx, int idx_dt, const void* topk_w,
                                                                int w_dt, int K, int64_t H, void* out, int64_t ldo,
-                                                               int vec) {
+                                                               int vec, int64_t cols) {
 #pragma clang fp contract(off)  // each product and sum rounds on its own
   __shared__ int64_t s_e[EP_COMBINE_MAX_K];
   __shared__ int32_t s_row[EP_COMBINE_MAX_K];
   __shared__ float s_w[EP_COMBINE_MAX_K];
   const int64_t t = blockIdx.x;
+  const int64_t c_begin = (int64_t)blockIdx.y * cols, c_end = min(H, c_begin + cols);
   const int k = threadIdx.x;
   if (k < K) {
     const int64_t a = t * K + k;
@@ -431,7 +482,7 @@ __global__ void __launch_bounds__(COMBINE_ROWS_THREADS) moe_combine_rows_kernel(
       // so the same bits.
       constexpr int64_t STEP = COMBINE_ROWS_THREADS * 8;
       constexpr int D = 2;
-      for (int64_t c0 = (int64_t)threadIdx.x * 8; c0 < H; c0 += D * STEP) {
+      for (int64_t c0 = c_begin + (int64_t)threadIdx.x * 8; c0 < c_end; c0 += D * STEP) {
         uint4 raw[D][8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
@@ -439,11 +490,11 @@ __global__ void __launch_bounds__(COMBINE_ROWS_THREADS) moe_combine_rows_kernel(
           const uint16_t* rowp = reinterpret_cast<const uint16_t*>(y) + min<int64_t>(max(s_row[j], 0), n - 1) * ldy;
 #pragma unroll
           for (int h = 0; h < D; ++h)
-            raw[h][u] = c0 + h * STEP < H ? *reinterpret_cast<const uint4*>(rowp + c0 + h * STEP) : make_uint4(0, 0, 0, 0);
+            raw[h][u] = c0 + h * STEP < c_end ? *reinterpret_cast<const uint4*>(rowp + c0 + h * STEP) : make_uint4(0, 0, 0, 0);
         }
 #pragma unroll
         for (int h = 0; h < D; ++h) {
-          if (c0 + h * STEP >= H) break;
+          if (c0 + h * STEP >= c_end) break;
           float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int u = 0; u < 8; ++u) {
@@ -470,7 +521,7 @@ __global__ void __launch_bounds__(COMBINE_ROWS_THREADS) moe_combine_rows_kernel(
       return;
     }
   }
-  for (int64_t c0 = (int64_t)threadIdx.x * 8; c0 < H; c0 += COMBINE_ROWS_THREADS * 8) {
+  for (int64_t c0 = c_begin + (int64_t)threadIdx.x * 8; c0 < c_end; c0 += COMBINE_ROWS_THREADS * 8) {
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int j0 = 0; j0 < K; j0 += 8) {
       // up to eight rows in flight at once: slots past K or dropped read row
@@ -630,12 +681,15 @@ extern "C" int ntlb_ep_partition(const void* keys, int key_dtype, int64_t key_st
                                                              (long long)(nb * buckets));
   hipStream_t st = as_stream(stream);
   const uint8_t* k = reinterpret_cast<const uint8_t*>(keys);
-  if (n > 0)
-    ep_hist_kernel<<<(unsigned)nb, EP_BLOCK, buckets * sizeof(int32_t), st>>>(k, key_dtype, key_stride, n, divisor,
-                                                                             buckets, ws);
+  if (n <= EP_SCAN_THREADS) {
+    ep_partition_small_kernel<<<1, EP_SCAN_THREADS, 0, st>>>(k, key_dtype, key_stride, (int)n, divisor, buckets, pos,
+                                                             inv, counts, offsets);
+    return check_launch(fn);
+  }
+  ep_hist_kernel<<<(unsigned)nb, EP_BLOCK, buckets * sizeof(int32_t), st>>>(k, key_dtype, key_stride, n, divisor,
+                                                                           buckets, ws);
   ep_scan_kernel<<<1, EP_SCAN_THREADS, 0, st>>>(ws, nb, buckets, counts, offsets);
-  if (n > 0)
-    ep_place_kernel<<<(unsigned)nb, EP_BLOCK, 0, st>>>(k, key_dtype, key_stride, n, divisor, buckets, ws, pos, inv);
+  ep_place_kernel<<<(unsigned)nb, EP_BLOCK, 0, st>>>(k, key_dtype, key_stride, n, divisor, buckets, ws, pos, inv);
   return check_launch(fn);
 }
 
@@ -799,9 +853,18 @@ extern "C" int ntlb_moe_combine_rows(const void* y, int64_t ldy, int64_t n, cons
   // the product rounds to the output dtype when torch's promotion of (y, w)
   // is that dtype: w of the same dtype, which is not fp32
   const bool round_p = w_dtype == out_dtype && out_dtype != NTLB_F32;
+  // A workgroup per token walks its row in serial passes of loads; with fewer
+  // tokens than two workgroups per compute unit the row is split at whole
+  // passes (32 tokens, K 8, H 7168: 14.2 us on 32 workgroups, 6.0
+  // on 224).  From 512 tokens on, every unit has its workgroups without.
+  constexpr int64_t PASS = COMBINE_ROWS_THREADS * 8;
+  const int64_t passes = cdiv(H, PASS);
+  const int64_t parts = std::min(passes, std::max<int64_t>(1, 512 / T));
+  const int64_t cols = cdiv(passes, parts) * PASS;
+  const dim3 grd((unsigned)T, (unsigned)cdiv(H, cols));
   auto launch = [&](auto outc, auto rpc) {
-    moe_combine_rows_kernel<decltype(outc)::value, decltype(rpc)::value><<<(unsigned)T, COMBINE_ROWS_THREADS, 0, st>>>(
-        y, ldy, n, pos, topk_idx, idx_dtype, topk_w, w_dtype, (int)K, H, out, ldo, vec);
+    moe_combine_rows_kernel<decltype(outc)::value, decltype(rpc)::value><<<grd, COMBINE_ROWS_THREADS, 0, st>>>(
+        y, ldy, n, pos, topk_idx, idx_dtype, topk_w, w_dtype, (int)K, H, out, ldo, vec, cols);
   };
   using B = std::integral_constant<int, DT_BF16>;
   using F = std::integral_constant<int, DT_F32>;

@@ -183,7 +183,8 @@ def compute_capacity(capacity_factor: float, num_tokens: int, top_k: int, num_ex
 def route_by_expert(expert_ids: torch.Tensor, n_experts: int, *, capacity: int = 0,
                     topk_w: Optional[torch.Tensor] = None) -> ExpertRouting:
     """One stable counting sort of expert_ids [T, k] (int32 or int64) by
-    expert on the GPU (ntlb_ep_partition: three kernels, no host sync).
+    expert on the GPU (ntlb_ep_partition: one kernel up to 1024 assignments,
+    three above, no host sync).
 
     capacity > 0 keeps, per expert with more rows than that, the `capacity`
     rows of highest routing weight topk_w [T, k], highest first
@@ -334,8 +335,8 @@ def expert_mlp(
                                   want_nan_rows=True)
         out_dtype = out_dtype or x_sorted.dtype
     h, qh = ops.gemm_swiglu_quant(qx, gu_codes, gu_scales, offsets=offsets, fmt=fmt, bits=bits, rounding=rounding,
-                                  seed=seed, offset=offset + 1, want_h=want_h, want_nan_rows=True,
-                                  b_nan_rows=gu_nan)
+                                  seed=seed, offset=offset + 1, want_h=want_h,
+                                  want_nan_rows=fmt != "e4m3", b_nan_rows=gu_nan)
     out = ops.gemm_grouped_blockscaled(qh, d_codes, d_scales, offsets, N=d_codes.shape[1], out_dtype=out_dtype,
                                        b_nan_rows=d_nan)
     return (out, h) if want_h else out
@@ -394,8 +395,10 @@ def local_moe_forward(
     and down are as for expert_mlp()."""
     if routing is None:
         routing = route_by_expert(expert_ids, n_experts, capacity=capacity, topk_w=topk_w)
+    # e4m3 codes carry a NaN through the products themselves; only the int
+    # grid needs the rows' flags (and the launch that clears them)
     qx = ops.quant_tile_1x128_fanout(tokens, routing.pos, routing.top_k, routing.rows, fmt=fmt, bits=bits,
-                                     rounding=rounding, seed=seed, offset=offset, want_nan_rows=True)
+                                     rounding=rounding, seed=seed, offset=offset, want_nan_rows=fmt != "e4m3")
     y = expert_mlp(qx, routing.offsets, gate_up, down, fmt=fmt, bits=bits, rounding=rounding, seed=seed,
                    offset=offset, out_dtype=tokens.dtype)
     return combine_rows(y, routing, expert_ids, topk_w, tokens.shape[0])

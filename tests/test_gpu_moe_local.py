@@ -51,7 +51,7 @@ def _reference_combine(y_rows: torch.Tensor, pos: torch.Tensor, ids: torch.Tenso
 
 
 def test_route_by_expert_is_the_stable_sort(gpu_device):
-    from lowbit import moe
+    from lowbit import ep, moe
 
     ids = _routing(1000, 32, 8, 11, gpu_device)
     r = moe.route_by_expert(ids, 32)
@@ -197,3 +197,57 @@ def test_c4_fanout_and_combine_full_size(gpu_device):
     pos_sub = torch.arange(rows.numel(), dtype=torch.int32)
     ref = _reference_combine(y_sub, pos_sub, sub_ids, w.cpu()[tok], 32, torch.bfloat16)
     assert torch.equal(out.cpu()[tok].view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("n,buckets", [(1, 1), (63, 5), (64, 4096), (65, 32), (1023, 1025), (1024, 4096), (1025, 32)])
+def test_partition_in_one_workgroup_is_the_stable_sort(gpu_device, n, buckets):
+    """Up to 1024 keys take one workgroup; 1025 is the first size of the three passes."""
+    from lowbit import ep
+
+    keys = torch.randint(0, buckets, (n,), generator=torch.Generator().manual_seed(n)).to(torch.int32)
+    pos, inv, counts, offsets = ep.partition(keys.to(gpu_device), divisor=1, buckets=buckets)
+    order = torch.sort(keys, stable=True).indices
+    c = torch.bincount(keys, minlength=buckets)
+    assert torch.equal(inv.cpu().long(), order)
+    assert torch.equal(pos.cpu().long()[order], torch.arange(n))
+    assert torch.equal(counts.cpu(), c)
+    assert torch.equal(offsets.cpu().long(), torch.cat([torch.zeros(1, dtype=torch.int64), c.cumsum(0)]))
+
+
+@pytest.mark.parametrize("H", [8, 1000, 1024, 1032, 7168])
+@pytest.mark.parametrize("w_dtype", [torch.bfloat16, torch.float32])
+def test_combine_split_over_columns_equals_whole_rows(gpu_device, H, w_dtype):
+    """Few tokens split their rows over workgroups; 512 tokens do not. Same bits."""
+    from lowbit import moe
+
+    T, E, k = 512, 16, 4
+    ids = _routing(T, E, k, 5, gpu_device)
+    g = torch.Generator(device=gpu_device).manual_seed(6)
+    w = torch.rand(T, k, generator=g, device=gpu_device).to(w_dtype)
+    y = torch.randn(T * k, H, generator=g, device=gpu_device).to(torch.bfloat16)
+    r = moe.route_by_expert(ids, E)
+    whole = moe.combine_rows(y, r, ids, w, T)
+    for t in (1, 3, 200):
+        part = moe.ExpertRouting(r.pos[: t * k].contiguous(), r.inv, r.counts, r.offsets, k)
+        assert torch.equal(moe.combine_rows(y, part, ids[:t], w[:t], t), whole[:t])
+
+
+def test_e4m3_expert_loop_carries_a_nan_without_flags(gpu_device):
+    """The token with the NaN is NaN in every column, the others keep their bits."""
+    from lowbit import moe
+
+    T, H, I, E, k = 40, 256, 128, 4, 2
+    g = torch.Generator(device=gpu_device).manual_seed(8)
+    ids = _routing(T, E, k, 9, gpu_device)
+    tw = torch.full((T, k), 0.5, device=gpu_device, dtype=torch.bfloat16)
+    x = torch.randn(T, H, generator=g, device=gpu_device).to(torch.bfloat16)
+    w = [torch.randn(E, *s, generator=g, device=gpu_device).to(torch.bfloat16) * 0.05
+         for s in ((I, H), (I, H), (H, I))]
+    gu = moe.quantize_expert_weights(moe.stack_gate_up(w[0], w[1]), fmt="e4m3")
+    down = moe.quantize_expert_weights(w[2], fmt="e4m3")
+    clean = moe.local_moe_forward(x, ids, tw, gu, down, n_experts=E, fmt="e4m3")
+    x[7, 130] = float("nan")
+    got = moe.local_moe_forward(x, ids, tw, gu, down, n_experts=E, fmt="e4m3")
+    assert torch.isnan(got[7]).all()
+    keep = torch.arange(T, device=gpu_device) != 7
+    assert torch.equal(got[keep], clean[keep])
