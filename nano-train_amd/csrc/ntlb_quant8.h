@@ -104,8 +104,8 @@ __device__ __forceinline__ void codes_from_quotients(const float (&vq)[N], const
         // gives +0, so the sign comes from the comparison, not from v.
         // The reference clamps after rounding (:102-106): at the clamp,
         // qmax + u rounds to qmax + 1 in fp32 when u >= 1 - 2^-18
-        const float uu = sr_uniform(rb[i]);
-        const float w = __builtin_floorf(__builtin_fabsf(vq[i]) + uu);
+        // (one fma: u = (r >> 8) * 2^-24 is exact, so it rounds as the sum)
+        const float w = __builtin_floorf(__builtin_fmaf((float)(rb[i] >> 8), 0x1p-24f, __builtin_fabsf(vq[i])));
         t = vq[i] >= 0.0f ? w : -w;
         t = __builtin_amdgcn_fmed3f(t, -qmaxf, qmaxf);
       } else {
