@@ -163,9 +163,9 @@ def _reference_operand(t: torch.Tensor, dq: torch.Tensor, dtype: torch.dtype, sr
 
 
 class _LinearPlan:
-    """The shape of one linear call for ntlb_linear_forward and its backwards:
-    sizes and layouts, no pointers and no tensors, and constant once made (so
-    calls of any thread or stream share it)."""
+    """One linear call for ntlb_linear_forward and its backwards: sizes, layouts
+    and the quantizers' settings, no pointers and no tensors, and constant once
+    made (so calls of any thread or stream share it)."""
 
     __slots__ = ("c", "ref", "M", "N", "K", "code_bytes", "ws_bytes")
 
@@ -257,7 +257,7 @@ class _HipLowBitLinear(torch.autograd.Function):
         ctx.plan = None
         if backend._one_call(x, weight, bias, needs):
             x2 = _rows_2d(x, K)
-            plan = backend._plan(x2, weight, bias)
+            plan = backend._plan(x2, weight, None if bias is None else bias.dtype)
             base = backend._next_offset()
             dev = x.device
             buf = torch.empty(plan.code_bytes, dtype=torch.uint8, device=dev)
@@ -390,8 +390,9 @@ class _HipLowBitLinear(torch.autograd.Function):
                     dw = ops.gemm_dense_tn(dy2.to(op), xdq.to(op), out_dtype=ctx.w_dtype)
             else:
                 x2, weight = ctx.saved_tensors
-                if (dy2.dtype == ctx.x_dtype == ctx.w_dtype and dy2.dtype in _RECIPE_DTYPES
-                        and x2.stride(0) == plan.c.ldx and weight.stride(0) == plan.c.ldw):
+                if dy2.dtype == ctx.x_dtype == ctx.w_dtype and dy2.dtype in _RECIPE_DTYPES:
+                    # quantizes anew: the settings of now, the pitches of the saved tensors
+                    plan = backend._plan(x2, weight, ctx.bias_dtype)
                     return (*_recipe_backward(plan, dy2, x2, weight, needs, ctx.x_shape, ctx.bias_dtype, ctx.offset),
                             None)
                 dx, dw = _fp8_recipe_backward(backend, dy2, x2, weight, ctx.offset, needs)
@@ -536,13 +537,15 @@ class HipLowBitBackend:
                     and self._rounding_mode != "stochastic")
         return True
 
-    def _plan(self, x2, weight, bias) -> _LinearPlan:
-        key = (x2.shape[0], weight.shape, x2.stride(0), weight.stride(0), x2.dtype, weight.dtype,
-               None if bias is None else bias.dtype)
+    def _plan(self, x2, weight, bias_dtype) -> _LinearPlan:
+        """The plan of a call, kept for the next one of the same sizes, pitches,
+        dtypes, device and settings (attributes that may change between calls)."""
+        key = (x2.shape[0], weight.shape, x2.stride(0), weight.stride(0), x2.dtype, weight.dtype, bias_dtype,
+               x2.get_device(), self.seed, self.code_format, self.bits, self._rounding_mode)
         plan = self._plans.get(key)
         if plan is None:
             plan = _LinearPlan(x2.shape[0], weight.shape[0], weight.shape[1], x2.stride(0), weight.stride(0), x2.dtype,
-                               weight.dtype, key[-1], ops.grid_code(self.code_format), (1 << (self.bits - 1)) - 1,
+                               weight.dtype, bias_dtype, ops.grid_code(self.code_format), (1 << (self.bits - 1)) - 1,
                                ops.rounding_code(self._rounding_mode), self.seed)
             if len(self._plans) >= _MAX_PLANS:  # ragged batches: keep it bounded
                 self._plans.clear()

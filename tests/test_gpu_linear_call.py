@@ -178,3 +178,37 @@ def test_colsum_of_few_columns_or_rows(gpu_device, shape, dtype):
         got = ops.colsum(t, out_dtype=torch.float32).double()
         ref = x.double().sum(0)
         assert float(((got - ref).abs() / x.double().abs().sum(0)).max()) <= M * 2.0 ** -24
+
+
+@pytest.mark.parametrize("recipe", ["ste", "fp8"])
+@pytest.mark.parametrize("attr,value", [("seed", 78), ("code_format", "e4m3"), ("bits", 4), ("_rounding_mode", "nearest")])
+def test_backend_attributes_are_read_at_every_call(gpu_device, attr, value, recipe):
+    """seed, code format, bits and rounding changed between two calls of one
+    shape: the later call's outputs and gradients are those of the general path
+    after the same change (the straight-through rule draws only in its forward)"""
+    M, N, K = 40, 192, 300
+    x = seeded((M, K), seed=20262161).to(gpu_device)
+    w = seeded((N, K), seed=20262162, std=0.02).to(gpu_device)
+    dy = seeded((M, N), seed=20262163, std=1e-3).to(gpu_device)
+    grads = recipe == "fp8"
+    out = []
+    for general in (False, True):
+        be = _backend("int_grid", "stochastic", recipe, K, N)
+        if general:
+            be._one_call = lambda *a: False
+        before = getattr(be, attr)
+        for change in (False, True):
+            if change:
+                setattr(be, attr, value)
+            t = [v.clone().requires_grad_(grads) for v in (x, w)]
+            y = be.linear(*t, None)
+            out.append([y, *(torch.autograd.grad(y, t, dy) if grads else ())])
+        if grads:  # changed back between a forward and its backward, which quantizes dY, W and X anew
+            t = [v.clone().requires_grad_(True) for v in (x, w)]
+            y = be.linear(*t, None)
+            setattr(be, attr, before)
+            out.append([y, *torch.autograd.grad(y, t, dy)])
+    half = len(out) // 2
+    assert not _same(out[0][0], out[1][0]), "the change should show in the output"
+    for one, gen in zip(out[:half], out[half:]):
+        assert all(_same(p, q) for p, q in zip(one, gen))
