@@ -208,7 +208,10 @@ def _rows_2d(t: torch.Tensor, cols: int) -> torch.Tensor:
     """t as [rows, cols] with unit column stride and a row pitch of at least cols"""
     t2 = t if t.dim() == 2 else t.reshape(-1, cols)
     s = t2.stride()
-    return t2 if s[1] == 1 and s[0] >= cols else t2.contiguous()
+    if s[1] == 1 and s[0] >= cols:
+        return t2
+    # one row may have any pitch and still count as contiguous (a transposed column: strides (1, 1))
+    return t2.contiguous().view(-1).view(-1, cols)
 
 
 def _workspace(need: int, device):

@@ -212,3 +212,24 @@ def test_backend_attributes_are_read_at_every_call(gpu_device, attr, value, reci
     assert not _same(out[0][0], out[1][0]), "the change should show in the output"
     for one, gen in zip(out[:half], out[half:]):
         assert all(_same(p, q) for p, q in zip(one, gen))
+
+
+@pytest.mark.parametrize("recipe", ["ste", "fp8"])
+def test_one_row_with_a_short_pitch(gpu_device, recipe):
+    """One token: a [1, N] gradient and a [1, K] input that are transposes of
+    columns have strides (1, 1), which torch counts as contiguous"""
+    N, K = 192, 256
+    x = seeded((1, K), seed=20262171).to(gpu_device)
+    w = seeded((N, K), seed=20262172, std=0.02).to(gpu_device)
+    b = seeded((N,), seed=20262173).to(gpu_device)
+    dy = seeded((1, N), seed=20262174, std=1e-3).to(gpu_device)
+    up = dy.reshape(N, 1).clone().t()
+    assert up.stride() == (1, 1)
+    one, gen = _both("e4m3", "nearest", recipe, x, w, b, up, general_dy=dy)
+    assert _agree(recipe, one, gen)
+    xt = x.reshape(K, 1).clone().t()
+    assert xt.stride() == (1, 1)
+    be = _backend("e4m3", "nearest", recipe, K, N)
+    t = [xt.requires_grad_(True), w.clone().requires_grad_(True), b.clone().requires_grad_(True)]
+    y = be.linear(*t)
+    assert _agree(recipe, [y, *torch.autograd.grad(y, t, dy)], gen)
