@@ -214,6 +214,21 @@ def _rows_2d(t: torch.Tensor, cols: int) -> torch.Tensor:
     return t2.contiguous().view(-1).view(-1, cols)
 
 
+def _saved_operand(t: torch.Tensor, cols: int) -> torch.Tensor:
+    """A matrix kept for the backward, as its saved-tensor hooks give it back:
+    the kernels get its address, so its place and layout are looked at here"""
+    ops._require_device(t)
+    return _rows_2d(t, cols)
+
+
+def _saved_codes(buf: torch.Tensor, nbytes: int) -> torch.Tensor:
+    """A forward's code buffer kept for the backward, checked as _saved_operand"""
+    ops._require_device(buf)
+    if buf.dtype != torch.uint8 or buf.numel() != nbytes:
+        raise RuntimeError(f"the saved codes came back as {buf.dtype}[{buf.numel()}], not uint8[{nbytes}]")
+    return buf.contiguous()
+
+
 def _workspace(need: int, device):
     ws = ops.split_workspace(need, device)
     return (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
@@ -377,6 +392,7 @@ class _HipLowBitLinear(torch.autograd.Function):
             dy2 = _rows_2d(dy, plan.N)
             if backend.backward_recipe == "ste":
                 (buf,) = ctx.saved_tensors
+                buf = _saved_codes(buf, plan.code_bytes)
                 if dy2.dtype == torch.bfloat16 and ctx.x_dtype == torch.bfloat16 and ctx.w_dtype == torch.bfloat16:
                     return (*_ste_backward(plan, dy2, buf, needs, ctx.x_shape, ctx.bias_dtype), None)
                 # another gradient dtype: the dequantized operands on the fp32 GEMM
@@ -392,8 +408,9 @@ class _HipLowBitLinear(torch.autograd.Function):
                     op = _gemm_op_dtype(dy2.dtype, xdq.dtype)
                     dw = ops.gemm_dense_tn(dy2.to(op), xdq.to(op), out_dtype=ctx.w_dtype)
             else:
-                x2, weight = ctx.saved_tensors
-                if dy2.dtype == ctx.x_dtype == ctx.w_dtype and dy2.dtype in _RECIPE_DTYPES:
+                x2, weight = (_saved_operand(t, plan.K) for t in ctx.saved_tensors)
+                if (dy2.dtype == x2.dtype == weight.dtype == ctx.x_dtype == ctx.w_dtype
+                        and dy2.dtype in _RECIPE_DTYPES):
                     # quantizes anew: the settings of now, the pitches of the saved tensors
                     plan = backend._plan(x2, weight, ctx.bias_dtype)
                     return (*_recipe_backward(plan, dy2, x2, weight, needs, ctx.x_shape, ctx.bias_dtype, ctx.offset),

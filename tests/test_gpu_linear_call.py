@@ -233,3 +233,31 @@ def test_one_row_with_a_short_pitch(gpu_device, recipe):
     t = [xt.requires_grad_(True), w.clone().requires_grad_(True), b.clone().requires_grad_(True)]
     y = be.linear(*t)
     assert _agree(recipe, [y, *torch.autograd.grad(y, t, dy)], gen)
+
+
+@pytest.mark.parametrize("recipe", ["ste", "fp8"])
+def test_saved_tensor_hooks(gpu_device, recipe):
+    """what was kept for the backward may go through host memory, or come back
+    in another layout; left in host memory, or cut short, it is an error
+    before any launch"""
+    M, N, K = 40, 192, 320
+    x = seeded((M, K), seed=20262191).to(gpu_device)
+    w = seeded((N, K), seed=20262192, std=0.02).to(gpu_device)
+    dy = seeded((M, N), seed=20262193, std=1e-3).to(gpu_device)
+
+    def grads(pack, unpack):
+        be = _backend("e4m3", "nearest", recipe, K, N)
+        t = [v.clone().requires_grad_(True) for v in (x, w)]
+        with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+            y = be.linear(*t, None)
+        return torch.autograd.grad(y, t, dy)
+
+    plain = grads(lambda s: s, lambda s: s)
+    layouts = [lambda s: s.cpu(), lambda s: s.t().contiguous().t() if s.dim() == 2 else s.clone()]
+    for pack in layouts:
+        assert all(_same(p, q) for p, q in zip(plain, grads(pack, lambda s: s.to(gpu_device))))
+    with pytest.raises(RuntimeError, match="ROCm device"):
+        grads(lambda s: s.cpu(), lambda s: s)
+    if recipe == "ste":
+        with pytest.raises(RuntimeError, match="saved codes"):
+            grads(lambda s: s, lambda s: s[:-256])
