@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define NTLB_ABI_VERSION 1
+#define NTLB_ABI_VERSION 2
 
 #define NTLB_OK 0
 #define NTLB_EINVAL (-1)       /* bad shape, stride, alignment or enum */
@@ -525,34 +525,37 @@ int ntlb_gemm_bf16_tn(const void* a, int64_t lda, const void* b, int64_t ldb, in
  * fp32 q * s values, its straight-through backward, and the backward with
  * quantized gradients.  The caller fills the shape fields of a plan (x [M, K]
  * with row pitch ldx, weight [N, K] with ldw, element dtypes; y has x's dtype)
- * and ntlb_linear_plan_init the sizes: code_bytes of the code buffer that the
- * forward writes and the straight-through backward reads, scratch bytes of
- * each backward, and the bytes of the zeroed split-K workspace each call can
- * use (as ntlb_gemm_blockscaled_ws; 0 or NULL: none).  A plan holds no
- * pointers and is not written after its init, so threads and streams may
- * share it.  Buffers are 256-byte aligned; y, dx and dw are contiguous.
+ * and ntlb_linear_plan_init the sizes: the bytes of X's and of W's code buffer,
+ * which the forward writes and the straight-through backward reads (X's for
+ * dw, W's for dx: each can be freed where its gradient is not wanted, and both
+ * may be parts of one allocation), the scratch bytes of each backward, and the
+ * bytes of the zeroed split-K workspace each call can use (as
+ * ntlb_gemm_blockscaled_ws; 0 or NULL: none).  A plan holds no pointers and is
+ * not written after its init, so threads and streams may share it.  Buffers
+ * are 256-byte aligned; y, dx and dw are contiguous.
  */
 typedef struct ntlb_linear_plan {
   int64_t M, N, K, ldx, ldw;
   int x_dtype, w_dtype, bias_dtype, grid, qmax, rounding;
   uint64_t seed;
-  int64_t code_bytes, ste_bytes, ste_pad_bytes, recipe_bytes, forward_ws, ste_ws, recipe_ws;
+  int64_t x_code_bytes, w_code_bytes, ste_bytes, ste_pad_bytes, recipe_bytes, forward_ws, ste_ws, recipe_ws;
 } ntlb_linear_plan;
 
 int ntlb_linear_plan_init(ntlb_linear_plan* plan);
 
 /* Forward; the activation draws at Philox offset `offset`, the weight at
  * offset + 1.  bias optional [N]. */
-int ntlb_linear_forward(const ntlb_linear_plan* plan, const void* x, const void* w, const void* bias, void* codes,
-                        void* y, void* workspace, int64_t ws_bytes, uint64_t offset, void* stream);
+int ntlb_linear_forward(const ntlb_linear_plan* plan, const void* x, const void* w, const void* bias, void* x_codes,
+                        void* w_codes, void* y, void* workspace, int64_t ws_bytes, uint64_t offset, void* stream);
 
-/* Straight-through backward of bf16 layers from the forward's code buffer:
- * dx = dY . bf16(W_dq), dw = dY^T . bf16(X_dq), db = the column sum of dY;
- * each output optional.  scratch: ste_bytes, or ste_pad_bytes where dY needs a
- * padded copy (N % 64 != 0, lddy % 8 != 0 or dY not 16-byte aligned). */
-int ntlb_linear_ste_backward(const ntlb_linear_plan* plan, const void* dy, int64_t lddy, const void* codes, void* dx,
-                             void* dw, void* db, int db_dtype, void* scratch, int64_t scratch_bytes, void* workspace,
-                             int64_t ws_bytes, void* stream);
+/* Straight-through backward of bf16 layers from the forward's code buffers
+ * (w_codes can be NULL where dx is, x_codes where dw is): dx = dY . bf16(W_dq),
+ * dw = dY^T . bf16(X_dq), db = the column sum of dY; each output optional.
+ * scratch: ste_bytes, or ste_pad_bytes where dY needs a padded copy (N % 64 !=
+ * 0, lddy % 8 != 0 or dY not 16-byte aligned). */
+int ntlb_linear_ste_backward(const ntlb_linear_plan* plan, const void* dy, int64_t lddy, const void* x_codes,
+                             const void* w_codes, void* dx, void* dw, void* db, int db_dtype, void* scratch,
+                             int64_t scratch_bytes, void* workspace, int64_t ws_bytes, void* stream);
 
 /* Backward with quantized gradients (dY per 1x128 and 128x1 tile at Philox
  * offset + 2, W at offset + 1, X at offset + 4); dY, dx and dw in x's dtype,

@@ -1,6 +1,6 @@
 // One low-bit Linear call per entry point: the launches of a forward, of its
 // straight-through backward and of the quantized-gradient backward, issued
-// from one host call over one code buffer and one scratch buffer
+// from one host call over the codes of X and of W and one scratch buffer
 // (te_backend.py:229-260 and its autograd; the recipe of benchmark config 3).
 // The device work is that of the separate entry points; what this file adds
 // on the device is the zeroing of the NaN row flags (int grid only, one
@@ -21,9 +21,13 @@
 
 namespace ntlb {
 
-__global__ void __launch_bounds__(256) zero_words_kernel(uint32_t* p, int64_t n) {
+// p [n] and p2 [n2] cleared
+__global__ void __launch_bounds__(256) zero_words_kernel(uint32_t* p, int64_t n, uint32_t* p2, int64_t n2) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) p[i] = 0u;
+  if (i < n)
+    p[i] = 0u;
+  else if (i < n + n2)
+    p2[i - n] = 0u;
 }
 
 // dst [M, ldd] (ldd % 8 == 0, 16-byte aligned) = src [M, N] of 16-bit values,
@@ -107,20 +111,29 @@ struct Carve {
   }
 };
 
-// the code buffer: X codes and scales, W codes and scales, NaN flags of X's
-// then W's rows (int grid)
+// the code buffers of X and of W, apart so that each can be kept as long as
+// its gradient needs it: codes, scales, and the NaN flags of the rows (int
+// grid; -1: none)
 struct CodeLayout {
-  int64_t xc, xs, wc, ws, flags, bytes;
+  int64_t c, s, flags, bytes;
 };
-static CodeLayout code_layout(const ntlb_linear_plan& p) {
-  const int64_t kp = up(p.K, 128), T = kp / 128;
+static CodeLayout x_layout(const ntlb_linear_plan& p) {
+  const int64_t kp = up(p.K, 128);
   Carve c;
   CodeLayout l;
-  l.xc = c.take(p.M * kp);
-  l.xs = c.take(T * up(p.M, 4) * 4);
-  l.wc = c.take(p.N * kp);
-  l.ws = c.take(cdiv(p.N, 128) * T * 4);
-  l.flags = p.grid == NTLB_GRID_INT ? c.take((p.M + p.N) * 4) : -1;
+  l.c = c.take(p.M * kp);
+  l.s = c.take(kp / 128 * up(p.M, 4) * 4);
+  l.flags = p.grid == NTLB_GRID_INT ? c.take(p.M * 4) : -1;
+  l.bytes = c.at;
+  return l;
+}
+static CodeLayout w_layout(const ntlb_linear_plan& p) {
+  const int64_t kp = up(p.K, 128);
+  Carve c;
+  CodeLayout l;
+  l.c = c.take(p.N * kp);
+  l.s = c.take(cdiv(p.N, 128) * (kp / 128) * 4);
+  l.flags = p.grid == NTLB_GRID_INT ? c.take(p.N * 4) : -1;
   l.bytes = c.at;
   return l;
 }
@@ -179,8 +192,9 @@ static int check_plan(const char* fn, const ntlb_linear_plan* p) {
   return NTLB_OK;
 }
 
-static void zero_words(void* p, int64_t n, hipStream_t st) {
-  zero_words_kernel<<<(unsigned)cdiv(n, 256), 256, 0, st>>>(reinterpret_cast<uint32_t*>(p), n);
+static void zero_words(int32_t* p, int64_t n, int32_t* p2, int64_t n2, hipStream_t st) {
+  zero_words_kernel<<<(unsigned)cdiv(n + n2, 256), 256, 0, st>>>(reinterpret_cast<uint32_t*>(p), n,
+                                                                 reinterpret_cast<uint32_t*>(p2), n2);
 }
 
 }  // namespace ntlb
@@ -191,7 +205,8 @@ extern "C" int ntlb_linear_plan_init(ntlb_linear_plan* p) {
   const char* fn = "ntlb_linear_plan_init";
   if (int rc = check_plan(fn, p)) return rc;
   const int64_t kp = up(p->K, 128), np = up(p->N, 128), mp = up(p->M, 128);
-  p->code_bytes = code_layout(*p).bytes;
+  p->x_code_bytes = x_layout(*p).bytes;
+  p->w_code_bytes = w_layout(*p).bytes;
   p->ste_bytes = ste_layout(*p).dy;
   p->ste_pad_bytes = ste_layout(*p).bytes;
   p->recipe_bytes = recipe_layout(*p).bytes;
@@ -202,43 +217,48 @@ extern "C" int ntlb_linear_plan_init(ntlb_linear_plan* p) {
 }
 
 extern "C" int ntlb_linear_forward(const ntlb_linear_plan* p, const void* x, const void* w, const void* bias,
-                                   void* codes, void* y, void* workspace, int64_t ws_bytes, uint64_t offset,
-                                   void* stream) {
+                                   void* x_codes, void* w_codes, void* y, void* workspace, int64_t ws_bytes,
+                                   uint64_t offset, void* stream) {
   const char* fn = "ntlb_linear_forward";
   if (int rc = check_plan(fn, p)) return rc;
-  if (!x || !w || !codes || !y) return fail(NTLB_EINVAL, "%s: NULL pointer", fn);
-  if (!aligned(codes, 256)) return fail(NTLB_EINVAL, "%s: the code buffer must be 256-byte aligned", fn);
-  const CodeLayout l = code_layout(*p);
-  uint8_t* b = reinterpret_cast<uint8_t*>(codes);
+  if (!x || !w || !x_codes || !w_codes || !y) return fail(NTLB_EINVAL, "%s: NULL pointer", fn);
+  if (!aligned(x_codes, 256) || !aligned(w_codes, 256))
+    return fail(NTLB_EINVAL, "%s: the code buffers must be 256-byte aligned", fn);
+  const CodeLayout lx = x_layout(*p), lw = w_layout(*p);
+  uint8_t* xb = reinterpret_cast<uint8_t*>(x_codes);
+  uint8_t* wb = reinterpret_cast<uint8_t*>(w_codes);
+  float* xs = reinterpret_cast<float*>(xb + lx.s);
+  float* ws = reinterpret_cast<float*>(wb + lw.s);
   const int64_t kp = up(p->K, 128), T = kp / 128, m4 = up(p->M, 4);
-  int32_t* nan_x = l.flags >= 0 ? reinterpret_cast<int32_t*>(b + l.flags) : nullptr;
-  int32_t* nan_w = nan_x ? nan_x + p->M : nullptr;
-  if (nan_x) zero_words(nan_x, p->M + p->N, as_stream(stream));
+  int32_t* nan_x = lx.flags >= 0 ? reinterpret_cast<int32_t*>(xb + lx.flags) : nullptr;
+  int32_t* nan_w = lw.flags >= 0 ? reinterpret_cast<int32_t*>(wb + lw.flags) : nullptr;
+  if (nan_x) zero_words(nan_x, p->M, nan_w, p->N, as_stream(stream));
   int rc = ntlb_quant_tile_1x128(x, p->x_dtype, p->M, p->K, p->ldx, p->grid, p->qmax, p->rounding,
-                                 NTLB_SCALE_AFTER_DIVIDE, p->seed, offset, b + l.xc, kp,
-                                 reinterpret_cast<float*>(b + l.xs), 1, m4, nullptr, 0, 0, nan_x, stream);
+                                 NTLB_SCALE_AFTER_DIVIDE, p->seed, offset, xb + lx.c, kp, xs, 1, m4, nullptr, 0, 0,
+                                 nan_x, stream);
   if (rc) return rc;
   rc = ntlb_quant_block_128x128(w, p->w_dtype, p->N, p->K, p->ldw, p->grid, p->qmax, p->rounding,
-                                NTLB_SCALE_AFTER_DIVIDE, p->seed, offset + 1, b + l.wc, kp, nullptr, 0,
-                                reinterpret_cast<float*>(b + l.ws), T, 1, nullptr, 0, 0, nan_w, stream);
+                                NTLB_SCALE_AFTER_DIVIDE, p->seed, offset + 1, wb + lw.c, kp, nullptr, 0, ws, T, 1,
+                                nullptr, 0, 0, nan_w, stream);
   if (rc) return rc;
-  return ntlb_gemm_blockscaled_ws(p->grid, b + l.xc, kp, reinterpret_cast<const float*>(b + l.xs), 1, m4, 0,
-                                  b + l.wc, kp, reinterpret_cast<const float*>(b + l.ws), T, 1, 7, p->M, p->N, kp,
+  return ntlb_gemm_blockscaled_ws(p->grid, xb + lx.c, kp, xs, 1, m4, 0, wb + lw.c, kp, ws, T, 1, 7, p->M, p->N, kp,
                                   bias, p->bias_dtype, y, p->x_dtype, p->N, nan_x, nan_w, workspace, ws_bytes,
                                   stream);
 }
 
-extern "C" int ntlb_linear_ste_backward(const ntlb_linear_plan* p, const void* dy, int64_t lddy, const void* codes,
-                                        void* dx, void* dw, void* db, int db_dtype, void* scratch,
-                                        int64_t scratch_bytes, void* workspace, int64_t ws_bytes, void* stream) {
+extern "C" int ntlb_linear_ste_backward(const ntlb_linear_plan* p, const void* dy, int64_t lddy, const void* x_codes,
+                                        const void* w_codes, void* dx, void* dw, void* db, int db_dtype,
+                                        void* scratch, int64_t scratch_bytes, void* workspace, int64_t ws_bytes,
+                                        void* stream) {
   const char* fn = "ntlb_linear_ste_backward";
   if (int rc = check_plan(fn, p)) return rc;
-  if (!dy || !scratch || ((dx || dw) && !codes)) return fail(NTLB_EINVAL, "%s: NULL pointer", fn);
+  if (!dy || !scratch || (dx && !w_codes) || (dw && !x_codes)) return fail(NTLB_EINVAL, "%s: NULL pointer", fn);
   if (p->x_dtype != NTLB_BF16 || p->w_dtype != NTLB_BF16) return fail(NTLB_EUNSUPPORTED, "%s: bf16 only", fn);
   if (lddy < p->N) return fail(NTLB_EINVAL, "%s: lddy < N", fn);
-  const CodeLayout l = code_layout(*p);
+  const CodeLayout lx = x_layout(*p), lw = w_layout(*p);
   const SteLayout sl = ste_layout(*p);
-  const uint8_t* b = reinterpret_cast<const uint8_t*>(codes);
+  const uint8_t* xb = reinterpret_cast<const uint8_t*>(x_codes);
+  const uint8_t* wb = reinterpret_cast<const uint8_t*>(w_codes);
   uint8_t* s = reinterpret_cast<uint8_t*>(scratch);
   const int64_t kp = up(p->K, 128), T = kp / 128, m4 = up(p->M, 4), n64 = up(p->N, 64);
   const bool pad_dy = p->N % 64 || lddy % 8 || !aligned(dy, 16);
@@ -260,10 +280,16 @@ extern "C" int ntlb_linear_ste_backward(const ntlb_linear_plan* p, const void* d
   const bool small_dx = dx && sl.wd >= 0 && near_rows, small_dw = dw && sl.xd >= 0 && near_rows;
   if (small_dx || small_dw) {
     DecodeArgs d{};
-    d.wc = b + l.wc; d.ws = reinterpret_cast<const float*>(b + l.ws);
-    d.xc = b + l.xc; d.xs = reinterpret_cast<const float*>(b + l.xs);
-    d.wrows = small_dx ? p->N : 0;
-    d.xrows = small_dw ? p->M : 0;
+    if (small_dx) {
+      d.wc = wb + lw.c;
+      d.ws = reinterpret_cast<const float*>(wb + lw.s);
+      d.wrows = p->N;
+    }
+    if (small_dw) {
+      d.xc = xb + lx.c;
+      d.xs = reinterpret_cast<const float*>(xb + lx.s);
+      d.xrows = p->M;
+    }
     d.kp = kp; d.T = T; d.m4 = m4; d.ld = up(p->K, 8);
     d.wd = reinterpret_cast<uint16_t*>(s + std::max<int64_t>(sl.wd, 0));
     d.xd = reinterpret_cast<uint16_t*>(s + std::max<int64_t>(sl.xd, 0));
@@ -298,14 +324,14 @@ extern "C" int ntlb_linear_ste_backward(const ntlb_linear_plan* p, const void* d
     if (int rc = check_launch(fn)) return rc;
   }
   if (dx && !small_dx) {
-    const int rc = ntlb_gemm_ste_dgrad_ws(NTLB_BF16, dy, lddy, p->M, p->N, p->grid, b + l.wc, kp,
-                                          reinterpret_cast<const float*>(b + l.ws), T, 1, 7, p->K, dx, NTLB_BF16,
+    const int rc = ntlb_gemm_ste_dgrad_ws(NTLB_BF16, dy, lddy, p->M, p->N, p->grid, wb + lw.c, kp,
+                                          reinterpret_cast<const float*>(wb + lw.s), T, 1, 7, p->K, dx, NTLB_BF16,
                                           p->K, workspace, ws_bytes, stream);
     if (rc) return rc;
   }
   if (dw && !small_dw) {
-    const int rc = ntlb_gemm_ste_wgrad(NTLB_BF16, dy, lddy, p->M, p->N, p->grid, b + l.xc, kp,
-                                       reinterpret_cast<const float*>(b + l.xs), 1, m4, 0, p->K, dw, NTLB_BF16,
+    const int rc = ntlb_gemm_ste_wgrad(NTLB_BF16, dy, lddy, p->M, p->N, p->grid, xb + lx.c, kp,
+                                       reinterpret_cast<const float*>(xb + lx.s), 1, m4, 0, p->K, dw, NTLB_BF16,
                                        p->K, stream);
     if (rc) return rc;
   }
@@ -338,7 +364,7 @@ extern "C" int ntlb_linear_recipe_backward(const ntlb_linear_plan* p, const void
   float* wsc = reinterpret_cast<float*>(b + l.ws);
   float* xts = reinterpret_cast<float*>(b + l.xts);
   int rc = NTLB_OK;
-  if (nan_m && (dx || dw)) zero_words(nan_m, p->M + p->N + p->K, as_stream(stream));
+  if (nan_m && (dx || dw)) zero_words(nan_m, p->M + p->N + p->K, nullptr, 0, as_stream(stream));
   // dY's 1x128 and 128x1 quantizations share one Philox offset: one pass over
   // dY writes both where its rows allow
   const bool dual = dx && dw && p->N % 8 == 0 && lddy % 8 == 0 && aligned(dy, 16) && dt != NTLB_F16;

@@ -14,7 +14,7 @@ import threading
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # NTLB_LIB_PATH points at another build of the same ABI (a tuned or debug build)
 LIB_PATH = os.environ.get("NTLB_LIB_PATH") or os.path.join(_HERE, "libntlowbit.so")
-ABI_VERSION = 1
+ABI_VERSION = 2
 
 NTLB_OK = 0
 NTLB_EINVAL = -1
@@ -63,8 +63,8 @@ SIGNATURES = {
                                        _I32, _I32, _I32, _U64, _U64, _P],
     "ntlb_gemm_bf16_tn": [_P, _I64, _P, _I64, _I64, _I64, _I64, _P, _I32, _I64, _P],
     "ntlb_linear_plan_init": [_P],
-    "ntlb_linear_forward": [_P, _P, _P, _P, _P, _P, _P, _I64, _U64, _P],
-    "ntlb_linear_ste_backward": [_P, _P, _I64, _P, _P, _P, _P, _I32, _P, _I64, _P, _I64, _P],
+    "ntlb_linear_forward": [_P, _P, _P, _P, _P, _P, _P, _P, _I64, _U64, _P],
+    "ntlb_linear_ste_backward": [_P, _P, _I64, _P, _P, _P, _P, _P, _I32, _P, _I64, _P, _I64, _P],
     "ntlb_linear_recipe_backward": [_P, _P, _I64, _P, _P, _P, _P, _P, _I32, _P, _I64, _P, _I64, _U64, _P],
     "ntlb_persistent_quant_ws_words": [_P, _I64, _I64],
     "ntlb_nf4_quant": [_P, _I32, _I64, _I64, _P, _P, _P, _P],
@@ -146,8 +146,9 @@ class LinearPlan(ctypes.Structure):
 
     _fields_ = [("M", _I64), ("N", _I64), ("K", _I64), ("ldx", _I64), ("ldw", _I64),
                 ("x_dtype", _I32), ("w_dtype", _I32), ("bias_dtype", _I32), ("grid", _I32), ("qmax", _I32),
-                ("rounding", _I32), ("seed", _U64), ("code_bytes", _I64), ("ste_bytes", _I64), ("ste_pad_bytes", _I64),
-                ("recipe_bytes", _I64), ("forward_ws", _I64), ("ste_ws", _I64), ("recipe_ws", _I64)]
+                ("rounding", _I32), ("seed", _U64), ("x_code_bytes", _I64), ("w_code_bytes", _I64), ("ste_bytes", _I64),
+                ("ste_pad_bytes", _I64), ("recipe_bytes", _I64), ("forward_ws", _I64), ("ste_ws", _I64),
+                ("recipe_ws", _I64)]
 
 
 # entry points that return a value instead of a status

@@ -167,7 +167,7 @@ class _LinearPlan:
     and the quantizers' settings, no pointers and no tensors, and constant once
     made (so calls of any thread or stream share it)."""
 
-    __slots__ = ("c", "ref", "M", "N", "K", "code_bytes", "ws_bytes")
+    __slots__ = ("c", "ref", "M", "N", "K", "x_bytes", "w_bytes", "ws_bytes")
 
     def __init__(self, M, N, K, ldx, ldw, xdt, wdt, bdt, grid, qmax, rounding, seed) -> None:
         self.c = _lib.LinearPlan(M=M, N=N, K=K, ldx=ldx, ldw=ldw, x_dtype=ops._dtype_code(xdt),
@@ -176,28 +176,26 @@ class _LinearPlan:
         self.ref = ctypes.addressof(self.c)
         self.M, self.N, self.K = M, N, K
         _lib.call("ntlb_linear_plan_init", self.ref)
-        self.code_bytes = self.c.code_bytes
+        self.x_bytes, self.w_bytes = self.c.x_code_bytes, self.c.w_code_bytes
         self.ws_bytes = self.c.forward_ws
 
-    def qtensors(self, buf: torch.Tensor):
-        """The code buffer's activation and weight as QTensors (views)."""
-        M, N, K, grid = self.M, self.N, self.K, self.c.grid
-        T, m4 = ops.cdiv(K, 128), ops.cdiv(M, 4) * 4
-        at = 0
+    def x_tensor(self, buf: torch.Tensor) -> QTensor:
+        """The activation's code buffer as a QTensor of views."""
+        M, K, T, m4 = self.M, self.K, ops.cdiv(self.K, 128), ops.cdiv(self.M, 4) * 4
+        codes, scales = _codes_and_scales(buf, M, T, T * m4)
+        return QTensor(codes, scales.view(T, m4), 1, m4, 0, self.c.grid, M, K, None, None)
 
-        def piece(nbytes):
-            nonlocal at
-            v = buf[at:at + nbytes]
-            at += ops.cdiv(nbytes, 256) * 256
-            return v
+    def w_tensor(self, buf: torch.Tensor) -> QTensor:
+        """The weight's code buffer as a QTensor of views."""
+        N, K, T = self.N, self.K, ops.cdiv(self.K, 128)
+        codes, scales = _codes_and_scales(buf, N, T, ops.cdiv(N, 128) * T)
+        return QTensor(codes, scales.view(-1, T), T, 1, 7, self.c.grid, N, K, None, None)
 
-        xc = piece(M * T * 128).view(M, T * 128)
-        xs = piece(T * m4 * 4).view(torch.float32).view(T, m4)
-        wc = piece(N * T * 128).view(N, T * 128)
-        ws = piece(ops.cdiv(N, 128) * T * 4).view(torch.float32).view(-1, T)
-        flags = piece((M + N) * 4).view(torch.int32) if grid == _lib.GRID_INT else None
-        nx, nw = (None, None) if flags is None else (flags[:M], flags[M:])
-        return (QTensor(xc, xs, 1, m4, 0, grid, M, K, nx, None), QTensor(wc, ws, T, 1, 7, grid, N, K, nw, None))
+
+def _codes_and_scales(buf: torch.Tensor, rows: int, blocks: int, n_scales: int):
+    """codes [rows, 128 * blocks] at the start of buf, the scales at the next 256 bytes"""
+    at = ops.cdiv(rows * blocks, 2) * 256
+    return (buf[:rows * blocks * 128].view(rows, blocks * 128), buf[at:at + 4 * n_scales].view(torch.float32))
 
 
 _MAX_PLANS = 64
@@ -234,8 +232,9 @@ def _workspace(need: int, device):
     return (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
 
 
-def _ste_backward(plan: _LinearPlan, dy2, buf, needs, x_shape, bias_dtype):
-    """dX, dW, db of the straight-through rule from the forward's code buffer (bf16)"""
+def _ste_backward(plan: _LinearPlan, dy2, xp, wp, needs, x_shape, bias_dtype):
+    """dX, dW, db of the straight-through rule from the forward's code buffers
+    at xp and wp (bf16)"""
     dev, bf = dy2.device, torch.bfloat16
     dx = torch.empty(x_shape, dtype=bf, device=dev) if needs[0] else None
     dw = torch.empty((plan.N, plan.K), dtype=bf, device=dev) if needs[1] else None
@@ -244,9 +243,9 @@ def _ste_backward(plan: _LinearPlan, dy2, buf, needs, x_shape, bias_dtype):
     padded = plan.N % 64 != 0 or ld % 8 != 0 or ptr % 16 != 0
     scratch = torch.empty(plan.c.ste_pad_bytes if padded else plan.c.ste_bytes, dtype=torch.uint8, device=dev)
     ws, ws_bytes = _workspace(plan.c.ste_ws if needs[0] else 0, dev)
-    _lib.call("ntlb_linear_ste_backward", plan.ref, ptr, ld, None if buf is None else buf.data_ptr(), ops._ptr(dx),
-              ops._ptr(dw), ops._ptr(db), 0 if db is None else ops._dtype_code(bias_dtype), scratch.data_ptr(),
-              scratch.numel(), ws, ws_bytes, ops._stream())
+    _lib.call("ntlb_linear_ste_backward", plan.ref, ptr, ld, xp, wp, ops._ptr(dx), ops._ptr(dw), ops._ptr(db),
+              0 if db is None else ops._dtype_code(bias_dtype), scratch.data_ptr(), scratch.numel(), ws, ws_bytes,
+              ops._stream())
     return dx, dw, db
 
 
@@ -278,22 +277,32 @@ class _HipLowBitLinear(torch.autograd.Function):
             plan = backend._plan(x2, weight, None if bias is None else bias.dtype)
             base = backend._next_offset()
             dev = x.device
-            buf = torch.empty(plan.code_bytes, dtype=torch.uint8, device=dev)
+            # a straight-through backward reads X's codes for dW and W's for dX: one
+            # buffer where both or none are kept, else one each, so that the
+            # other is given back after the call
+            ste = backend.backward_recipe == "ste"
+            keep_x, keep_w = ste and needs[1], ste and needs[0]
+            if keep_x == keep_w:
+                xb = torch.empty(plan.x_bytes + plan.w_bytes, dtype=torch.uint8, device=dev)
+                xp, kept = xb.data_ptr(), (xb,) if keep_x else ()
+                wp = xp + plan.x_bytes
+            else:
+                xb = torch.empty(plan.x_bytes, dtype=torch.uint8, device=dev)
+                wb = torch.empty(plan.w_bytes, dtype=torch.uint8, device=dev)
+                xp, wp, kept = xb.data_ptr(), wb.data_ptr(), (xb,) if keep_x else (wb,)
             y = torch.empty((*x.shape[:-1], N), dtype=out_dtype, device=dev)
             ws, ws_bytes = (None, 0) if plan.ws_bytes == 0 else _workspace(plan.ws_bytes, dev)
             if bias is not None and bias.stride(-1) != 1:
                 bias = bias.contiguous()
             _lib.call("ntlb_linear_forward", plan.ref, x2.data_ptr(), weight.data_ptr(),
-                      None if bias is None else bias.data_ptr(), buf.data_ptr(), y.data_ptr(), ws, ws_bytes, base,
+                      None if bias is None else bias.data_ptr(), xp, wp, y.data_ptr(), ws, ws_bytes, base,
                       ops._stream())
             if needs[0] or needs[1] or needs[2]:
                 ctx.plan, ctx.backend, ctx.offset = plan, backend, base
                 ctx.bias_dtype = None if bias is None else bias.dtype
                 ctx.x_shape, ctx.x_dtype, ctx.w_dtype = x.shape, out_dtype, weight.dtype
-                if backend.backward_recipe == "ste":
-                    ctx.save_for_backward(buf)
-                else:
-                    ctx.save_for_backward(x2, weight)
+                ctx.kept_x, ctx.kept_w = keep_x, keep_w
+                ctx.save_for_backward(*(kept if ste else (x2, weight)))
             return y
         x2 = x.reshape(-1, K)
         if x2.stride(-1) != 1:
@@ -391,20 +400,22 @@ class _HipLowBitLinear(torch.autograd.Function):
         if plan is not None:
             dy2 = _rows_2d(dy, plan.N)
             if backend.backward_recipe == "ste":
-                (buf,) = ctx.saved_tensors
-                buf = _saved_codes(buf, plan.code_bytes)
+                buf, nx = None, plan.x_bytes if ctx.kept_x else 0
+                xp = wp = None
+                if ctx.kept_x or ctx.kept_w:
+                    buf = _saved_codes(ctx.saved_tensors[0], nx + (plan.w_bytes if ctx.kept_w else 0))
+                    xp, wp = buf.data_ptr() if ctx.kept_x else None, buf.data_ptr() + nx if ctx.kept_w else None
                 if dy2.dtype == torch.bfloat16 and ctx.x_dtype == torch.bfloat16 and ctx.w_dtype == torch.bfloat16:
-                    return (*_ste_backward(plan, dy2, buf, needs, ctx.x_shape, ctx.bias_dtype), None)
+                    return (*_ste_backward(plan, dy2, xp, wp, needs, ctx.x_shape, ctx.bias_dtype), None)
                 # another gradient dtype: the dequantized operands on the fp32 GEMM
-                qx, qw = plan.qtensors(buf)
                 dx = dw = None
                 if needs[0]:
-                    wdq = ops.dequant(qw, out_dtype=ctx.w_dtype)
+                    wdq = ops.dequant(plan.w_tensor(buf[nx:]), out_dtype=ctx.w_dtype)
                     op = _gemm_op_dtype(dy2.dtype, wdq.dtype)
                     dx = ops.gemm_dense(dy2.to(op), wdq.to(op), b_transposed=True,
                                         out_dtype=ctx.x_dtype).reshape(ctx.x_shape)
                 if needs[1]:
-                    xdq = ops.dequant(qx, out_dtype=ctx.x_dtype)
+                    xdq = ops.dequant(plan.x_tensor(buf), out_dtype=ctx.x_dtype)
                     op = _gemm_op_dtype(dy2.dtype, xdq.dtype)
                     dw = ops.gemm_dense_tn(dy2.to(op), xdq.to(op), out_dtype=ctx.w_dtype)
             else:

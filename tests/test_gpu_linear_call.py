@@ -261,3 +261,52 @@ def test_saved_tensor_hooks(gpu_device, recipe):
     if recipe == "ste":
         with pytest.raises(RuntimeError, match="saved codes"):
             grads(lambda s: s, lambda s: s[:-256])
+
+
+@pytest.mark.parametrize("grads", [(True, True, True), (True, False, True), (False, True, False), (False, False, True)])
+def test_saved_memory_follows_the_wanted_gradients(gpu_device, grads):
+    """the storage kept for a straight-through backward: W's codes for dX, X's
+    codes for dW, neither for db, as the general path keeps them (plus the
+    alignment of the parts and the int grid's row flags)"""
+    M, N, K = 500, 700, 1000
+    x = seeded((M, K), seed=20262181).to(gpu_device)
+    w = seeded((N, K), seed=20262182, std=0.02).to(gpu_device)
+    b = seeded((N,), seed=20262183).to(gpu_device)
+    held = []
+    for general in (False, True):
+        be = _backend("int_grid", "nearest", "ste", K, N)
+        if general:
+            be._one_call = lambda *a: False
+        t = [v.clone().requires_grad_(g) for v, g in zip((x, w, b), grads)]
+        storages = {}
+
+        def pack(s):
+            storages[s.untyped_storage().data_ptr()] = s.untyped_storage().nbytes()
+            return s
+
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda s: s):
+            be.linear(*t)
+        held.append(sum(storages.values()))
+    assert held[0] <= held[1] + 6 * 256 + 4 * (M + N), held
+
+
+@pytest.mark.parametrize("grads", [(True, True), (True, False), (False, True)])
+def test_gradient_of_another_dtype(gpu_device, grads):
+    """an fp32 dY handed to the backward: the dequantized operands, rebuilt from
+    the parts that were kept"""
+    M, N, K = 70, 200, 300
+    x = seeded((M, K), seed=20262195).to(gpu_device)
+    w = seeded((N, K), seed=20262196, std=0.02).to(gpu_device)
+    dy = seeded((M, N), seed=20262197, std=1e-3, dtype=torch.float32).to(gpu_device)
+    from lowbit.backend import _HipLowBitLinear
+
+    out = []
+    for general in (False, True):
+        be = _backend("int_grid", "nearest", "ste", K, N)
+        if general:
+            be._one_call = lambda *a: False
+        t = [v.clone().requires_grad_(g) for v, g in zip((x, w), grads)]
+        y = be.linear(*t, None)
+        out.append(_HipLowBitLinear.backward(y.grad_fn, dy))
+    assert all(_same(p, q) for p, q in zip(*out))
+    assert [v is not None for v in out[0]] == [*grads, False, False]
