@@ -264,7 +264,7 @@ int ntlb_gemm_blockscaled_ws(int grid, const uint8_t* a, int64_t lda, const floa
                              void* stream);
 
 /* Workspace bytes ntlb_gemm_blockscaled_ws uses for this shape on the current
- * device (0: the shape runs unsplit). */
+ * device (0: the shape runs unsplit, or on tiles below 256x256). */
 int64_t ntlb_gemm_workspace_bytes(int64_t M, int64_t N, int64_t Kp);
 
 /*
@@ -530,7 +530,9 @@ int ntlb_gemm_bf16_tn(const void* a, int64_t lda, const void* b, int64_t ldb, in
  * dw, W's for dx: each can be freed where its gradient is not wanted, and both
  * may be parts of one allocation), the scratch bytes of each backward, and the
  * bytes of the zeroed split-K workspace each call can use (as
- * ntlb_gemm_blockscaled_ws; 0 or NULL: none).  A plan holds no pointers and is
+ * ntlb_gemm_blockscaled_ws; 0 or NULL: none; the straight-through backward uses
+ * none where dY, or its padded copy, has a row pitch of at most
+ * ste_free_pitch).  A plan holds no pointers and is
  * not written after its init, so threads and streams may share it.  Buffers
  * are 256-byte aligned; y, dx and dw are contiguous.
  */
@@ -539,6 +541,7 @@ typedef struct ntlb_linear_plan {
   int x_dtype, w_dtype, bias_dtype, grid, qmax, rounding;
   uint64_t seed;
   int64_t x_code_bytes, w_code_bytes, ste_bytes, ste_pad_bytes, recipe_bytes, forward_ws, ste_ws, recipe_ws;
+  int64_t ste_free_pitch;
 } ntlb_linear_plan;
 
 int ntlb_linear_plan_init(ntlb_linear_plan* plan);

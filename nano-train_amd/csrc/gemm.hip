@@ -622,7 +622,7 @@ static void launch_store(const GemmArgs& g, dim3 grd, dim3 blk, hipStream_t st) 
 extern "C" int64_t ntlb_gemm_workspace_bytes(int64_t M, int64_t N, int64_t Kp) {
   if (M <= 0 || N <= 0 || Kp <= 0 || Kp % BK) return 0;
   const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-  if (tiles > 0x7FFFFFFF) return 0;
+  if (tiles > 0x7FFFFFFF || small_gemm_fits(M, N, Kp)) return 0;
   return split_ws_bytes(split_plan(tiles, (int)(Kp / BK), SPLIT_MIN_BLOCKS));
 }
 

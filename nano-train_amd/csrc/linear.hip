@@ -143,14 +143,16 @@ static CodeLayout w_layout(const ntlb_linear_plan& p) {
 // GEMM decodes), and the padded dY (only touched where dY needs it)
 struct SteLayout {
   int64_t colsum, wd, xd, dy, bytes;
+  int64_t near_pitch;  // the widest row pitch of dY that those tiles take: beyond it 32-bit offsets could overflow
 };
 static SteLayout ste_layout(const ntlb_linear_plan& p) {
   Carve c;
   SteLayout l;
+  l.near_pitch = up(p.N, 64) + 8;
   const int64_t k8 = up(p.K, 8), lim = (int64_t)0x7FFFFFFF;
-  const bool small_dx = bf16_small_fits(p.M, p.K, up(p.N, 64), true) && (p.M + 256) * (up(p.N, 64) + 8) * 2 < lim &&
+  const bool small_dx = bf16_small_fits(p.M, p.K, up(p.N, 64), true) && (p.M + 256) * l.near_pitch * 2 < lim &&
                         (p.N + 64) * k8 * 2 < lim;
-  const bool small_dw = bf16_small_fits(p.N, p.K, up(p.M, 64), false) && (p.M + 64) * (up(p.N, 64) + 8) * 2 < lim &&
+  const bool small_dw = bf16_small_fits(p.N, p.K, up(p.M, 64), false) && (p.M + 64) * l.near_pitch * 2 < lim &&
                         (p.M + 64) * k8 * 2 < lim;
   l.colsum = c.take(std::max<int64_t>(ntlb_colsum_workspace_bytes(p.M, p.N), 4));
   l.wd = small_dx ? c.take(p.N * k8 * 2) : -1;
@@ -207,8 +209,10 @@ extern "C" int ntlb_linear_plan_init(ntlb_linear_plan* p) {
   const int64_t kp = up(p->K, 128), np = up(p->N, 128), mp = up(p->M, 128);
   p->x_code_bytes = x_layout(*p).bytes;
   p->w_code_bytes = w_layout(*p).bytes;
-  p->ste_bytes = ste_layout(*p).dy;
-  p->ste_pad_bytes = ste_layout(*p).bytes;
+  const SteLayout sl = ste_layout(*p);
+  p->ste_bytes = sl.dy;
+  p->ste_pad_bytes = sl.bytes;
+  p->ste_free_pitch = sl.wd >= 0 ? sl.near_pitch : 0;
   p->recipe_bytes = recipe_layout(*p).bytes;
   p->forward_ws = ntlb_gemm_workspace_bytes(p->M, p->N, kp);
   p->ste_ws = ntlb_gemm_dq_workspace_bytes(NTLB_BF16, p->M, p->K, p->N);
@@ -275,8 +279,7 @@ extern "C" int ntlb_linear_ste_backward(const ntlb_linear_plan* p, const void* d
     dy = pad;
     lddy = n64;
   }
-  // row pitches beyond the padded one could leave 32-bit offsets
-  const bool near_rows = lddy <= n64 + 8;
+  const bool near_rows = lddy <= sl.near_pitch;
   const bool small_dx = dx && sl.wd >= 0 && near_rows, small_dw = dw && sl.xd >= 0 && near_rows;
   if (small_dx || small_dw) {
     DecodeArgs d{};

@@ -148,7 +148,7 @@ class LinearPlan(ctypes.Structure):
                 ("x_dtype", _I32), ("w_dtype", _I32), ("bias_dtype", _I32), ("grid", _I32), ("qmax", _I32),
                 ("rounding", _I32), ("seed", _U64), ("x_code_bytes", _I64), ("w_code_bytes", _I64), ("ste_bytes", _I64),
                 ("ste_pad_bytes", _I64), ("recipe_bytes", _I64), ("forward_ws", _I64), ("ste_ws", _I64),
-                ("recipe_ws", _I64)]
+                ("recipe_ws", _I64), ("ste_free_pitch", _I64)]
 
 
 # entry points that return a value instead of a status

@@ -242,7 +242,8 @@ def _ste_backward(plan: _LinearPlan, dy2, xp, wp, needs, x_shape, bias_dtype):
     ld, ptr = dy2.stride(0), dy2.data_ptr()
     padded = plan.N % 64 != 0 or ld % 8 != 0 or ptr % 16 != 0
     scratch = torch.empty(plan.c.ste_pad_bytes if padded else plan.c.ste_bytes, dtype=torch.uint8, device=dev)
-    ws, ws_bytes = _workspace(plan.c.ste_ws if needs[0] else 0, dev)
+    pitch = ops.cdiv(plan.N, 64) * 64 if padded else ld
+    ws, ws_bytes = _workspace(plan.c.ste_ws if needs[0] and pitch > plan.c.ste_free_pitch else 0, dev)
     _lib.call("ntlb_linear_ste_backward", plan.ref, ptr, ld, xp, wp, ops._ptr(dx), ops._ptr(dw), ops._ptr(db),
               0 if db is None else ops._dtype_code(bias_dtype), scratch.data_ptr(), scratch.numel(), ws, ws_bytes,
               ops._stream())

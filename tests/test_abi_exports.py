@@ -123,3 +123,30 @@ def test_ep_entry_points_validate_without_gpu():
     assert b"scale group" in L.ntlb_last_error()
     # the split-K workspace size: zero for a K that is not whole 128-blocks
     assert L.ntlb_gemm_workspace_bytes(512, 1024, 1000) == 0
+
+
+def test_workspace_sizes_follow_the_tile_rule():
+    """split-K workspace only for products that run on 256x256 tiles: none for
+    those on smaller tiles, on their own or as part of a linear call"""
+    from lowbit import _lib
+
+    L = _lib.lib()
+    for m, n, kp in ((16, 4096, 4096), (512, 1024, 2304), (2048, 4096, 4096), (640, 768, 4608)):
+        assert L.ntlb_gemm_workspace_bytes(m, n, kp) == 0, (m, n, kp)
+    for m, n, kp in ((1500, 1600, 4608), (4100, 4000, 2304), (8192, 7168, 18432)):
+        assert L.ntlb_gemm_workspace_bytes(m, n, kp) > 0, (m, n, kp)
+
+    def plan(m, n, k):
+        p = _lib.LinearPlan(M=m, N=n, K=k, ldx=k, ldw=k, x_dtype=_lib.BF16, w_dtype=_lib.BF16, grid=_lib.GRID_E4M3,
+                            qmax=127)
+        _lib.call("ntlb_linear_plan_init", ctypes.addressof(p))
+        return p
+
+    p = plan(16, 4096, 4096)
+    assert p.forward_ws == p.recipe_ws == 0
+    # dX on small tiles: workspace only for a dY of wide pitch, which the 256x256 tiles take
+    p = plan(500, 1500, 4600)
+    assert p.ste_free_pitch == 1536 + 8 and p.ste_ws > 0
+    # 8192 x 7168 over 18432: every product fills the chip
+    p = plan(8192, 18432, 7168)
+    assert p.ste_free_pitch == 0 and p.ste_ws > 0 and p.recipe_ws > 0

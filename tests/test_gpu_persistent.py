@@ -198,6 +198,40 @@ def test_fused_gemm_split_tail_and_bias(gpu_device, fmt):
     assert rel_fro_bf16(y_bias[rows], ref) <= 1e-3
 
 
+@pytest.mark.parametrize("fmt", ["nf4", "mxfp4", "fp8p"])
+@pytest.mark.parametrize("M,N,K,splits", [(1100, 1030, 320, False), (1100, 1030, 2112, True), (70, 17001, 192, False)])
+def test_ragged_fused_gemm_on_256_tiles(gpu_device, fmt, M, N, K, splits):
+    """shapes past the rows kernel's limit, with ragged edges, a K of an odd
+    number of 64-blocks and, in the second, a split tail; fp32 output with a
+    bias against a float64 product of the stored bf16 values: fp32 sums of K
+    products, at most (K + 2) * 2^-24 of the terms' magnitudes"""
+    from lowbit import _lib, persistent as P
+
+    assert (int(_lib.lib().ntlb_gemm_lowbit_workspace_bytes(M, N, K)) > 0) == splits
+    x = seeded((M, K), seed=20260514).to(gpu_device)
+    w = seeded((N, K), seed=20260515, std=0.02).to(gpu_device)
+    bias = seeded((N,), seed=20260516, std=0.5).to(gpu_device)
+    bf = torch.bfloat16
+    if fmt == "nf4":
+        q = P.quantize_nf4_blocks(w, 64)
+        wdq = P.dequantize_nf4_blocks(*q, num_values=N * K, block=64, target_dtype=bf)
+        run = lambda b, od: P.linear_nf4(x, *q, out_features=N, block=64, bias=b, out_dtype=od)
+    elif fmt == "mxfp4":
+        q = P.quantize_mxfp4(w)
+        wdq = P.dequantize_mxfp4(*q, num_values=N * K, target_dtype=bf)
+        run = lambda b, od: P.linear_mxfp4(x, *q, out_features=N, bias=b, out_dtype=od)
+    else:
+        q = P.quantize_fp8_persistent(w, granularity="per_channel")
+        wdq = P.dequantize_fp8_persistent(*q, target_dtype=bf)
+        run = lambda b, od: P.linear_fp8p(x, *q, bias=b, out_dtype=od)
+    wdq = wdq.reshape(N, K).double()
+    y = run(bias, torch.float32)
+    ref = x.double() @ wdq.T + bias.double()
+    mag = x.double().abs() @ wdq.abs().T + bias.double().abs()
+    assert float(((y.double() - ref).abs() / mag).max()) <= (K + 2) * 2.0 ** -24
+    assert torch.equal(run(bias, bf), y.to(bf)) and torch.equal(run(bias, torch.float32), y)
+
+
 @pytest.mark.parametrize("M,N,K", [(256, 256, 256), (130, 200, 320), (512, 512, 2048)])
 def test_mxfp4_fused_gemm(gpu_device, M, N, K):
     from lowbit import persistent as P
