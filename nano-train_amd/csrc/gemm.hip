@@ -663,10 +663,7 @@ extern "C" int ntlb_gemm_blockscaled_ws(int grid, const uint8_t* a, int64_t lda,
   if (workspace && !aligned(workspace, 256)) return fail(NTLB_EINVAL, "%s: workspace must be 256-byte aligned", fn);
   // B's scale is uniform over each wave's columns for 128x128 blocks and tensor scales
   const bool b_uniform = (b_shift == 7) || (sb_row == 0);
-  if (small_gemm_fits(M, N, Kp)) {
-    small_gemm_launch(grid, b_uniform, g, as_stream(stream));
-    return check_launch(fn);
-  }
+  if (small_gemm_fits(M, N, Kp)) return small_gemm_launch(fn, grid, b_uniform, g, as_stream(stream));
   int64_t grid_wgs = tiles;
   if (workspace) {
     const SplitPlan plan = split_plan(tiles, (int)(Kp / BK), SPLIT_MIN_BLOCKS);

@@ -1,6 +1,7 @@
 // bf16 GEMM on tiles below 256x256, fp32 accumulation: the products of
 // gemm_dq.hip over plain bf16 matrices whose 256x256 tiles would leave most of
-// the chip idle (the gradients of small layers, the dense GEMMs).
+// the chip idle (dX and dW of small straight-through layers, dW of persistent
+// ones).
 //
 // 16*MB x 16*NB tiles, a workgroup's WK waves dividing the contraction, each
 // wave with its own multi-stage LDS copies and no barrier in the K loop, as
@@ -130,10 +131,6 @@ struct Copies {
 };
 
 __device__ __forceinline__ void store4(const Bf16Args& g, int64_t m, int64_t n, v4f v) {
-  if (g.bias) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) v[q] += load_elem(g.bias, g.bias_dtype, min<int64_t>(n + q, g.N - 1));
-  }
   if (g.vec_out && n + 4 <= g.N && g.y_dtype == DT_BF16) {
     const v2bf p0 = {(__bf16)v[0], (__bf16)v[1]}, p1 = {(__bf16)v[2], (__bf16)v[3]};
     *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(g.y) + m * g.ldy + n) =
@@ -145,7 +142,7 @@ __device__ __forceinline__ void store4(const Bf16Args& g, int64_t m, int64_t n, 
     if (n + q < g.N) store_elem(g.y, g.y_dtype, m * g.ldy + n + q, v[q]);
 }
 
-template <bool TA, bool TB, int MB, int NB, int WK, int NS>
+template <bool TA, int MB, int NB, int WK, int NS>
 __global__ void __launch_bounds__(64 * WK) gemm_bf16_small_kernel(Bf16Args g) {
   constexpr int WB = (MB + NB) * 16 * ROWB;
   static_assert(MB * NB * 1024 <= WB, "the partial tiles fit the first stage");
@@ -163,7 +160,7 @@ __global__ void __launch_bounds__(64 * WK) gemm_bf16_small_kernel(Bf16Args g) {
     for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = (v4f){0.f, 0.f, 0.f, 0.f};
   if (k0 < k1) {
     Copies<TA, MB, 1> ca;
-    Copies<TB, NB, 1> cb;
+    Copies<true, NB, 1> cb;
     ca.init(g.a, m0, 0, lane);
     cb.init(g.b, n0, 0, lane);
     uint8_t* const s0 = st0 + wave * WB;
@@ -192,7 +189,7 @@ __global__ void __launch_bounds__(64 * WK) gemm_bf16_small_kernel(Bf16Args g) {
       const uint8_t* tb = ta + MB * 16 * ROWB;
       v8i bf[NB];
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) bf[nb] = frag<TB, NB>(tb, nb * 16, lane);
+      for (int nb = 0; nb < NB; ++nb) bf[nb] = frag<true, NB>(tb, nb * 16, lane);
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
         const v8i af = frag<TA, MB>(ta, mb * 16, lane);
@@ -232,7 +229,7 @@ __global__ void __launch_bounds__(64 * WK) gemm_bf16_small_kernel(Bf16Args g) {
 
 constexpr int MID = 128;
 
-template <bool TA, bool TB, int ODT>
+template <bool TA, int ODT>
 __global__ void __launch_bounds__(256, 2) gemm_bf16_mid_kernel(Bf16Args g) {
   constexpr int ST = MID * ROWB;  // 16 KiB per operand stage
   __shared__ __attribute__((aligned(16))) uint8_t la0[ST];
@@ -256,7 +253,7 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16_mid_kernel(Bf16Args g) {
     n0 = (int64_t)(in_group / gsize) * MID;
   }
   Copies<TA, 8, 4> ca;
-  Copies<TB, 8, 4> cb;
+  Copies<true, 8, 4> cb;
   ca.init(g.a, m0, wave, lane);
   cb.init(g.b, n0, wave, lane);
   const int nk = (int)(g.Kc / KSTEP);
@@ -278,7 +275,7 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16_mid_kernel(Bf16Args g) {
     cb.issue(BUF ? lb0 : lb1, kn);
     v8i bf[4];
 #pragma unroll
-    for (int tn = 0; tn < 4; ++tn) bf[tn] = frag<TB, 8>(tb, wn * 64 + tn * 16, lane);
+    for (int tn = 0; tn < 4; ++tn) bf[tn] = frag<true, 8>(tb, wn * 64 + tn * 16, lane);
 #pragma unroll
     for (int tm = 0; tm < 4; ++tm) {
       const v8i af = frag<TA, 8>(ta, wm * 64 + tm * 16, lane);
@@ -302,12 +299,7 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16_mid_kernel(Bf16Args g) {
     for (int t = 0; t < 2; ++t) {
 #pragma unroll
       for (int tn = 0; tn < 4; ++tn) {
-        v4f v = acc[part * 2 + t][tn];
-        if (g.bias) {
-          const int64_t n = n0 + wn * 64 + tn * 16 + (lane >> 4) * 4;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) v[q] += load_elem(g.bias, g.bias_dtype, min<int64_t>(n + q, g.N - 1));
-        }
+        const v4f v = acc[part * 2 + t][tn];
         uint8_t* dst = stage_w + (t * 16 + (lane & 15)) * pitch + (tn * 16 + (lane >> 4) * 4) * esz;
         if constexpr (ODT == DT_F32) {
           *reinterpret_cast<v4f*>(dst) = v;
@@ -347,36 +339,61 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16_mid_kernel(Bf16Args g) {
 // every instance explicitly: the host stubs of implicitly instantiated ones
 // are not all emitted here (ROCm 7.2 hipcc)
 #define NTLB_BF16_CASES(X) X(1, 1, 8, 2) X(1, 2, 4, 3) X(2, 2, 4, 3) X(2, 4, 4, 3) X(4, 4, 4, 2) X(4, 4, 2, 2)
-#define NTLB_BF16_INST(MB, NB, WK, NS)                                                            \
-  template __global__ void gemm_bf16_small_kernel<true, true, MB, NB, WK, NS>(Bf16Args);          \
-  template __global__ void gemm_bf16_small_kernel<false, true, MB, NB, WK, NS>(Bf16Args);         \
-  template __global__ void gemm_bf16_small_kernel<false, false, MB, NB, WK, NS>(Bf16Args);
-#define NTLB_BF16_MID_INST(ODT)                                        \
-  template __global__ void gemm_bf16_mid_kernel<true, true, ODT>(Bf16Args);   \
-  template __global__ void gemm_bf16_mid_kernel<false, true, ODT>(Bf16Args);  \
-  template __global__ void gemm_bf16_mid_kernel<false, false, ODT>(Bf16Args);
+#define NTLB_BF16_INST(MB, NB, WK, NS)                                              \
+  template __global__ void gemm_bf16_small_kernel<true, MB, NB, WK, NS>(Bf16Args);  \
+  template __global__ void gemm_bf16_small_kernel<false, MB, NB, WK, NS>(Bf16Args);
 NTLB_BF16_CASES(NTLB_BF16_INST)
-NTLB_BF16_MID_INST(DT_F32)
-NTLB_BF16_MID_INST(DT_BF16)
-NTLB_BF16_MID_INST(DT_F16)
 #undef NTLB_BF16_INST
-#undef NTLB_BF16_MID_INST
+template __global__ void gemm_bf16_mid_kernel<true, DT_F32>(Bf16Args);
+template __global__ void gemm_bf16_mid_kernel<true, DT_BF16>(Bf16Args);
+template __global__ void gemm_bf16_mid_kernel<true, DT_F16>(Bf16Args);
+template __global__ void gemm_bf16_mid_kernel<false, DT_BF16>(Bf16Args);
 
-struct Plan {
-  int mb, nb, wk, ns;
-};
+template <bool TA>
+static int launch(const char* fn, const Bf16Plan& p, const Bf16Args& g, hipStream_t st) {
+  if (p.mb == 8) {
+    const dim3 grd((unsigned)(cdiv(g.M, MID) * cdiv(g.N, MID))), blk(256);
+    if (g.y_dtype == DT_BF16) {
+      gemm_bf16_mid_kernel<TA, DT_BF16><<<grd, blk, 0, st>>>(g);
+      return check_launch(fn);
+    }
+    if constexpr (TA) {
+      if (g.y_dtype == DT_F32)
+        gemm_bf16_mid_kernel<TA, DT_F32><<<grd, blk, 0, st>>>(g);
+      else
+        gemm_bf16_mid_kernel<TA, DT_F16><<<grd, blk, 0, st>>>(g);
+      return check_launch(fn);
+    }
+  }
+  const dim3 grd((unsigned)cdiv(g.N, 16 * p.nb), (unsigned)cdiv(g.M, 16 * p.mb)), blk(64 * p.wk);
+#define NTLB_BF16_CASE(MB, NB, WK, NS)                                              \
+  if (p.mb == MB && p.nb == NB && p.wk == WK && p.ns == NS) {                       \
+    gemm_bf16_small_kernel<TA, MB, NB, WK, NS><<<grd, blk, 0, st>>>(g);             \
+    return check_launch(fn);                                                        \
+  }
+  NTLB_BF16_CASES(NTLB_BF16_CASE)
+#undef NTLB_BF16_CASE
+  return fail(NTLB_EUNSUPPORTED, "%s: no kernel for a %d x %d tile", fn, 16 * p.mb, 16 * p.nb);
+}
 
-// The tile of a product (mb = 8: 128x128; mb = 0: the 256x256 tiles of
-// gemm_dq.hip): the smallest one whose workgroups all run at once, as the
+}  // namespace bfs
+
+// The tile: the smallest one whose workgroups all run at once, as the
 // blockwise products choose it.  Measured (both operands transposed, bf16 out,
 // in a graph, us; this kernel / 256x256 tiles): 1000 x K 1003: 4.9 / 25 at 64
 // rows, 7.8 / 25 at 512, 9.9 / 26 at 1003, 13.7 / 26 at 1541, 19 / 27 at 4096;
 // 2048 x K 2048: 7.7 / 44 at 128 rows, 12.4 / 44 at 512, 21 / 46 at 1003, 33 / 45
-// at 2048, 36 / 46 at 4096.  Between 128x128 and 256x256 tiles the estimates
-// decide: 1.05 us a K step for 128x128 tiles, 1.4 for 256x256 ones, whose
-// split-K tail (big_split: the caller has its workspace) adds about 30 us.
-static Plan plan(int64_t M, int64_t N, int nk, bool big_split) {
+// at 2048, 36 / 46 at 4096.
+//
+// 128x128 tiles run two to a compute unit, and up to two of them for each unit
+// they beat unsplit 256x256 tiles at every K: 512 tiles (4096 x 2048) 6.7 / 7.8 at K
+// 64, 21.5 / 27 at 1024, 36 / 47 at 2048, 129 / 162 at 8192, while 529 tiles (2880 x
+// 2880), a second round of them, take 8.6 / 8.1, 37 / 27, 65 / 46 and 239 / 161.
+// Where the 256x256 tiles would split their tail (big_split), an estimate
+// decides: 1.05 us a K step here, 1.4 / split there and 30 us for the exchange.
+Bf16Plan bf16_small_plan(int64_t M, int64_t N, int64_t Kc, bool big_split) {
   const int64_t cus = split_device_cus();
+  const int nk = (int)(Kc / bfs::KSTEP);
   auto wgs = [&](int64_t rows, int64_t cols) { return cdiv(M, rows) * cdiv(N, cols); };
   if (wgs(16, 16) <= cus) return {1, 1, 8, 2};
   if (wgs(16, 32) <= cus || M <= 16) return {1, 2, 4, 3};
@@ -384,50 +401,15 @@ static Plan plan(int64_t M, int64_t N, int nk, bool big_split) {
   if (wgs(32, 64) <= cus) return {2, 4, 4, 3};
   if (wgs(64, 64) <= cus) return {4, 4, 4, 2};
   if (wgs(64, 64) <= 2 * cus) return {4, 4, 2, 2};
-  if (wgs(MID, MID) <= 2 * cus) {
+  if (wgs(bfs::MID, bfs::MID) <= 2 * cus) {
     const int split = big_split ? split_plan(wgs(256, 256), nk, DQ_SPLIT_MIN_STEPS).s : 1;
-    if (1.05 * nk + 3 < 1.4 * nk / split + (split > 1 ? 30 : 6)) return {8, 8, 4, 2};
+    if (split == 1 || 1.05 * nk + 3 < 1.4 * nk / split + 30) return {8, 8, 4, 2};
   }
   return {0, 0, 0, 0};
 }
 
-template <bool TA, bool TB>
-static void launch(const Plan& p, const Bf16Args& g, hipStream_t st) {
-  if (p.mb == 8) {
-    const dim3 grd((unsigned)(cdiv(g.M, MID) * cdiv(g.N, MID))), blk(256);
-    if (g.y_dtype == DT_F32)
-      gemm_bf16_mid_kernel<TA, TB, DT_F32><<<grd, blk, 0, st>>>(g);
-    else if (g.y_dtype == DT_F16)
-      gemm_bf16_mid_kernel<TA, TB, DT_F16><<<grd, blk, 0, st>>>(g);
-    else
-      gemm_bf16_mid_kernel<TA, TB, DT_BF16><<<grd, blk, 0, st>>>(g);
-    return;
-  }
-  const dim3 grd((unsigned)cdiv(g.N, 16 * p.nb), (unsigned)cdiv(g.M, 16 * p.mb)), blk(64 * p.wk);
-#define NTLB_BF16_CASE(MB, NB, WK, NS)                                                  \
-  if (p.mb == MB && p.nb == NB && p.wk == WK && p.ns == NS) {                           \
-    gemm_bf16_small_kernel<TA, TB, MB, NB, WK, NS><<<grd, blk, 0, st>>>(g);             \
-    return;                                                                             \
-  }
-  NTLB_BF16_CASES(NTLB_BF16_CASE)
-#undef NTLB_BF16_CASE
-}
-
-}  // namespace bfs
-
-bool bf16_small_fits(int64_t M, int64_t N, int64_t Kc, bool big_split) {
-  return bfs::plan(M, N, (int)(Kc / bfs::KSTEP), big_split).mb != 0;
-}
-
-void bf16_small_launch(const Bf16Args& g, hipStream_t st) {
-  const int nk = (int)(g.Kc / bfs::KSTEP);
-  bfs::Plan p = bfs::plan(g.M, g.N, nk, false);
-  if (g.a.tr)
-    bfs::launch<true, true>(p, g, st);
-  else if (g.b.tr)
-    bfs::launch<false, true>(p, g, st);
-  else
-    bfs::launch<false, false>(p, g, st);
+int bf16_small_launch(const char* fn, const Bf16Plan& p, const Bf16Args& g, hipStream_t st) {
+  return g.a.tr ? bfs::launch<true>(fn, p, g, st) : bfs::launch<false>(fn, p, g, st);
 }
 
 }  // namespace ntlb

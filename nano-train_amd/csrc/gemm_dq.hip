@@ -1931,9 +1931,10 @@ extern "C" int ntlb_gemm_bf16_tn(const void* a, int64_t lda, const void* b, int6
                                  int64_t K, void* y, int y_dtype, int64_t ldy, void* stream) {
   const char* fn = "ntlb_gemm_bf16_tn";
   const int64_t kc = (K + 63) / 64 * 64;
+  const Bf16Plan plan = M < 1 || N < 1 || K < 1 ? Bf16Plan{} : bf16_small_plan(M, N, kc, false);
   if (M < 1 || N < 1 || K < 1 || !a || !b || !y || lda < M || ldb < N || !aligned(a, 16) || !aligned(b, 16) ||
       lda % 8 || ldb % 8 || (K + 64) * lda * 2 >= (int64_t)0x7FFFFFFF || (K + 64) * ldb * 2 >= (int64_t)0x7FFFFFFF ||
-      !valid_dtype(y_dtype) || ldy < N || !bf16_small_fits(M, N, kc, false))
+      !valid_dtype(y_dtype) || ldy < N || !plan.fits())
     return ntlb_gemm_dense_tn(NTLB_BF16, a, lda, b, ldb, M, N, K, y, y_dtype, ldy, stream);  // or its error
   Bf16Args g{};
   g.a = Bf16Operand{a, lda, M, K, true};
@@ -1941,6 +1942,5 @@ extern "C" int ntlb_gemm_bf16_tn(const void* a, int64_t lda, const void* b, int6
   g.M = M; g.N = N; g.Kc = kc;
   g.y = y; g.y_dtype = y_dtype; g.ldy = ldy;
   g.vec_out = aligned(y, 16) && ((ldy * dtype_size(y_dtype)) % 16 == 0);
-  bf16_small_launch(g, as_stream(stream));
-  return check_launch(fn);
+  return bf16_small_launch(fn, plan, g, as_stream(stream));
 }

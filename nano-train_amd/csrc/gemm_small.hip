@@ -455,7 +455,7 @@ static SmallPlan small_plan(int64_t M, int64_t N, int nk) {
 bool small_gemm_fits(int64_t M, int64_t N, int64_t Kp) { return small_plan(M, N, (int)(Kp / BK)).mb != 0; }
 
 template <int GRID, bool B_UNIFORM>
-static void small_launch(const SmallPlan& p, const GemmArgs& g, hipStream_t st) {
+static int small_launch(const char* fn, const SmallPlan& p, const GemmArgs& g, hipStream_t st) {
   if (p.mb == 8) {
     const dim3 grd((unsigned)(cdiv(g.M, MID) * cdiv(g.N, MID))), blk(256);
     if (g.y_dtype == DT_F32)
@@ -464,13 +464,13 @@ static void small_launch(const SmallPlan& p, const GemmArgs& g, hipStream_t st) 
       gemm_mid_kernel<GRID, B_UNIFORM, DT_F16><<<grd, blk, 0, st>>>(g);
     else
       gemm_mid_kernel<GRID, B_UNIFORM, DT_BF16><<<grd, blk, 0, st>>>(g);
-    return;
+    return check_launch(fn);
   }
   const dim3 grd((unsigned)cdiv(g.N, 16 * p.nb), (unsigned)cdiv(g.M, 16 * p.mb)), blk(64 * p.wk);
 #define NTLB_SMALL_CASE(MB, NB, WK, NS)                                                      \
   if (p.mb == MB && p.nb == NB && p.wk == WK && p.ns == NS) {                                \
     gemm_small_kernel<GRID, B_UNIFORM, MB, NB, WK, NS><<<grd, blk, 0, st>>>(g);              \
-    return;                                                                                  \
+    return check_launch(fn);                                                                 \
   }
   NTLB_SMALL_CASE(1, 1, 1, 3)
   NTLB_SMALL_CASE(1, 1, 8, 2)
@@ -480,21 +480,14 @@ static void small_launch(const SmallPlan& p, const GemmArgs& g, hipStream_t st) 
   NTLB_SMALL_CASE(4, 4, 4, 2)
   NTLB_SMALL_CASE(4, 4, 2, 2)
 #undef NTLB_SMALL_CASE
+  return fail(NTLB_EUNSUPPORTED, "%s: no kernel for a %d x %d tile", fn, 16 * p.mb, 16 * p.nb);
 }
 
-void small_gemm_launch(int grid, bool b_uniform, const GemmArgs& g, hipStream_t st) {
+int small_gemm_launch(const char* fn, int grid, bool b_uniform, const GemmArgs& g, hipStream_t st) {
   const SmallPlan p = small_plan(g.M, g.N, (int)(g.Kp / BK));
-  if (grid == GRID_E4M3) {
-    if (b_uniform)
-      small_launch<GRID_E4M3, true>(p, g, st);
-    else
-      small_launch<GRID_E4M3, false>(p, g, st);
-  } else {
-    if (b_uniform)
-      small_launch<GRID_INT, true>(p, g, st);
-    else
-      small_launch<GRID_INT, false>(p, g, st);
-  }
+  if (grid == GRID_E4M3)
+    return b_uniform ? small_launch<GRID_E4M3, true>(fn, p, g, st) : small_launch<GRID_E4M3, false>(fn, p, g, st);
+  return b_uniform ? small_launch<GRID_INT, true>(fn, p, g, st) : small_launch<GRID_INT, false>(fn, p, g, st);
 }
 
 // ---------------------------------------------------------------------------

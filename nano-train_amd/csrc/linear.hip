@@ -143,6 +143,7 @@ static CodeLayout w_layout(const ntlb_linear_plan& p) {
 // GEMM decodes), and the padded dY (only touched where dY needs it)
 struct SteLayout {
   int64_t colsum, wd, xd, dy, bytes;
+  Bf16Plan dx, dw;     // their tiles
   int64_t near_pitch;  // the widest row pitch of dY that those tiles take: beyond it 32-bit offsets could overflow
 };
 static SteLayout ste_layout(const ntlb_linear_plan& p) {
@@ -150,9 +151,11 @@ static SteLayout ste_layout(const ntlb_linear_plan& p) {
   SteLayout l;
   l.near_pitch = up(p.N, 64) + 8;
   const int64_t k8 = up(p.K, 8), lim = (int64_t)0x7FFFFFFF;
-  const bool small_dx = bf16_small_fits(p.M, p.K, up(p.N, 64), true) && (p.M + 256) * l.near_pitch * 2 < lim &&
+  l.dx = bf16_small_plan(p.M, p.K, up(p.N, 64), true);
+  l.dw = bf16_small_plan(p.N, p.K, up(p.M, 64), false);
+  const bool small_dx = l.dx.fits() && (p.M + 256) * l.near_pitch * 2 < lim &&
                         (p.N + 64) * k8 * 2 < lim;
-  const bool small_dw = bf16_small_fits(p.N, p.K, up(p.M, 64), false) && (p.M + 64) * l.near_pitch * 2 < lim &&
+  const bool small_dw = l.dw.fits() && (p.M + 64) * l.near_pitch * 2 < lim &&
                         (p.M + 64) * k8 * 2 < lim;
   l.colsum = c.take(std::max<int64_t>(ntlb_colsum_workspace_bytes(p.M, p.N), 4));
   l.wd = small_dx ? c.take(p.N * k8 * 2) : -1;
@@ -313,7 +316,7 @@ extern "C" int ntlb_linear_ste_backward(const ntlb_linear_plan* p, const void* d
       g.Kc = n64;
       g.y = dx;
       g.vec_out = aligned(dx, 16) && p->K % 8 == 0;
-      bf16_small_launch(g, as_stream(stream));
+      if (int rc = bf16_small_launch(fn, sl.dx, g, as_stream(stream))) return rc;
     }
     if (small_dw) {
       g.a = Bf16Operand{dy, lddy, p->N, p->M, true};
@@ -322,9 +325,8 @@ extern "C" int ntlb_linear_ste_backward(const ntlb_linear_plan* p, const void* d
       g.Kc = up(p->M, 64);
       g.y = dw;
       g.vec_out = aligned(dw, 16) && p->K % 8 == 0;
-      bf16_small_launch(g, as_stream(stream));
+      if (int rc = bf16_small_launch(fn, sl.dw, g, as_stream(stream))) return rc;
     }
-    if (int rc = check_launch(fn)) return rc;
   }
   if (dx && !small_dx) {
     const int rc = ntlb_gemm_ste_dgrad_ws(NTLB_BF16, dy, lddy, p->M, p->N, p->grid, wb + lw.c, kp,

@@ -8,8 +8,8 @@
 namespace ntlb {
 
 // One operand of Y[M,N] = A . B^T over plain bf16 matrices.
-//   tr = false: [rows, >= Kc] row-major, the contraction contiguous; columns
-//     past the contraction are zero or meet zeros of the other operand
+//   tr = false (A only): [rows, >= Kc] row-major, the contraction contiguous;
+//     columns past the contraction are zero or meet zeros of B
 //   tr = true: stored transposed, element (r, k) at p[k * ld + r]; contraction
 //     rows at or past kvalid read zero
 // 16-byte aligned with whole 16-byte rows, addressed with 32-bit byte offsets
@@ -25,8 +25,6 @@ struct Bf16Operand {
 struct Bf16Args {
   Bf16Operand a, b;
   int64_t M, N, Kc;  // Kc a multiple of 64
-  const void* bias;
-  int bias_dtype;
   void* y;
   int y_dtype;
   int64_t ldy;
@@ -37,10 +35,17 @@ struct Bf16Args {
 // steps per range
 constexpr int DQ_SPLIT_MIN_STEPS = 9;
 
-// whether a product of this shape runs on these tiles rather than on 256x256
-// ones (big_split: those would have a split-K workspace), and the launch (a tr
-// B with a non-tr A, both tr, or neither)
-bool bf16_small_fits(int64_t M, int64_t N, int64_t Kc, bool big_split);
-void bf16_small_launch(const Bf16Args& g, hipStream_t st);
+// The tile of a product: 16*mb x 16*nb with the contraction divided among wk
+// waves and ns copy stages (mb = 8: 128x128; mb = 0: the 256x256 tiles, not
+// these).  big_split: the 256x256 tiles would have a split-K workspace.
+struct Bf16Plan {
+  int mb, nb, wk, ns;
+  bool fits() const { return mb != 0; }
+};
+Bf16Plan bf16_small_plan(int64_t M, int64_t N, int64_t Kc, bool big_split);
+
+// launch the product on its plan's tile (a status; B tr, a bf16 y where A is
+// not tr)
+int bf16_small_launch(const char* fn, const Bf16Plan& p, const Bf16Args& g, hipStream_t st);
 
 }  // namespace ntlb

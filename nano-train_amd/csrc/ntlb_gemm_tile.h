@@ -1,5 +1,5 @@
 // What the blockwise-scaled GEMM kernels share (gemm.hip: 256x256 tiles;
-// gemm_small.hip: 16x16 to 64x64 tiles): the launch arguments, the swizzled
+// gemm_small.hip: 16x16 to 128x128 tiles): the launch arguments, the swizzled
 // LDS tile layout with its fragment reads, and the MFMA of one 128-wide K
 // block.
 #pragma once
@@ -159,7 +159,7 @@ constexpr int SPLIT_MIN_BLOCKS = 9;
 // are the better choice for the shape; false leaves the product to the
 // 256x256-tile kernel
 bool small_gemm_fits(int64_t M, int64_t N, int64_t Kp);
-void small_gemm_launch(int grid, bool b_uniform, const GemmArgs& g, hipStream_t st);
+int small_gemm_launch(const char* fn, int grid, bool b_uniform, const GemmArgs& g, hipStream_t st);
 
 // the same for per-expert products: M_total rows over n_experts experts of N
 // weight rows, B's scale uniform over a wave's columns
