@@ -1777,13 +1777,23 @@ extern "C" int ntlb_comm_quant_dequant(const void* x, int x_dtype, int64_t R, in
   // against 368-370)
   const int64_t gx = cdiv(cdiv(K, 8), 256);
   if (gx > 0x7FFFFFFF) return fail(NTLB_EUNSUPPORTED, "%s: rows too long", fn);
-  // but at least four rows each, which share the column groups, the scales and
-  // their reciprocals (5001 rows of 7168 with the amax pass, one / four / eight
-  // rows a workgroup: strip groups, stochastic 61.5 / 56.2 / 55.6, to nearest 42.3 /
-  // 42.9 / 44.7; channel groups 68.4 / 62.7 / 58.6 and 58.4 / 50.2 / 47.1; at 1003
-  // columns, strips 37.1 / 37.0 / 46.7)
-  dim3 grd((unsigned)gx,
-           (unsigned)std::max<int64_t>(1, std::min<int64_t>(cdiv(R, 4), std::min<int64_t>(65535, 8192 / gx)))),
+  // Rows of a workgroup share its column groups, scales and reciprocals, up to
+  // four rows, but follow each other: a payload whose waves all run at once
+  // takes one row each, and rows are shared as far as the waves exceed a
+  // chip-full of about 3400 (one group per chunk), or 896 where every element
+  // has its own scale and reciprocal to share (1792, and 3400
+  // with at most two rows, where the elements are loaded one by one).  The kernel alone in a
+  // graph, us, one / two / four rows: strips to nearest 16 x 7168 2.8 / 3.3 / 4.4,
+  // 256 x 7168 4.1 / 4.1 / 4.8, 1000 x 7168 8.0 / 6.9 / 6.7, 2000 x 2048 5.3 / 5.0 / 5.2, 5001 x
+  // 256 4.9 / 4.6 / 5.1, 1000 x 1003 4.7 / 5.4 / 7.3; stochastic 16 x 7168 3.2 / 4.0 / 5.7,
+  // 1000 x 7168 11.6 / 10.5 / 10.4, 1000 x 1003 6.5 / 8.7 / 12.1, 5001 x 1003 18.5 / 18.0 /
+  // 18.9; channel scales 256 x 2048 3.9 / 4.3 / 5.2, 1000 x 2048 7.4 / 5.8 / 5.6,
+  // 5001 x 7168 86 / 50 / 36.
+  const int64_t waves = R * cdiv(cdiv(K, 8), 64);
+  const int64_t full = gc % 8 == 0 ? 3400 : vec ? 896 : 1792;
+  const int64_t most = gc % 8 == 0 && !vec ? 2 : 4;
+  const int64_t rows = std::max<int64_t>(1, std::min(most, waves / full));
+  dim3 grd((unsigned)gx, (unsigned)std::max<int64_t>(1, std::min(cdiv(R, rows), std::min<int64_t>(65535, 8192 / gx)))),
       blk(256);
   hipStream_t st = as_stream(stream);
   NTLB_DISPATCH_DT(x_dtype, NTLB_DISPATCH_GRID_SR(grid, sr, {

@@ -50,6 +50,23 @@ def test_comm_quant_dequant_parity(gpu_device, granularity, rounding, shape, dty
     assert x.grad is not None and torch.equal(x.grad, torch.ones_like(x))
 
 
+# rows of one wave each, on both sides of the counts from which a workgroup
+# takes a second, third and fourth row (3400 waves per row with a scale per
+# chunk, 896 with one per element, 1792 of those where K is no multiple of 8)
+@pytest.mark.parametrize("granularity,shape", [("tensor", (6799, 64)), ("tensor", (6801, 64)), ("tensor", (10201, 72)),
+                                               ("tensor", (13605, 40)), ("tile_1x128", (6803, 129)),
+                                               ("channel", (1793, 64)), ("channel", (2689, 72)), ("channel", (3587, 64)),
+                                               ("channel", (3585, 65)), ("channel", (7171, 63))])
+@pytest.mark.parametrize("rounding", ["nearest", "stochastic"])
+def test_comm_quant_dequant_rows_per_workgroup(gpu_device, granularity, shape, rounding):
+    from lowbit import moe
+
+    x = seeded(shape, seed=20260403, outliers=0.01).to(gpu_device)
+    out = moe.comm_quant_dequant(x, granularity=granularity, rounding_mode=rounding, seed=9, offset=4)
+    rc = O.ROUND_STOCHASTIC if rounding == "stochastic" else O.ROUND_NEAREST
+    assert_bits_equal(out.float().cpu().numpy(), _ref_comm(x, granularity, rc, 8, 9, 4).float().numpy(), "comm dq")
+
+
 def test_comm_quant_dequant_special_values(gpu_device):
     from lowbit import moe
 
