@@ -423,7 +423,7 @@ int ntlb_gemm_dense_tn(int op_dtype, const void* a, int64_t lda, const void* b, 
 
 /* Bias gradient of F.linear (te_backend.py:253-259 under autograd):
  * out[n] = sum over m of x[m, n] in fp32, cast to out_dtype.  Deterministic:
- * fp32 partials per 256-row chunk in `workspace` (fp32, at least
+ * fp32 partials per 64- or 256-row chunk in `workspace` (fp32, at least
  * ntlb_colsum_workspace_bytes(M, N) bytes), added in chunk order. */
 int ntlb_colsum(const void* x, int x_dtype, int64_t M, int64_t N, int64_t ldx, float* workspace, int64_t ws_bytes,
                 void* out, int out_dtype, void* stream);

@@ -1142,9 +1142,10 @@ __global__ void __launch_bounds__(256) colsum_partial_kernel(const void* x, int6
   }
 }
 
-// The same sums where the chunks above would be fewer than the compute units:
-// 64 rows by 128 columns per workgroup, a wave's 16 rows all loaded before
-// they are added (dY 1003 x 1541: 16 workgroups and 38 us became 208 and 5).
+// The same sums on more workgroups: 64 rows by 128 columns each, a wave's 16
+// rows all loaded before they are added, by 4-byte (fp32: 8-byte) loads that
+// need no 16-byte rows (dY 1003 x 1541: 16 workgroups and 47 us for the call
+// became 208 and 7.8).  colsum_small says which sums take it.
 constexpr int CS_ROWS_S = 64, CS_COLS_S = 128;
 
 template <int IN_DT>
@@ -1885,12 +1886,33 @@ extern "C" int ntlb_gemm_dense_tn(int op_dtype, const void* a, int64_t lda, cons
   return finish(fn, g, el, SRC_TDIRECT, SRC_TDIRECT, y_dtype, ldy, stream);
 }
 
-// whether the 256-row x 512-column chunks would leave compute units idle
-static bool colsum_small(int64_t M, int64_t N) { return cdiv(M, CS_ROWS) * cdiv(N, CS_COLS) < split_device_cus(); }
+// Where the 256-row x 512-column chunks would leave compute units idle, the
+// 64-row chunks are in question; the workspace holds either's partials.
+static bool colsum_few(int64_t M, int64_t N) { return cdiv(M, CS_ROWS) * cdiv(N, CS_COLS) < split_device_cus(); }
+
+// Which of those sums take the 64-row chunks.  The large chunks load 16 bytes
+// a lane and have a quarter of the partials; a wave of theirs with columns
+// past N, or without 16-byte rows, loads element by element.  The call in a
+// graph, us, large / 64-row chunks:
+//   rows without 16-byte alignment: 1024 x 1023 43 / 8.5, 65000 x 511 73 / 70
+//   fp32: 256 x 4096 15.7 / 6.5, 4096 x 8192 34 / 26, 16384 x 1024 31 / 24, 65000 x 512
+//     37 / 64
+//   16 bits, N in whole chunks: 64 x 8192 5.4 / 6.5, 160 x 1024 6.2 / 6.5, 256 x 4096
+//     7.7 / 7.1, 1024 x 14336 11.4 / 8.2, 1024 x 18432 12.1 / 16.6, 2048 x 8192 9.3 / 11.8,
+//     3072 x 512 8.6 / 8.0, 4096 x 512 8.0 / 8.7, 8192 x 1024 8.8 / 12.1
+//   16 bits, other N: 64 x 768 6.5 / 6.1, 2048 x 11008 19 / 18, 8192 x 768 15.9 / 11.8,
+//     16384 x 768 18 / 20, 16384 x 64 21 / 15, 65000 x 64 26 / 42
+static bool colsum_small(const void* x, int dt, int64_t M, int64_t N, int64_t ld) {
+  if (!colsum_few(M, N)) return false;
+  if (!aligned(x, 16) || ld * dtype_size(dt) % 16) return true;
+  if (dt == NTLB_F32) return M <= 16384;
+  if (N % CS_COLS) return M <= (N < CS_COLS ? 16384 : 8192);
+  return M >= 192 && M <= 3072 && cdiv(M, CS_ROWS_S) * (N / CS_COLS_S) <= 7 * (int64_t)split_device_cus();
+}
 
 extern "C" int64_t ntlb_colsum_workspace_bytes(int64_t M, int64_t N) {
   if (M <= 0 || N <= 0) return 0;
-  return cdiv(M, colsum_small(M, N) ? CS_ROWS_S : CS_ROWS) * N * 4;
+  return cdiv(M, colsum_few(M, N) ? CS_ROWS_S : CS_ROWS) * N * 4;
 }
 
 extern "C" int ntlb_colsum(const void* x, int x_dtype, int64_t M, int64_t N, int64_t ldx, float* workspace,
@@ -1901,7 +1923,7 @@ extern "C" int ntlb_colsum(const void* x, int x_dtype, int64_t M, int64_t N, int
   if (N == 0) return NTLB_OK;
   if (!out) return fail(NTLB_EINVAL, "%s: NULL output", fn);
   hipStream_t st = as_stream(stream);
-  const bool small = colsum_small(M, N);
+  const bool small = colsum_small(x, x_dtype, M, N, ldx);
   const int64_t chunks = cdiv(M, small ? CS_ROWS_S : CS_ROWS);
   if (M > 0) {
     if (!x || !workspace) return fail(NTLB_EINVAL, "%s: NULL input or workspace", fn);

@@ -165,11 +165,13 @@ def test_small_straight_through_gradients_match_float64(gpu_device, mnk):
         assert float(((got.double() - ref).abs() / ref.abs().clamp(min=float(ref.abs().max()) * 1e-3)).max()) <= 2.0 ** -7
 
 
-@pytest.mark.parametrize("shape", [(1, 1), (63, 130), (64, 128), (1003, 1541), (300, 70), (70000, 3)])
+@pytest.mark.parametrize("shape", [(1, 1), (63, 130), (64, 128), (1003, 1541), (300, 70), (70000, 3), (191, 1024),
+                                   (193, 1024), (3073, 512), (2049, 8192), (8193, 768), (16385, 64)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
 def test_colsum_of_few_columns_or_rows(gpu_device, shape, dtype):
-    """column sums on the 64-row chunks (odd columns and pitches, one row, many
-    rows) against float64; M fp32 additions"""
+    """column sums on the 64-row and the 256-row chunks, at both sides of the
+    rule's lines (odd columns and pitches, one row, many rows) against float64;
+    M fp32 additions"""
     from lowbit import ops
 
     M, N = shape
