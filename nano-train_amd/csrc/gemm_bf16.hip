@@ -90,8 +90,8 @@ __device__ __forceinline__ v4f mma(const v8i& p, const v8i& q, v4f acc) {
 }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t operand_rsrc(const Bf16Operand& o) {
-  return __builtin_amdgcn_make_buffer_rsrc((void*)o.p, (short)0, (int)((o.tr ? o.kvalid : o.rows) * o.ld * 2),
-                                           0x00020000);
+  const int64_t bytes = o.tr ? stored_rows_extent(o.kvalid, o.ld, o.rows, 2) : o.rows * o.ld * 2;
+  return __builtin_amdgcn_make_buffer_rsrc((void*)o.p, (short)0, (int)bytes, 0x00020000);
 }
 
 // The copies of one operand's K step (16*B operand rows, 2*B KiB-copies of 64

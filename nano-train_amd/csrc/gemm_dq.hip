@@ -340,13 +340,14 @@ struct Stager<SRC_CODES, EL, GRID, SCM> {
 };
 
 // Buffer resource over the first kvalid stored rows of a transposed operand:
-// reads at or past kvalid*ld*eb bytes return zero, which zero-fills the
-// contraction past kvalid (and keeps the lanes past the last stored row in
-// bounds).  Lanes whose operand row r lies past the operand's rows read
-// whatever follows in memory: those values reach only output rows or columns
-// that are never stored.  The entry points check (kvalid + 64) * ld * eb < 2^31.
+// reads past the last stored row's values return zero, which zero-fills the
+// contraction past kvalid and keeps every lane inside the matrix.  Lanes whose
+// operand row r lies past the operand's rows read zero there and the next
+// stored row elsewhere: those values reach only output rows or columns that
+// are never stored.  The entry points check (kvalid + 64) * ld * eb < 2^31.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t trows_rsrc(const Operand& o, int eb) {
-  return __builtin_amdgcn_make_buffer_rsrc((void*)o.p, (short)0, (int)(o.kvalid * o.ld * eb), 0x00020000);
+  return __builtin_amdgcn_make_buffer_rsrc((void*)o.p, (short)0, (int)stored_rows_extent(o.kvalid, o.ld, o.rows, eb),
+                                           0x00020000);
 }
 
 // TDIRECT: wave w takes contraction rows [w*CPW, w*CPW + CPW) of the K step,

@@ -1,4 +1,5 @@
-// bf16 GEMMs on tiles below 256x256 (gemm_bf16.hip): what their callers pass.
+// bf16 GEMMs on tiles below 256x256 (gemm_bf16.hip): what their callers pass,
+// and the extent of an operand stored transposed (gemm_dq.hip's too).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -6,6 +7,17 @@
 #include <cstdint>
 
 namespace ntlb {
+
+// Bytes from the first to the last value of kvalid stored rows of pitch ld and
+// `rows` values of eb bytes, the last row's end rounded up to a 16-byte load:
+// the extent of a buffer resource over a matrix stored transposed.  It ends
+// there and not at kvalid * ld, because a column slice of a larger matrix may
+// be the end of its allocation.
+__host__ __device__ inline int64_t stored_rows_extent(int64_t kvalid, int64_t ld, int64_t rows, int eb) {
+  if (kvalid <= 0) return 0;
+  const int64_t last = (rows * eb + 15) / 16 * 16, pitch = ld * eb;
+  return (kvalid - 1) * pitch + (last < pitch ? last : pitch);
+}
 
 // One operand of Y[M,N] = A . B^T over plain bf16 matrices.
 //   tr = false (A only): [rows, >= Kc] row-major, the contraction contiguous;

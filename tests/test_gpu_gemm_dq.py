@@ -401,3 +401,25 @@ def test_ste_wgrad_with_db_matches_colsum(gpu_device, M, N, K):
     qi = ops.quant_tile_1x128(x, fmt="int_grid")
     with pytest.raises((LowBitKernelError, ValueError, RuntimeError)):
         ops.ste_wgrad(dy, qi, out_dtype=torch.bfloat16, db_dtype=torch.float32)
+
+
+# dY's columns are the end of the rows of a 32 MiB allocation: small tiles, and
+# the 256x256 ones; N of no whole tile and no whole 16 bytes
+@pytest.mark.parametrize("M,pitch,N,K", [(1024, 16384, 200, 320), (4096, 4096, 2888, 3000), (4096, 4096, 2885, 3000)])
+def test_wgrad_of_a_slice_at_the_end_of_its_allocation(gpu_device, M, pitch, N, K):
+    """dW = dY^T . X where the last row of dY ends the allocation (no bytes of the
+    row's pitch follow it), against float64: one bf16 rounding of an fp32 sum"""
+    from lowbit import ops
+
+    torch.cuda.empty_cache()
+    big = torch.empty((M, pitch), dtype=torch.bfloat16, device=gpu_device)
+    assert big.numel() * 2 % (2 << 20) == 0
+    big.copy_(seeded((M, pitch), seed=20262161, std=1e-3))
+    dy = big[:, pitch - N:]
+    x = seeded((M, K), seed=20262162).to(gpu_device)
+    ref = dy.double().T @ x.double()
+    qx = ops.quant_tile_1x128(x, fmt="e4m3")
+    xq = ops.dequant(qx, out_dtype=torch.bfloat16).double()
+    for got, want in ((ops.gemm_bf16_tn(dy, x), ref), (ops.gemm_dense_tn(dy, x), ref),
+                      (ops.ste_wgrad(dy, qx, out_dtype=torch.bfloat16), dy.double().T @ xq)):
+        assert float((got.double() - want).norm() / want.norm()) <= 2.0 ** -9

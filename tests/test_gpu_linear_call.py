@@ -312,3 +312,15 @@ def test_gradient_of_another_dtype(gpu_device, grads):
         out.append(_HipLowBitLinear.backward(y.grad_fn, dy))
     assert all(_same(p, q) for p, q in zip(*out))
     assert [v is not None for v in out[0]] == [*grads, False, False]
+
+
+@pytest.mark.parametrize("mnk", [(64, 256, 320), (500, 1536, 4600)])
+def test_wide_gradient_rows(gpu_device, mnk):
+    """a dY whose row pitch is past the one the small dX and dW tiles take (the
+    last columns of a wider gradient): the 256x256 tiles, dX with its split tail"""
+    M, N, K = mnk
+    x = seeded((M, K), seed=20262201).to(gpu_device)
+    w = seeded((N, K), seed=20262202, std=0.02).to(gpu_device)
+    big = seeded((M, 2 * N), seed=20262203, std=1e-3).to(gpu_device)
+    one, gen = _both("e4m3", "nearest", "ste", x, w, None, big[:, N:], general_dy=big[:, N:].contiguous())
+    assert _agree("ste", one, gen)
