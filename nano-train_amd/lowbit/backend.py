@@ -167,7 +167,7 @@ class _LinearPlan:
     and the quantizers' settings, no pointers and no tensors, and constant once
     made (so calls of any thread or stream share it)."""
 
-    __slots__ = ("c", "ref", "M", "N", "K", "x_bytes", "w_bytes", "ws_bytes")
+    __slots__ = ("c", "ref", "M", "N", "K", "x_bytes", "w_bytes", "code_bytes", "ws_bytes")
 
     def __init__(self, M, N, K, ldx, ldw, xdt, wdt, bdt, grid, qmax, rounding, seed) -> None:
         self.c = _lib.LinearPlan(M=M, N=N, K=K, ldx=ldx, ldw=ldw, x_dtype=ops._dtype_code(xdt),
@@ -177,6 +177,7 @@ class _LinearPlan:
         self.M, self.N, self.K = M, N, K
         _lib.call("ntlb_linear_plan_init", self.ref)
         self.x_bytes, self.w_bytes = self.c.x_code_bytes, self.c.w_code_bytes
+        self.code_bytes = self.x_bytes + self.w_bytes
         self.ws_bytes = self.c.forward_ws
 
     def x_tensor(self, buf: torch.Tensor) -> QTensor:
@@ -271,7 +272,6 @@ class _HipLowBitLinear(torch.autograd.Function):
         needs = ctx.needs_input_grad
         out_dtype = x.dtype
         K = x.shape[-1]
-        N = weight.shape[0]
         ctx.plan = None
         if backend._one_call(x, weight, bias, needs):
             x2 = _rows_2d(x, K)
@@ -282,16 +282,15 @@ class _HipLowBitLinear(torch.autograd.Function):
             # buffer where both or none are kept, else one each, so that the
             # other is given back after the call
             ste = backend.backward_recipe == "ste"
-            keep_x, keep_w = ste and needs[1], ste and needs[0]
-            if keep_x == keep_w:
-                xb = torch.empty(plan.x_bytes + plan.w_bytes, dtype=torch.uint8, device=dev)
-                xp, kept = xb.data_ptr(), (xb,) if keep_x else ()
+            if not ste or needs[0] == needs[1]:
+                xb = torch.empty(plan.code_bytes, dtype=torch.uint8, device=dev)
+                xp = xb.data_ptr()
                 wp = xp + plan.x_bytes
             else:
                 xb = torch.empty(plan.x_bytes, dtype=torch.uint8, device=dev)
                 wb = torch.empty(plan.w_bytes, dtype=torch.uint8, device=dev)
-                xp, wp, kept = xb.data_ptr(), wb.data_ptr(), (xb,) if keep_x else (wb,)
-            y = torch.empty((*x.shape[:-1], N), dtype=out_dtype, device=dev)
+                xp, wp = xb.data_ptr(), wb.data_ptr()
+            y = torch.empty((plan.M, plan.N) if x.dim() == 2 else (*x.shape[:-1], plan.N), dtype=out_dtype, device=dev)
             ws, ws_bytes = (None, 0) if plan.ws_bytes == 0 else _workspace(plan.ws_bytes, dev)
             if bias is not None and bias.stride(-1) != 1:
                 bias = bias.contiguous()
@@ -302,9 +301,13 @@ class _HipLowBitLinear(torch.autograd.Function):
                 ctx.plan, ctx.backend, ctx.offset = plan, backend, base
                 ctx.bias_dtype = None if bias is None else bias.dtype
                 ctx.x_shape, ctx.x_dtype, ctx.w_dtype = x.shape, out_dtype, weight.dtype
-                ctx.kept_x, ctx.kept_w = keep_x, keep_w
-                ctx.save_for_backward(*(kept if ste else (x2, weight)))
+                if not ste:
+                    ctx.save_for_backward(x2, weight)
+                elif needs[0] or needs[1]:
+                    ctx.save_for_backward(xb if needs[1] else wb)
+                ctx.kept_x, ctx.kept_w = ste and needs[1], ste and needs[0]
             return y
+        N = weight.shape[0]
         x2 = x.reshape(-1, K)
         if x2.stride(-1) != 1:
             x2 = x2.contiguous()
@@ -559,10 +562,10 @@ class HipLowBitBackend:
         granularities in blockscaled mode, and a backward that reads codes (the
         straight-through rule of bf16 layers under round to nearest) or
         quantizes its own operands."""
+        shape, stride = weight.shape, weight.stride()
         if (self._activation_granularity != "tile_1x128" or self._weight_granularity != "block_128x128"
-                or self.forward_mode != "blockscaled" or weight.dim() != 2 or weight.stride(1) != 1
-                or weight.stride(0) < weight.shape[1] or weight.shape[0] == 0
-                or (bias is not None and bias.device.type != "cuda")):
+                or self.forward_mode != "blockscaled" or len(shape) != 2 or stride[1] != 1 or stride[0] < shape[1]
+                or shape[0] == 0 or (bias is not None and not bias.is_cuda)):
             return False
         if (needs[0] or needs[1]) and self.backward_recipe == "ste":
             return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
