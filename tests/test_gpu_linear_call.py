@@ -125,9 +125,9 @@ def test_gradient_subsets_and_strides(gpu_device, recipe, grads):
 
 
 @pytest.mark.parametrize("fmt", ["e4m3", "int_grid"])
-@pytest.mark.parametrize("recipe", ["ste", "fp8"])
+@pytest.mark.parametrize("recipe,rounding", [("ste", "nearest"), ("fp8", "nearest"), ("fp8", "stochastic")])
 @pytest.mark.parametrize("mnk", [(20, 72, 200), (300, 700, 1500), (1100, 2100, 700)])
-def test_nan_and_inf_operands(gpu_device, mnk, fmt, recipe):
+def test_nan_and_inf_operands(gpu_device, mnk, fmt, recipe, rounding):
     """NaN and infinities in x, the weight and dY: NaN exactly where the flagged
     products of the general path have it, every other value the same"""
     M, N, K = mnk
@@ -137,7 +137,7 @@ def test_nan_and_inf_operands(gpu_device, mnk, fmt, recipe):
     x[3, 17], x[5, K - 1], x[M - 1, 4] = float("nan"), float("inf"), float("-inf")
     w[7, 100], w[N - 1, 5] = float("nan"), float("inf")
     dy[9, 11], dy[2, N - 1] = float("nan"), float("inf")
-    one, gen = _both(fmt, "nearest", recipe, x, w, None, dy)
+    one, gen = _both(fmt, rounding, recipe, x, w, None, dy)
     assert torch.isnan(one[0][3]).all() and torch.isnan(one[0][:, 7]).all() and not torch.isnan(one[0][0, 0])
     assert _agree(recipe, one, gen)
 

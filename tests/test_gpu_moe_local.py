@@ -232,7 +232,8 @@ def test_combine_split_over_columns_equals_whole_rows(gpu_device, H, w_dtype):
         assert torch.equal(moe.combine_rows(y, part, ids[:t], w[:t], t), whole[:t])
 
 
-def test_e4m3_expert_loop_carries_a_nan_without_flags(gpu_device):
+@pytest.mark.parametrize("rounding", ["nearest", "stochastic"])
+def test_e4m3_expert_loop_carries_a_nan_without_flags(gpu_device, rounding):
     """The token with the NaN is NaN in every column, the others keep their bits."""
     from lowbit import moe
 
@@ -245,9 +246,10 @@ def test_e4m3_expert_loop_carries_a_nan_without_flags(gpu_device):
          for s in ((I, H), (I, H), (H, I))]
     gu = moe.quantize_expert_weights(moe.stack_gate_up(w[0], w[1]), fmt="e4m3")
     down = moe.quantize_expert_weights(w[2], fmt="e4m3")
-    clean = moe.local_moe_forward(x, ids, tw, gu, down, n_experts=E, fmt="e4m3")
+    kw = dict(n_experts=E, fmt="e4m3", rounding=rounding, seed=21, offset=8)
+    clean = moe.local_moe_forward(x, ids, tw, gu, down, **kw)
     x[7, 130] = float("nan")
-    got = moe.local_moe_forward(x, ids, tw, gu, down, n_experts=E, fmt="e4m3")
+    got = moe.local_moe_forward(x, ids, tw, gu, down, **kw)
     assert torch.isnan(got[7]).all()
     keep = torch.arange(T, device=gpu_device) != 7
     assert torch.equal(got[keep], clean[keep])
