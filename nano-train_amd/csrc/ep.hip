@@ -853,10 +853,11 @@ extern "C" int ntlb_moe_combine_rows(const void* y, int64_t ldy, int64_t n, cons
   // the product rounds to the output dtype when torch's promotion of (y, w)
   // is that dtype: w of the same dtype, which is not fp32
   const bool round_p = w_dtype == out_dtype && out_dtype != NTLB_F32;
-  // A workgroup per token walks its row in serial passes of loads; with fewer
-  // tokens than two workgroups per compute unit the row is split at whole
-  // passes (32 tokens, K 8, H 7168: 14.2 us on 32 workgroups, 6.0
-  // on 224).  From 512 tokens on, every unit has its workgroups without.
+  // A workgroup per token walks its row in serial passes of loads; where a
+  // second workgroup per token still leaves no more than two for a compute
+  // unit (up to 256 tokens) the row is split at whole passes into 512 / T
+  // parts.  K 8, H 7168, us in a graph, whole rows / split: 1 token 10.0 / 4.1, 32
+  // 10.3 / 4.3, 100 10.4 / 6.6, 256 11.4 / 10.0; 257 tokens, whole, 15.4.
   constexpr int64_t PASS = COMBINE_ROWS_THREADS * 8;
   const int64_t passes = cdiv(H, PASS);
   const int64_t parts = std::min(passes, std::max<int64_t>(1, 512 / T));

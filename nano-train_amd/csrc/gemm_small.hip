@@ -661,7 +661,11 @@ __global__ void __launch_bounds__(512) gemm_small_grouped_swiglu_kernel(GemmArgs
 //   gate/up 8 experts 2048 x 2048            1:  40 |  20 |  19  32:  40 |  19 |  21  64:  47 |  27 |  20  128: 46 | 38 | 35
 //   down 8 experts 2048 x 1024               1:  17 |  10 |  10  32:  17 |  10 |  12  64:  19 |  16 |  12  128: 19 | 22 | 21
 // So up to 24 rows each, and up to 64 where the 256x256 tiles leave half of
-// the chip's 256 compute units without a tile.
+// the chip's 256 compute units without a tile.  The counts themselves would
+// move the line only where a few experts get every row: the whole loop at H
+// 7168, I 2048, 32 experts, top 8 takes, 256x256 tiles | here, at 24 rows each 417 |
+// 313 evenly, 418 | 371 by Zipf(1.2), 186 | 198 with all rows on 8 experts (16
+// rows each: 181 | 136).
 static int grouped_mb(int64_t R, int64_t E, int64_t N) {
   if (E > 16384) return 0;  // the row tiles are the grid's y
   if (R <= 4 * E) return 1;

@@ -407,7 +407,8 @@ enum RefreshFmt : int { REFRESH_NONE = 0, REFRESH_NF4 = 1, REFRESH_FP8 = 2 };
 // entry 32 is c = 1.  The four-level binary search this replaces took about 40
 // VALU instructions per weight and bound the quantizers (the two-pass
 // per_channel quantize pass at [14336, 4096]: 79 us); the lookup takes six and
-// one 8-byte LDS read whose 33 entries lie in distinct banks.
+// one 8-byte LDS read (33 entries, 66 words over 64 banks: only entry 32, c = 1
+// alone, shares its banks with entry 0).
 constexpr float kNF4t[15] = {-0x1.b239b2p-1f, -0x1.38a4e2p-1f, -0x1.d709p-2f, -0x1.5bd4eep-2f, -0x1.e079dap-3f,
                              -0x1.1a7178p-3f, -0x1.74f0e4p-5f, 0x1.45f5fep-5f, 0x1.ec90c4p-4f, 0x1.a0cfcp-3f,
                              0x1.2b05a8p-2f, 0x1.8ea7f2p-2f, 0x1.00da06p-1f, 0x1.491b5ep-1f, 0x1.b913b2p-1f};
