@@ -17,6 +17,7 @@
 #include "ntlb_device.h"
 #include "ntlb_gemm_bf16.h"
 #include "ntlb_host.h"
+#include "ntlb_small_tile.h"
 #include "ntlb_splitk.h"
 
 namespace ntlb {
@@ -33,8 +34,6 @@ typedef __attribute__((address_space(3))) v4s* lds_v4s_ptr;
 
 constexpr int ROWB = 128;   // bytes of a row's K step
 constexpr int KSTEP = 64;
-
-constexpr int vmcnt_imm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
 
 // Row-major stage [16*B rows][128 bytes]: 16-byte chunk c of row r at slot
 // c ^ perm(r), conflict-free for the 16-row fragment reads
@@ -208,26 +207,9 @@ __global__ void __launch_bounds__(64 * WK) gemm_bf16_small_kernel(Bf16Args g) {
     __builtin_amdgcn_s_waitcnt(0);  // nothing of this wave is in flight into LDS past here
     asm volatile("" ::: "memory");
   }
-  __syncthreads();
-  v4f* red = reinterpret_cast<v4f*>(st0);
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) red[(wave * MB * NB + mb * NB + nb) * 64 + lane] = acc[mb][nb];
-  __syncthreads();
-  // lane l of block (mb, nb): row m0 + 16*mb + l%16, columns n0 + 16*nb + 4*(l/16) + 0..3
-  for (int q = threadIdx.x; q < MB * NB * 64; q += 64 * WK) {
-    const int b = q >> 6, l = q & 63;
-    v4f v = red[q];
-#pragma unroll
-    for (int w = 1; w < WK; ++w) v += red[w * MB * NB * 64 + q];
-    const int64_t m = m0 + (b / NB) * 16 + (l & 15);
-    const int64_t n = n0 + (b % NB) * 16 + (l >> 4) * 4;
-    if (m < g.M && n < g.N) store4(g, m, n, v);
-  }
+  sum_partials<MB, NB, WK>(reinterpret_cast<v4f*>(st0), acc, wave, lane, m0, n0, g.M, g.N,
+                           [&](int64_t m, int64_t n, v4f v) { store4(g, m, n, v); });
 }
-
-constexpr int MID = 128;
 
 template <bool TA, int ODT>
 __global__ void __launch_bounds__(256, 2) gemm_bf16_mid_kernel(Bf16Args g) {
@@ -238,20 +220,8 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16_mid_kernel(Bf16Args g) {
   __shared__ __attribute__((aligned(16))) uint8_t lb1[ST];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
-  // each XCD walks a contiguous range of a raster of four row tiles
-  const int num_n = (int)((g.N + MID - 1) / MID), num_m = (int)((g.M + MID - 1) / MID);
   int64_t m0, n0;
-  {
-    const int nwg = (int)gridDim.x, xcd = (int)blockIdx.x & 7, local = (int)blockIdx.x >> 3;
-    const int per = nwg >> 3, extra = nwg & 7;
-    const int pid = xcd * per + min(xcd, extra) + local;
-    constexpr int GROUP_M = 4;
-    const int group = pid / (GROUP_M * num_n);
-    const int gsize = min(num_m - group * GROUP_M, GROUP_M);
-    const int in_group = pid - group * GROUP_M * num_n;
-    m0 = (int64_t)(group * GROUP_M + in_group % gsize) * MID;
-    n0 = (int64_t)(in_group / gsize) * MID;
-  }
+  mid_tile(g.M, g.N, m0, n0);
   Copies<TA, 8, 4> ca;
   Copies<true, 8, 4> cb;
   ca.init(g.a, m0, wave, lane);
@@ -289,51 +259,10 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16_mid_kernel(Bf16Args g) {
     step(std::integral_constant<int, 0>(), ks);
     if (ks + 1 < nk) step(std::integral_constant<int, 1>(), ks + 1);
   }
-  // each wave stages 32 of its 64 rows at a time and stores whole row segments
+  // each wave stages its rows in its 16 KiB of the idle stages
   uint8_t* stage_w = wave == 0 ? la0 : wave == 1 ? lb0 : wave == 2 ? la1 : lb1;
-  constexpr int esz = ODT == DT_F32 ? 4 : 2, pitch = 64 * esz + 16, cpr = 64 * esz / 16, epc = 16 / esz;
-  static_assert(32 * pitch <= ST, "staged rows fit a stage");
-#pragma unroll
-  for (int part = 0; part < 2; ++part) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-#pragma unroll
-      for (int tn = 0; tn < 4; ++tn) {
-        const v4f v = acc[part * 2 + t][tn];
-        uint8_t* dst = stage_w + (t * 16 + (lane & 15)) * pitch + (tn * 16 + (lane >> 4) * 4) * esz;
-        if constexpr (ODT == DT_F32) {
-          *reinterpret_cast<v4f*>(dst) = v;
-        } else if constexpr (ODT == DT_BF16) {
-          const v2bf p0 = {(__bf16)v[0], (__bf16)v[1]}, p1 = {(__bf16)v[2], (__bf16)v[3]};
-          *reinterpret_cast<uint2*>(dst) =
-              make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
-        } else {
-          const __half h[4] = {f32_to_f16(v[0]), f32_to_f16(v[1]), f32_to_f16(v[2]), f32_to_f16(v[3])};
-          *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(h);
-        }
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int j = 0; j < cpr / 2; ++j) {
-      const int q = lane + 64 * j, row = q / cpr, c = q % cpr;
-      const int64_t m = m0 + wm * 64 + part * 32 + row, n = n0 + wn * 64 + c * epc;
-      const uint8_t* src = stage_w + row * pitch + c * 16;
-      if (m >= g.M || n >= g.N) continue;
-      uint8_t* ydst = reinterpret_cast<uint8_t*>(g.y) + (m * g.ldy + n) * esz;
-      if (g.vec_out && n + epc <= g.N) {
-        store16_nt(ydst, src);
-      } else {
-        using E = std::conditional_t<esz == 4, uint32_t, uint16_t>;
-#pragma nounroll
-        for (int e = 0; e < epc && n + e < g.N; ++e)
-          reinterpret_cast<E*>(ydst)[e] = reinterpret_cast<const E*>(src)[e];
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    __builtin_amdgcn_wave_barrier();
-  }
+  mid_store<ODT>(stage_w, lane, m0 + wm * 64, n0 + wn * 64, g.M, g.N, g.y, g.ldy, g.vec_out, [](int) { return 0; },
+                 [&](int tm, int tn, int) { return acc[tm][tn]; });
 }
 
 // every instance explicitly: the host stubs of implicitly instantiated ones
@@ -401,7 +330,7 @@ Bf16Plan bf16_small_plan(int64_t M, int64_t N, int64_t Kc, bool big_split) {
   if (wgs(32, 64) <= cus) return {2, 4, 4, 3};
   if (wgs(64, 64) <= cus) return {4, 4, 4, 2};
   if (wgs(64, 64) <= 2 * cus) return {4, 4, 2, 2};
-  if (wgs(bfs::MID, bfs::MID) <= 2 * cus) {
+  if (wgs(MID, MID) <= 2 * cus) {
     const int split = big_split ? split_plan(wgs(256, 256), nk, DQ_SPLIT_MIN_STEPS).s : 1;
     if (split == 1 || 1.05 * nk + 3 < 1.4 * nk / split + 30) return {8, 8, 4, 2};
   }

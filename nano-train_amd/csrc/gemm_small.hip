@@ -20,12 +20,10 @@
 
 #include "ntlb_gemm_tile.h"
 #include "ntlb_host.h"
+#include "ntlb_small_tile.h"
 #include "ntlb_splitk.h"
 
 namespace ntlb {
-
-// s_waitcnt with only vmcnt set
-constexpr int vmcnt_imm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
 
 // One wave's copies of a 16*MB-row A and 16*NB-row B K block into LDS: copy t
 // moves rows 8t .. 8t+7 (lane i: row i/8, physical chunk i%8, which holds the
@@ -209,23 +207,8 @@ __global__ void __launch_bounds__(64 * WK) gemm_small_kernel(GemmArgs g) {
     small_k_loop<GRID, B_UNIFORM, MB, NB, NS>(g, cp, m0, n0, kb0, kb1, st0 + wave * WB, st1 + wave * WB,
                                               st2 + (NS > 2 ? wave * WB : 0), lane, acc);
   }
-  __syncthreads();  // every wave is done with its stages: the partials go where the first one was
-  v4f* red = reinterpret_cast<v4f*>(st0);
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) red[(wave * MB * NB + mb * NB + nb) * 64 + lane] = acc[mb][nb];
-  __syncthreads();
-  // lane l of block (mb, nb) holds row m0 + 16*mb + l%16, columns n0 + 16*nb + 4*(l/16) + 0..3
-  for (int q = threadIdx.x; q < MB * NB * 64; q += 64 * WK) {
-    const int b = q >> 6, l = q & 63;
-    v4f v = red[q];
-#pragma unroll
-    for (int w = 1; w < WK; ++w) v += red[w * MB * NB * 64 + q];
-    const int64_t m = m0 + (b / NB) * 16 + (l & 15);
-    const int64_t n = n0 + (b % NB) * 16 + (l >> 4) * 4;
-    if (m < g.M && n < g.N) small_store4(g, m, n, v, g.nan_b);
-  }
+  sum_partials<MB, NB, WK>(reinterpret_cast<v4f*>(st0), acc, wave, lane, m0, n0, g.M, g.N,
+                           [&](int64_t m, int64_t n, v4f v) { small_store4(g, m, n, v, g.nan_b); });
 }
 
 // ---------------------------------------------------------------------------
@@ -236,7 +219,6 @@ __global__ void __launch_bounds__(64 * WK) gemm_small_kernel(GemmArgs g) {
 // 64x64 tiles: per 16x16x128 MFMA a wave reads 1 KiB of LDS (0.75 on the
 // 256x256 tiles' 128x64 waves), which at the MFMA rate is the LDS bandwidth.
 // ---------------------------------------------------------------------------
-constexpr int MID = 128;
 constexpr int MID_TILE = MID * BK;  // 16 KiB per operand stage
 
 template <int GRID, bool B_UNIFORM, int ODT>
@@ -248,20 +230,8 @@ __global__ void __launch_bounds__(256, 2) gemm_mid_kernel(GemmArgs g) {
   __shared__ float ls0[2 * MID], ls1[2 * MID];  // A row scales, then B row scales
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
-  // each XCD walks a contiguous range of a raster of four row tiles
-  const int num_n = (int)((g.N + MID - 1) / MID), num_m = (int)((g.M + MID - 1) / MID);
   int64_t m0, n0;
-  {
-    const int nwg = (int)gridDim.x, xcd = (int)blockIdx.x & 7, local = (int)blockIdx.x >> 3;
-    const int per = nwg >> 3, extra = nwg & 7;
-    const int pid = xcd * per + min(xcd, extra) + local;
-    constexpr int GROUP_M = 4;
-    const int group = pid / (GROUP_M * num_n);
-    const int gsize = min(num_m - group * GROUP_M, GROUP_M);
-    const int in_group = pid - group * GROUP_M * num_n;
-    m0 = (int64_t)(group * GROUP_M + in_group % gsize) * MID;
-    n0 = (int64_t)(in_group / gsize) * MID;
-  }
+  mid_tile(g.M, g.N, m0, n0);
   const bool own_a = tid < MID;
   const int64_t srow = own_a ? min<int64_t>(m0 + tid, g.M - 1) : min<int64_t>(n0 + tid - MID, g.N - 1);
   const float* s_src = own_a ? g.sa + (srow >> g.a_shift) * g.sa_row : g.sb + (srow >> g.b_shift) * g.sb_row;
@@ -352,22 +322,16 @@ __global__ void __launch_bounds__(256, 2) gemm_mid_kernel(GemmArgs g) {
     if (kt + 1 < nk) step(std::integral_constant<int, 1>(), kt + 1);
   }
 
-  // epilogue: each wave stages 32 of its 64 rows at a time in its 16 KiB of the
-  // idle stages and stores whole 128-byte (fp32: 256-byte) row segments
+  // each wave stages its rows in its 16 KiB of the idle stages
   uint8_t* stage_w = wave == 0 ? la0 : wave == 1 ? lb0 : wave == 2 ? la1 : lb1;
-  constexpr int esz = ODT == DT_F32 ? 4 : 2, pitch = 64 * esz + 16, cpr = 64 * esz / 16, epc = 16 / esz;
-  static_assert(32 * pitch <= MID_TILE, "staged rows fit a stage");
   const float qnan = __uint_as_float(0x7FC00000u);
-#pragma unroll
-  for (int part = 0; part < 2; ++part) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int tm = part * 2 + t;
-      const bool nan_m = g.nan_a && g.nan_a[min<int64_t>(m0 + wm * 64 + tm * 16 + (lane & 15), g.M - 1)] != 0;
-#pragma unroll
-      for (int tn = 0; tn < 4; ++tn) {
+  const int64_t mw = m0 + wm * 64, nw = n0 + wn * 64;
+  mid_store<ODT>(
+      stage_w, lane, mw, nw, g.M, g.N, g.y, g.ldy, g.vec_out,
+      [&](int tm) { return g.nan_a && g.nan_a[min<int64_t>(mw + tm * 16 + (lane & 15), g.M - 1)] != 0; },
+      [&](int tm, int tn, bool nan_m) {
         v4f v = acc[tm][tn];
-        const int64_t n = n0 + wn * 64 + tn * 16 + (lane >> 4) * 4;
+        const int64_t n = nw + tn * 16 + (lane >> 4) * 4;
         if (g.bias) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) v[q] += load_elem(g.bias, g.bias_dtype, min<int64_t>(n + q, g.N - 1));
@@ -377,40 +341,8 @@ __global__ void __launch_bounds__(256, 2) gemm_mid_kernel(GemmArgs g) {
           for (int q = 0; q < 4; ++q) v[q] = g.nan_b[min<int64_t>(n + q, g.N - 1)] ? qnan : v[q];
         }
         if (nan_m) v = (v4f){qnan, qnan, qnan, qnan};
-        uint8_t* dst = stage_w + (t * 16 + (lane & 15)) * pitch + (tn * 16 + (lane >> 4) * 4) * esz;
-        if constexpr (ODT == DT_F32) {
-          *reinterpret_cast<v4f*>(dst) = v;
-        } else if constexpr (ODT == DT_BF16) {
-          const v2bf p0 = {(__bf16)v[0], (__bf16)v[1]}, p1 = {(__bf16)v[2], (__bf16)v[3]};
-          *reinterpret_cast<uint2*>(dst) =
-              make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
-        } else {
-          const __half h[4] = {f32_to_f16(v[0]), f32_to_f16(v[1]), f32_to_f16(v[2]), f32_to_f16(v[3])};
-          *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(h);
-        }
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's staging writes are done
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int j = 0; j < cpr / 2; ++j) {
-      const int q = lane + 64 * j, row = q / cpr, c = q % cpr;
-      const int64_t m = m0 + wm * 64 + part * 32 + row, n = n0 + wn * 64 + c * epc;
-      const uint8_t* src = stage_w + row * pitch + c * 16;
-      if (m >= g.M || n >= g.N) continue;
-      uint8_t* ydst = reinterpret_cast<uint8_t*>(g.y) + (m * g.ldy + n) * esz;
-      if (g.vec_out && n + epc <= g.N) {
-        store16_nt(ydst, src);
-      } else {
-        using E = std::conditional_t<esz == 4, uint32_t, uint16_t>;
-#pragma nounroll
-        for (int e = 0; e < epc && n + e < g.N; ++e)
-          reinterpret_cast<E*>(ydst)[e] = reinterpret_cast<const E*>(src)[e];
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // the re-reads are done before the next part overwrites
-    __builtin_amdgcn_wave_barrier();
-  }
+        return v;
+      });
 }
 
 struct SmallPlan {
