@@ -167,7 +167,7 @@ class _LinearPlan:
     and the quantizers' settings, no pointers and no tensors, and constant once
     made (so calls of any thread or stream share it)."""
 
-    __slots__ = ("c", "ref", "M", "N", "K", "x_bytes", "w_bytes", "code_bytes", "ws_bytes")
+    __slots__ = ("c", "ref", "M", "N", "K", "x_strides", "w_strides", "x_bytes", "w_bytes", "code_bytes", "ws_bytes")
 
     def __init__(self, M, N, K, ldx, ldw, xdt, wdt, bdt, grid, qmax, rounding, seed) -> None:
         self.c = _lib.LinearPlan(M=M, N=N, K=K, ldx=ldx, ldw=ldw, x_dtype=ops._dtype_code(xdt),
@@ -175,6 +175,7 @@ class _LinearPlan:
                                  grid=grid, qmax=qmax, rounding=rounding, seed=seed)
         self.ref = ctypes.addressof(self.c)
         self.M, self.N, self.K = M, N, K
+        self.x_strides, self.w_strides = (ldx, 1), (ldw, 1)
         _lib.call("ntlb_linear_plan_init", self.ref)
         self.x_bytes, self.w_bytes = self.c.x_code_bytes, self.c.w_code_bytes
         self.code_bytes = self.x_bytes + self.w_bytes
@@ -213,15 +214,9 @@ def _rows_2d(t: torch.Tensor, cols: int) -> torch.Tensor:
     return t2.contiguous().view(-1).view(-1, cols)
 
 
-def _saved_operand(t: torch.Tensor, cols: int) -> torch.Tensor:
-    """A matrix kept for the backward, as its saved-tensor hooks give it back:
-    the kernels get its address, so its place and layout are looked at here"""
-    ops._require_device(t)
-    return _rows_2d(t, cols)
-
-
 def _saved_codes(buf: torch.Tensor, nbytes: int) -> torch.Tensor:
-    """A forward's code buffer kept for the backward, checked as _saved_operand"""
+    """A forward's code buffer kept for the backward, as its saved-tensor hooks
+    give it back: the kernels get its address, so it is looked at here"""
     ops._require_device(buf)
     if buf.dtype != torch.uint8 or buf.numel() != nbytes:
         raise RuntimeError(f"the saved codes came back as {buf.dtype}[{buf.numel()}], not uint8[{nbytes}]")
@@ -302,6 +297,7 @@ class _HipLowBitLinear(torch.autograd.Function):
                 ctx.bias_dtype = None if bias is None else bias.dtype
                 ctx.x_shape, ctx.x_dtype, ctx.w_dtype = x.shape, out_dtype, weight.dtype
                 if not ste:
+                    ctx.settings = backend._settings()
                     ctx.save_for_backward(x2, weight)
                 elif needs[0] or needs[1]:
                     ctx.save_for_backward(xb if needs[1] else wb)
@@ -423,11 +419,18 @@ class _HipLowBitLinear(torch.autograd.Function):
                     op = _gemm_op_dtype(dy2.dtype, xdq.dtype)
                     dw = ops.gemm_dense_tn(dy2.to(op), xdq.to(op), out_dtype=ctx.w_dtype)
             else:
-                x2, weight = (_saved_operand(t, plan.K) for t in ctx.saved_tensors)
+                x2, weight = ctx.saved_tensors  # looked at as _saved_codes does
+                if not (x2.is_cuda and weight.is_cuda):
+                    ops._require_device(x2, weight)
+                if x2.numel() != plan.M * plan.K or weight.numel() != plan.N * plan.K:
+                    raise RuntimeError("a saved tensor came back with another size")
+                if (x2.stride() != plan.x_strides or weight.stride() != plan.w_strides
+                        or ctx.settings != backend._settings()):
+                    # quantizes anew: the pitches of the tensors that came back, the settings of now
+                    x2, weight = _rows_2d(x2, plan.K), _rows_2d(weight, plan.K)
+                    plan = backend._plan(x2, weight, ctx.bias_dtype)
                 if (dy2.dtype == x2.dtype == weight.dtype == ctx.x_dtype == ctx.w_dtype
                         and dy2.dtype in _RECIPE_DTYPES):
-                    # quantizes anew: the settings of now, the pitches of the saved tensors
-                    plan = backend._plan(x2, weight, ctx.bias_dtype)
                     return (*_recipe_backward(plan, dy2, x2, weight, needs, ctx.x_shape, ctx.bias_dtype, ctx.offset),
                             None)
                 dx, dw = _fp8_recipe_backward(backend, dy2, x2, weight, ctx.offset, needs)
@@ -571,6 +574,10 @@ class HipLowBitBackend:
             return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
                     and self._rounding_mode != "stochastic")
         return True
+
+    def _settings(self):
+        """What a plan holds besides the shapes: may change between calls"""
+        return (self.seed, self.code_format, self.bits, self._rounding_mode)
 
     def _plan(self, x2, weight, bias_dtype) -> _LinearPlan:
         """The plan of a call, kept for the next one of the same sizes, pitches,
